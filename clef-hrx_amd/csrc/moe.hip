@@ -11,6 +11,7 @@
 // S1 (kernels/swiglu.loom:43-51) and C1 (kernels/omni_combine_ordered.loom:51-79,
 // kernels/omni_combine.loom:50-77).
 #include "common.hpp"
+#include "gemm_dma.hpp"
 #include "kernels.hpp"
 #include "group.hpp"
 #include "route.hpp"
@@ -642,51 +643,145 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 
 // Router gate projection: logits[t][e] = bf16(sum_k x[t][k] * w[e][k]) with
 // f32 accumulation on the bf16 MFMA -- the bf16 linear that produces the
 // Omni router logits (src/omni.rs:764 -> Engine::linear, src/ops.rs:95-175,
-// kernels/gemm_bf16_reference.loom). One workgroup per 32 tokens; wave w
-// computes experts 32w..32w+31 (x in the MFMA A slot, so lane l holds expert
-// 32w + l%32 for tokens 8(i/4) + 4(l/32) + i%4, i < 16). No barriers: waves
-// past the expert count leave at once.
-__global__ __launch_bounds__(256) void router_gate_kernel(const uint16_t* __restrict__ x,
-                                                          const uint16_t* __restrict__ w, int64_t tokens,
-                                                          int hidden, int experts, uint16_t* __restrict__ out) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int e0 = wave * 32;
-  if (e0 >= experts) return;
-  const int64_t t0 = (int64_t)blockIdx.x * 32;
-  const int r = lane & 31, kb = (lane >> 5) * 8;
-  const bool tok_ok = t0 + r < tokens;
-  const uint16_t* xa = x + (tok_ok ? t0 + r : 0) * (int64_t)hidden + kb;
-  const uint16_t* wb = w + (int64_t)(e0 + r) * hidden + kb;
-  v16f acc = {};
-  // hidden % 64 == 0: four 16-k MFMAs per iteration, their loads issued first
-  for (int k = 0; k < hidden; k += 64) {
-    u4 a[4], b[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      a[s] = tok_ok ? *reinterpret_cast<const u4*>(xa + k + 16 * s) : u4{0u, 0u, 0u, 0u};
-      b[s] = *reinterpret_cast<const u4*>(wb + k + 16 * s);
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
-                                                    __builtin_bit_cast(bf16x8_t, b[s]), acc, 0, 0, 0);
+// kernels/gemm_bf16_reference.loom). One wave per workgroup computes 32 tokens
+// x 32 experts (x in the MFMA A slot, so lane l holds expert l % 32 for
+// tokens 8(i/4) + 4(l/32) + i%4, i < 16) as one chain of 32x32x16 MFMAs in
+// ascending k: the chain fixes the f32 summation order, and its latency
+// (hidden / 16 MFMAs, 2 us at hidden 2048) is the floor at any token count.
+//
+// What bounded it: loads straight into the MFMA layout with one 64-k step in
+// flight paid a memory round trip per step (26.4 us at 1 token, 44.3 us at
+// 4096, hidden 2048). Here each wave keeps kRouterDepth steps in flight by
+// LDS DMA into its own ring (no barriers; 56 of the 63 vector memory
+// operations the wave can count), in whole 128-byte row pieces, 16-byte
+// chunk c of row r stored at c ^ ((r >> 1) & 7) (conflict-free 32-row reads).
+// Rows past the last token re-read it; their results are not stored.
+// The expert groups of one token block run on one XCD (workgroup b is on XCD
+// b % 8) and share its x rows in that XCD's L2.
+constexpr int kRouterDepth = 7;                          // 64-k steps in flight
+[[maybe_unused]] constexpr int kRouterRing = kRouterDepth + 1;
+constexpr int kRouterStage = 8192;                       // 32 x rows and 32 w rows of 128 bytes
+constexpr int kRouterInst = kRouterStage / 1024;         // DMA instructions per step
+
+__device__ __forceinline__ void router_wait(int steps_behind) {
+  // k-step kt has landed once at most the DMA of the steps after it is outstanding
+  switch (steps_behind) {
+    case 0: wait_vmcnt<0>(); break;
+    case 1: wait_vmcnt<kRouterInst>(); break;
+    case 2: wait_vmcnt<2 * kRouterInst>(); break;
+    case 3: wait_vmcnt<3 * kRouterInst>(); break;
+    case 4: wait_vmcnt<4 * kRouterInst>(); break;
+    case 5: wait_vmcnt<5 * kRouterInst>(); break;
+    default: wait_vmcnt<6 * kRouterInst>(); break;
   }
+}
+
+__global__ __launch_bounds__(64) void router_gate_kernel(const uint16_t* __restrict__ x,
+                                                         const uint16_t* __restrict__ w, int64_t tokens,
+                                                         int hidden, int experts, uint16_t* __restrict__ out) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(kRouterInst * kRouterDepth < 64, "vmcnt range");
+  __shared__ __align__(16) char lds[kRouterRing * kRouterStage];
+  const int groups = experts / 32;
+  const int64_t j = blockIdx.x / 8;
+  const int e0 = (int)(j % groups) * 32;
+  const int64_t t0 = (j / groups * 8 + blockIdx.x % 8) * 32;
+  if (t0 >= tokens) return;
+  const int lane = threadIdx.x;
+  const int r = lane & 31, h = lane >> 5;
+  // DMA instruction q moves rows 8q .. 8q+7 of x (q < 4) or of w: lane ->
+  // row 8q + lane / 8, stored chunk lane % 8
+  const char* src[kRouterInst];
+#pragma unroll
+  for (int q = 0; q < kRouterInst; ++q) {
+    const int row = 8 * (q & 3) + (lane >> 3);
+    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
+    const int64_t t = t0 + row < tokens ? t0 + row : tokens - 1;
+    src[q] = reinterpret_cast<const char*>(q < 4 ? x + t * hidden : w + (int64_t)(e0 + row) * hidden) + 16 * chunk;
+  }
+  auto issue = [&](char* stage, int kt) {
+#pragma unroll
+    for (int q = 0; q < kRouterInst; ++q)
+      __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src[q] + (int64_t)kt * 128), (lds_ptr_t)(stage + q * 1024), 16, 0,
+                                       0);
+  };
+  const int steps = hidden / 64;
+  v16f acc = {};
+  // The ring named as distinct restrict pointers of one body, so that the
+  // compiler keeps the other stages' DMA in flight across a stage's reads.
+  auto body = [&](char* __restrict__ s0, char* __restrict__ s1, char* __restrict__ s2, char* __restrict__ s3,
+                  char* __restrict__ s4, char* __restrict__ s5, char* __restrict__ s6, char* __restrict__ s7) {
+    static_assert(kRouterRing == 8, "one pointer per ring stage");
+    // FULL: a step with kRouterDepth more behind it (no branches)
+    auto step = [&](const char* rd, char* nx, int kt, auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
+      if constexpr (FULL)
+        wait_vmcnt<(kRouterDepth - 1) * kRouterInst>();
+      else
+        router_wait(steps - 1 - kt);
+      __builtin_amdgcn_sched_barrier(0);
+      u4 a[4], b[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int off = r * 128 + (((2 * s + h) ^ ((r >> 1) & 7)) << 4);
+        a[s] = *reinterpret_cast<const u4*>(rd + off);
+        b[s] = *reinterpret_cast<const u4*>(rd + 4096 + off);
+      }
+      // into the stage that step kt - 1 read (its MFMAs have its values)
+      if (FULL || kt + kRouterDepth < steps) issue(nx, kt + kRouterDepth);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
+                                                      __builtin_bit_cast(bf16x8_t, b[s]), acc, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    char* st[kRouterRing] = {s0, s1, s2, s3, s4, s5, s6, s7};
+#pragma unroll
+    for (int i = 0; i < kRouterDepth; ++i)
+      if (i < steps) issue(st[i], i);
+    int kt = 0;
+    for (; kt + kRouterRing - 1 + kRouterDepth < steps; kt += kRouterRing) {
+      step(s0, s7, kt, std::true_type{});
+      step(s1, s0, kt + 1, std::true_type{});
+      step(s2, s1, kt + 2, std::true_type{});
+      step(s3, s2, kt + 3, std::true_type{});
+      step(s4, s3, kt + 4, std::true_type{});
+      step(s5, s4, kt + 5, std::true_type{});
+      step(s6, s5, kt + 6, std::true_type{});
+      step(s7, s6, kt + 7, std::true_type{});
+    }
+    for (; kt < steps; kt += kRouterRing) {
+      step(s0, s7, kt, std::false_type{});
+      if (kt + 1 < steps) step(s1, s0, kt + 1, std::false_type{});
+      if (kt + 2 < steps) step(s2, s1, kt + 2, std::false_type{});
+      if (kt + 3 < steps) step(s3, s2, kt + 3, std::false_type{});
+      if (kt + 4 < steps) step(s4, s3, kt + 4, std::false_type{});
+      if (kt + 5 < steps) step(s5, s4, kt + 5, std::false_type{});
+      if (kt + 6 < steps) step(s6, s5, kt + 6, std::false_type{});
+      if (kt + 7 < steps) step(s7, s6, kt + 7, std::false_type{});
+    }
+  };
+  auto st = [&](int i) { return lds + i * kRouterStage; };
+  body(st(0), st(1), st(2), st(3), st(4), st(5), st(6), st(7));
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const int64_t t = t0 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    const int64_t t = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
     if (t < tokens) out[t * experts + e0 + r] = (uint16_t)f32_to_bf16(acc[i]);
   }
+#endif
 }
 
 hipError_t launch_router_gate(const uint16_t* x, const uint16_t* w, int64_t tokens, int hidden, int experts,
                               uint16_t* out, hipStream_t stream) {
   const int64_t blocks = (tokens + 31) / 32;
   if (blocks == 0) return hipSuccess;
-  router_gate_kernel<<<(unsigned)blocks, 256, 0, stream>>>(x, w, tokens, hidden, experts, out);
+  const int64_t grid = (blocks + 7) / 8 * 8 * (experts / 32);
+  router_gate_kernel<<<(unsigned)grid, 64, 0, stream>>>(x, w, tokens, hidden, experts, out);
   return hipGetLastError();
 }
 

@@ -111,3 +111,16 @@ def test_router_logits_one_hot_weights_are_exact():
     w[np.arange(experts), cols] = 0x3F80  # 1.0
     got = host_u16(clef_i4.router_logits(dev_bf16(x), dev_bf16(w)))
     assert np.array_equal(got, x[:, cols])
+
+
+@pytest.mark.parametrize("tokens,hidden,experts", [(1, 64, 32), (33, 448, 128), (32, 512, 96), (65, 960, 64),
+                                                   (300, 1024, 128), (5, 4096, 32)])
+def test_router_logits_integer_inputs_are_exact(tokens, hidden, experts):
+    """Small integer inputs make every f32 partial sum exact, so the logits
+    equal bf16 of the integer dot product: fewer k-steps than the load ring
+    holds, ring remainders, partial token blocks and each expert group count."""
+    rng = np.random.default_rng(tokens * 7 + hidden)
+    x = rng.integers(-4, 5, (tokens, hidden)).astype(np.float32)
+    w = rng.integers(-3, 4, (experts, hidden)).astype(np.float32)
+    got = host_u16(clef_i4.router_logits(dev_bf16(BF(x)), dev_bf16(BF(w))))
+    assert np.array_equal(got, BF(x @ w.T))
