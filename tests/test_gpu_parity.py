@@ -1188,6 +1188,75 @@ def test_gemm_f6_gate_up_silu_window_edges():
     assert_same_u16(bf16_host(got), want, "gate_up window edges vs oracle")
 
 
+# (m, n, k): every bf6 kernel at its edges. Split-K tiles of 32 x 32, 32 x 64
+# and 64 x 64 (fewer k-steps than waves, uneven and several rounds per wave,
+# ragged rows); persistent tiles of 128 x 128, 128 x 256 and 256 x 256 with
+# fewer k-steps than ring stages, exactly as many, one more, and several tiles
+# per workgroup.
+F6_PATHS = [(1, 256, 256), (33, 1024, 1280), (64, 2048, 2304), (100, 4096, 512), (200, 2048, 1792),
+            (250, 4096, 768), (140, 7168, 2304),
+            (300, 4096, 256), (300, 4096, 512), (385, 4096, 768), (300, 4096, 1024), (100, 66048, 1024),
+            (600, 8192, 256), (600, 8192, 512), (577, 8192, 768), (620, 22016, 768),
+            (1030, 8192, 256), (1100, 8192, 768), (2100, 8192, 1280)]
+
+
+def _f6_path_operands(m, n, k, weights):
+    """x with a NaN row, an infinite value and a -0 row; weights whose rows
+    reach tiny, large and zero scales; the host forms for the oracle."""
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n + k)
+    x = torch.randn((m, k), generator=g, device="cuda", dtype=torch.bfloat16)
+    if m > 40:
+        x[m - 5] = float("nan")
+        x[37, 3] = float("inf")
+        x[m - 2] = -0.0
+    qs = []
+    for _ in range(weights):
+        w = torch.randn((n, k), generator=g, device="cuda", dtype=torch.bfloat16) * 0.02
+        w[64:80] *= 1e-4
+        w[80:96] *= 300.0
+        w[96:98] = 0.0
+        qs.append(clef_i4.load_quantized_weight(w))
+    rows = sorted({0, 1 % m, m // 3, m - 1, min(37, m - 1), max(m - 5, 0), max(m - 2, 0), min(127, m - 1),
+                   min(128, m - 1), min(256, m - 1)})
+    a_codes, a_scales, _ = oracle.prepare(bf16_host(x[rows]), oracle.activation_stride(k))
+    host = [(u32_host(q.codes), q.scales.cpu().numpy()) for q in qs]
+    return x, qs, rows, a_codes, a_scales, host
+
+
+@pytest.mark.parametrize("m,n,k", F6_PATHS)
+@pytest.mark.parametrize("resid", [False, True])
+def test_gemm_f6_every_path(m, n, k, resid):
+    """All rows bit-equal to the INT4-operand GEMM, sampled rows to the oracle."""
+    x, (q,), rows, a_codes, a_scales, host = _f6_path_operands(m, n, k, 1)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    res = torch.randn((m, n), generator=g, device="cuda", dtype=torch.bfloat16) if resid else None
+    fw, a = clef_i4.f6_weight(q), clef_i4.prepare_f6(x)
+    want = bf16_host(clef_i4.project_prepared(clef_i4.prepare(x), q, residual=res))
+    for _ in range(2):
+        got = bf16_host(clef_i4.project_f6(a, fw, residual=res))
+        assert_same_bf16_nan_aware(got, want, f"gemm_f6 m={m} n={n} k={k}")
+    sub = oracle.gemm(a_codes, a_scales, *host[0], n, k, residual=bf16_host(res)[rows] if resid else None)
+    assert_same_bf16_nan_aware(got[rows], sub, "gemm_f6 sampled rows vs oracle")
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 256, 256), (31, 1024, 1280), (64, 4096, 768), (100, 2304, 2304),
+                                   (100, 12288, 256), (90, 12288, 768), (90, 12288, 2048), (257, 4096, 512),
+                                   (128, 17408, 512), (385, 8192, 256), (400, 8192, 1024), (620, 12288, 768),
+                                   (300, 12288, 256), (400, 12288, 1280), (1100, 12288, 512)])
+def test_gemm_f6_gate_up_every_path(m, n, k):
+    """The fused gate/up on each kernel: all rows bit-equal to the unfused
+    INT4-operand path, sampled rows to the oracle."""
+    x, (qg, qu), rows, a_codes, a_scales, host = _f6_path_operands(m, n, k, 2)
+    a = clef_i4.prepare(x)
+    want = bf16_host(clef_i4.swiglu(clef_i4.project_prepared(a, qg), clef_i4.project_prepared(a, qu)))
+    fg, fu, af = clef_i4.f6_weight(qg), clef_i4.f6_weight(qu), clef_i4.prepare_f6(x)
+    for _ in range(2):
+        got = bf16_host(clef_i4.project_gate_up_f6(af, fg, fu))
+        assert_same_bf16_nan_aware(got, want, f"gate_up m={m} n={n} k={k}")
+    sub = oracle.swiglu(*(oracle.gemm(a_codes, a_scales, *h, n, k) for h in host))
+    assert_same_bf16_nan_aware(got[rows], sub, "gate_up sampled rows vs oracle")
+
+
 def test_gemm_f6_gate_up_rejects():
     fw = clef_i4.F6Weight(torch.zeros(192 * 256 * 3 // 4, dtype=torch.uint8, device="cuda"),
                           torch.ones(192, device="cuda"), 192, 256)
