@@ -40,6 +40,7 @@ SIGNATURES = {
     "clef_i4_retile": (ctypes.c_int, [_P, _I64, _I32, _I32, _I32, _P, _P]),
     "clef_i4_pack_weight_workspace_bytes": (_SZ, [_I64, _I32, _I32]),
     "clef_i4_pack_weight": (ctypes.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _SZ, _P]),
+    "clef_i4_pack_checkpoint": (ctypes.c_int, [_P, _I64, _I32, _I32, _I32, _P, _P, _P]),
     "clef_untile_rows": (ctypes.c_int, [_P, _I64, _I32, _P, _P]),
     "clef_tile_rows": (ctypes.c_int, [_P, _I64, _I32, _P, _P]),
     "clef_i4_gemm": (ctypes.c_int, [_P, _I32, _P, _P, _P, _I64, _I32, _I32, _P, _P, _P]),
@@ -409,16 +410,10 @@ def load_quantized_weight(w: torch.Tensor, bits: int = 4, tiled_checkpoint: bool
 
 def _pack(w: torch.Tensor, bits: int, tiled_checkpoint: bool) -> QuantizedWeight:
     rows, cols = w.shape
-    if tiled_checkpoint:
-        dense = torch.empty_like(w)
-        _check(lib().clef_untile_rows(_ptr(w), rows, cols, _ptr(dense), _stream()))
-        w = dense
     codes = torch.empty(rows * cols // (32 // bits), dtype=torch.int32, device=w.device)
     scales = torch.empty(rows, dtype=torch.float32, device=w.device)
-    ws_bytes = int(lib().clef_i4_pack_weight_workspace_bytes(rows, cols, bits))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=w.device)
-    _check(lib().clef_i4_pack_weight(_ptr(w), rows, cols, bits, _ptr(codes), _ptr(scales), _ptr(ws),
-                                     ws_bytes, _stream()))
+    _check(lib().clef_i4_pack_checkpoint(_ptr(w), rows, cols, bits, int(tiled_checkpoint), _ptr(codes), _ptr(scales),
+                                         _stream()))
     return QuantizedWeight(codes, scales, rows, cols, activation_stride(cols, bits), bits)
 
 

@@ -31,6 +31,11 @@ int hip_status(hipError_t e) {
 
 bool aligned(const void* p, size_t a) { return p && (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
+bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + b_bytes && y < x + a_bytes;
+}
+
 hipStream_t hs(clef_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 constexpr const char* kAlign = "device pointer is NULL or not 16-byte aligned";
@@ -179,6 +184,10 @@ int clef_i4_pack_weight(const uint16_t* w, int64_t rows, int32_t cols, int32_t b
   if (!aligned(w, 16) || !aligned(tiled, 16) || !aligned(scales, 4) || !aligned(workspace, 16))
     return fail(kAlign);
   if (workspace_bytes < clef_i4_pack_weight_workspace_bytes(rows, cols, bits)) return fail(kWorkspace);
+  const size_t in_bytes = (size_t)rows * cols * 2, out_bytes = (size_t)rows * cols * bits / 8;
+  if (!overlap(w, in_bytes, tiled, out_bytes) && !overlap(w, in_bytes, scales, (size_t)rows * 4))
+    return hip_status(clef::launch_pack_weight(w, rows, cols, bits, false, tiled, scales, hs(stream)));
+  // packing over the weight itself: through the row-major codes in the workspace
   uint32_t* staging = static_cast<uint32_t*>(workspace);
   const int32_t words = stride / (32 / bits);
   if (int rc = hip_status(clef::launch_prepare(w, rows, cols, stride, bits, staging, hs(stream))))
@@ -187,6 +196,19 @@ int clef_i4_pack_weight(const uint16_t* w, int64_t rows, int32_t cols, int32_t b
     return rc;
   return hip_status(hipMemcpyAsync(scales, staging + rows * words, (size_t)rows * 4,
                                    hipMemcpyDeviceToDevice, hs(stream)));
+}
+
+int clef_i4_pack_checkpoint(const uint16_t* w, int64_t rows, int32_t cols, int32_t bits,
+                            int32_t checkpoint_tiled, uint32_t* tiled, float* scales, clef_stream_t stream) {
+  if (checkpoint_tiled && !(rows > 0 && cols > 0 && rows % 256 == 0 && cols % 64 == 0))
+    return fail("tiled layout requires 256-row and 64-column multiples");
+  if (checkpoint_tiled && !aligned(w, 16)) return fail(kAlign);
+  if (!(rows > 0 && cols > 0 && rows % 256 == 0 && cols % 256 == 0))
+    return fail("unsupported quantized weight shape");
+  if (int rc = check_prepare(rows, cols, stride_for(cols, bits), bits)) return rc;
+  if (!aligned(w, 16) || !aligned(tiled, 16) || !aligned(scales, 4)) return fail(kAlign);
+  return hip_status(
+      clef::launch_pack_weight(w, rows, cols, bits, checkpoint_tiled != 0, tiled, scales, hs(stream)));
 }
 
 int clef_untile_rows(const uint16_t* tiled, int64_t rows, int32_t cols, uint16_t* out,

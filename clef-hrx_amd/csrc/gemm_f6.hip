@@ -56,17 +56,39 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 typedef unsigned f6_v2u __attribute__((ext_vector_type(2)));
 typedef unsigned f6_v4u __attribute__((ext_vector_type(4)));
 
+// e3m2 values of the codes in the low nibbles of n's four bytes, one per byte:
+// two 8-entry table lookups (codes 0..7 and -8..-1 by their low three bits)
+// and a select by the sign nibble bit.
+__device__ __forceinline__ uint32_t f6_bytes(uint32_t n) {
+  constexpr auto four = [](uint32_t a) {
+    uint32_t t = 0;
+    for (uint32_t i = 0; i < 4; ++i) t |= e3m2_of_nibble(a + i) << (8 * i);
+    return t;
+  };
+  constexpr uint32_t p0 = four(0), p1 = four(4), n0 = four(8), n1 = four(12);
+  const uint32_t sel = n & 0x07070707u;
+  const uint32_t pos = __builtin_amdgcn_perm(p1, p0, sel), neg = __builtin_amdgcn_perm(n1, n0, sel);
+  const uint32_t mask = ((n >> 3) & 0x01010101u) * 0xFFu;
+  return (neg & mask) | (pos & ~mask);
+}
+
 // 32 codes (four packed words, code j in nibble j % 8 of word j / 8) -> 32
 // e3m2 values, value j at bits 6j of out[0..5].
 __device__ __forceinline__ void f6_pack32(const uint32_t (&w)[4], uint32_t (&out)[6]) {
+  uint32_t q[8];  // 24 bits each: values 4i .. 4i + 3
 #pragma unroll
-  for (int d = 0; d < 6; ++d) out[d] = 0;
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t ev = f6_bytes(w[i] & 0x0F0F0F0Fu), od = f6_bytes((w[i] >> 4) & 0x0F0F0F0Fu);
+    const uint32_t p02 = (ev & 0x00FF00FFu) | ((od & 0x00FF00FFu) << 6);                // pairs 0 and 2 of the word
+    const uint32_t p13 = ((ev >> 8) & 0x00FF00FFu) | ((od >> 2) & 0x3FC03FC0u);         // pairs 1 and 3
+    q[2 * i] = (p02 & 0xFFFFu) | ((p13 & 0xFFFFu) << 12);
+    q[2 * i + 1] = (p02 >> 16) | ((p13 >> 16) << 12);
+  }
 #pragma unroll
-  for (int j = 0; j < 32; ++j) {
-    const uint32_t v = e3m2_of_nibble((w[j >> 3] >> (4 * (j & 7))) & 15u);
-    const int bit = 6 * j, d = bit >> 5, sh = bit & 31;
-    out[d] |= v << sh;
-    if (sh > 26) out[d + 1] |= v >> (32 - sh);
+  for (int i = 0; i < 2; ++i) {
+    out[3 * i] = q[4 * i] | (q[4 * i + 1] << 24);
+    out[3 * i + 1] = (q[4 * i + 1] >> 8) | (q[4 * i + 2] << 16);
+    out[3 * i + 2] = (q[4 * i + 2] >> 16) | (q[4 * i + 3] << 8);
   }
 }
 
@@ -91,23 +113,20 @@ __global__ __launch_bounds__(256) void f6_rows_kernel(const uint32_t* __restrict
 }
 
 // Tiled INT4 weight (the reference layout: 128-row x 256-k blocks of 32 words
-// per row) -> bf6 tiled weight (header comment); one thread per 32 codes.
-__global__ __launch_bounds__(256) void f6_tiled_kernel(const uint32_t* __restrict__ w, int64_t n, int k,
+// per row) -> bf6 tiled weight (header comment); one thread per 32 codes, in
+// the order of the INT4 weight, so that a wave reads one KiB and writes two
+// runs of 768 bytes (8 rows of each 128-k block). Codes through byte-permute
+// tables: 12288 x 4096 23.5 -> 13.9 us.
+__global__ __launch_bounds__(256) void f6_tiled_kernel(const uint32_t* __restrict__ w, int64_t total,
                                                        uint8_t* __restrict__ out) {
-  const int groups = k / 32;
-  const int kb4 = k / 256, kb6 = k / 128;
-  const int64_t total = n * groups;
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t row = t / groups;
-    const int g = (int)(t - row * groups);
-    const int64_t panel = row / 128;
-    const int r = (int)(row % 128);
-    const int q = 4 * g;  // first word of the group in the row
-    const uint4 in = *reinterpret_cast<const uint4*>(w + (panel * kb4 + q / 32) * 4096 + r * 32 + q % 32);
+    const uint4 in = reinterpret_cast<const uint4*>(w)[t];
+    const int g = (int)(t & 7), r = (int)(t >> 3) & 127;
+    const int64_t block = t >> 10;  // panel * kb4 + 256-k block: its two 128-k blocks are 2 block, 2 block + 1
     const uint32_t wv[4] = {in.x, in.y, in.z, in.w};
     uint32_t o[6];
     f6_pack32(wv, o);
-    uint8_t* blk = out + (panel * kb6 + g / 4) * 12288 + r * 96;
+    uint8_t* blk = out + (2 * block + (g >> 2)) * 12288 + r * 96;
     const int s = (r >> 3) & 1;
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
@@ -1114,7 +1133,7 @@ hipError_t launch_f6_rows(const uint32_t* a, int a_words, int64_t rows, int k, u
 hipError_t launch_f6_tiled(const uint32_t* w_tiled, int64_t n, int k, uint8_t* out, hipStream_t stream) {
   const int64_t total = n * (k / 32);
   const int64_t blocks = (total + 255) / 256;
-  f6_tiled_kernel<<<(unsigned)(blocks < 8192 ? blocks : 8192), 256, 0, stream>>>(w_tiled, n, k, out);
+  f6_tiled_kernel<<<(unsigned)(blocks < 8192 ? blocks : 8192), 256, 0, stream>>>(w_tiled, total, out);
   return hipGetLastError();
 }
 

@@ -42,6 +42,10 @@ hipError_t launch_prepare_attention_gate(const uint16_t* x, const uint16_t* q_ga
                                          int stride, int bits, uint32_t* out, hipStream_t stream);
 hipError_t launch_prepare_norm(const uint16_t* x, const uint16_t* weight, int64_t rows, int width, int stride,
                                int bits, uint32_t* out, uint16_t* normalized, hipStream_t stream);
+// Q1 of a weight (rows of a checkpoint-tiled matrix when checkpoint_tiled)
+// with the codes stored in the tiled layout, scales [rows].
+hipError_t launch_pack_weight(const uint16_t* w, int64_t rows, int cols, int bits, bool checkpoint_tiled,
+                              uint32_t* tiled, float* scales, hipStream_t stream);
 hipError_t launch_retile(const uint32_t* codes, int64_t rows, int in_words, int words,
                          uint32_t* tiled, hipStream_t stream);
 hipError_t launch_tile_permute(const uint16_t* src, int64_t rows, int cols, uint16_t* dst,

@@ -60,6 +60,29 @@ struct PlainSource {
   }
 };
 
+// A weight in the checkpoint's tiling [rows/256][cols/64][256][64]
+// (src/checkpoint.rs:24-32): a lane's 16 values lie in one 64-column piece, so
+// the rows are read where they stand instead of being untiled first.
+struct CheckpointSource {
+  static constexpr bool kRowNorm = false;
+  static constexpr bool kLdsTable = false;
+  const uint16_t* x;
+  int width;
+  using Raw = PlainSource::Raw;
+  __device__ __forceinline__ Raw fetch(int64_t row, int col) const {
+    // a tile's 256 rows take 256 * width values in either layout; 64-column
+    // piece ks of row r at (ks * 256 + r) * 64
+    return PlainSource{x}.fetch((row >> 8) * 256 * width + (row & 255) * 64, (col >> 6) * 16384 + (col & 63));
+  }
+  __device__ __forceinline__ void convert(const Raw& r, float* v) const { PlainSource{x}.convert(r, v); }
+  __device__ __forceinline__ void load16(int64_t row, int col, float* v) const { convert(fetch(row, col), v); }
+};
+// Whether fetch takes the row instead of its element offset.
+template <class Src>
+constexpr bool kFetchByRow = false;
+template <>
+constexpr bool kFetchByRow<CheckpointSource> = true;
+
 // S1 applied on load (kernels/prepare_integer_register.loom:155-172): the
 // rotation sees f32(bf16(swiglu)) exactly as if h had been materialized.
 struct SwigluSource {
@@ -249,14 +272,22 @@ __device__ __forceinline__ void store_codes_f6(uint32_t* out, int64_t row, int c
 }
 
 // Codes of one 16-value group, in the output layout of BITS (out_row: the
-// row's first word for BITS 4 and 8; out: the whole buffer for bf6).
-template <int BITS>
+// row's first word for BITS 4 and 8; out: the whole buffer for bf6). TILED
+// (BITS 4 and 8): the weight layout of Q2, word (n, q) at ((n / 128) * blocks_k
+// + q / 32) * 4096 + (n % 128) * 32 + q % 32 (kernels/retile_codes.loom:2-5);
+// a lane's 16 values stay inside one 32-word piece.
+template <int BITS, bool TILED>
 __device__ __forceinline__ void store_group(uint32_t* out, uint32_t* out_row, int64_t row, int col, int width,
                                             const float* nat, float inv, bool valid) {
-  if constexpr (BITS == 6)
+  if constexpr (BITS == 6) {
     store_codes_f6(out, row, col, width, nat, inv, valid);
-  else
+  } else if constexpr (TILED) {
+    constexpr int kPiece = 32 * 32 / BITS;  // columns of a 32-word piece
+    const int64_t block = (row >> 7) * (width / kPiece) + col / kPiece;
+    store_codes<BITS>(out + block * 4096 + (row & 127) * 32, col % kPiece, nat, inv, valid);
+  } else {
     store_codes<BITS>(out_row, col, nat, inv, valid);
+  }
 }
 
 // Where a prepared buffer's f32 row scales start.
@@ -266,9 +297,11 @@ __device__ __forceinline__ float* scales_of(uint32_t* out, int64_t rows, int wid
   return reinterpret_cast<float*>(out + rows * out_words);
 }
 
-template <int P, int BITS, class Src>
+// TILED: codes in the weight layout (store_group), row scales to `wscales`.
+template <int P, int BITS, class Src, bool TILED>
 __global__ __launch_bounds__(256) void prepare_kernel(Src src, int64_t rows, int width,
-                                                      int out_words, uint32_t* __restrict__ out) {
+                                                      int out_words, uint32_t* __restrict__ out,
+                                                      float* __restrict__ wscales) {
   __shared__ __align__(16) float lds[16 * kGroupLds];
   __shared__ uint32_t gmax[16];
   const int tid = threadIdx.x;
@@ -321,7 +354,7 @@ __global__ __launch_bounds__(256) void prepare_kernel(Src src, int64_t rows, int
     for (int p = 0; p < P; ++p) {
       const int grp = grp0 + 16 * p;
       if (active && grp < G) {
-        src.load16(row * width, grp * 256 + 16 * L, v[p]);
+        src.load16(kFetchByRow<Src> ? row : row * width, grp * 256 + 16 * L, v[p]);
       } else {
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[p][i] = 0.0f;
@@ -396,9 +429,9 @@ __global__ __launch_bounds__(256) void prepare_kernel(Src src, int64_t rows, int
       nat[4 * c + 3] = t.w;
     }
     group_lds_order();
-    if (on) store_group<BITS>(out, out + row * out_words, row, grp * 256 + 16 * L, width, nat, inv, valid);
+    if (on) store_group<BITS, TILED>(out, out + row * out_words, row, grp * 256 + 16 * L, width, nat, inv, valid);
   }
-  if (active && grp0 == 0 && L == 0) scales_of<BITS>(out, rows, width, out_words)[row] = scale;
+  if (active && grp0 == 0 && L == 0) (TILED ? wscales : scales_of<BITS>(out, rows, width, out_words))[row] = scale;
 }
 
 // Rows of G <= 16 groups, as prepare_kernel<1> but persistent: a workgroup
@@ -406,9 +439,10 @@ __global__ __launch_bounds__(256) void prepare_kernel(Src src, int64_t rows, int
 // block's inputs before rotating and packing the current one, so HBM latency
 // overlaps the work instead of being paid once per workgroup.
 // The body runs as workgroup `block` of `nblocks` walking the row blocks.
-template <int BITS, class Src>
+template <int BITS, class Src, bool TILED>
 __device__ __forceinline__ void prepare_loop_body(Src src, int64_t rows, int width, int out_words,
-                                                  uint32_t* __restrict__ out, int64_t block, int64_t nblocks) {
+                                                  uint32_t* __restrict__ out, float* __restrict__ wscales,
+                                                  int64_t block, int64_t nblocks) {
   // 20 KiB: eight workgroups fill a CU's LDS. Each group's maximum goes to
   // the padding float of its first LDS row, which the transposes never touch.
   __shared__ __align__(16) float lds[16 * kGroupLds];
@@ -434,7 +468,7 @@ __device__ __forceinline__ void prepare_loop_body(Src src, int64_t rows, int wid
   int64_t row = blk * rows_per_block + row_local;
   int64_t in_off = row * width, out_off = row * out_words;
   typename Src::Raw raw{};
-  if (lane_on && row < rows) raw = src.fetch(in_off, col);
+  if (lane_on && row < rows) raw = src.fetch(kFetchByRow<Src> ? row : in_off, col);
   for (; blk < nblk; blk += nblocks, row += step, in_off += in_step, out_off += out_step) {
     const bool on = lane_on && row < rows;
     float v[16];
@@ -444,7 +478,7 @@ __device__ __forceinline__ void prepare_loop_body(Src src, int64_t rows, int wid
 #pragma unroll
       for (int i = 0; i < 16; ++i) v[i] = 0.0f;
     }
-    if (lane_on && row + step < rows) raw = src.fetch(in_off + in_step, col);
+    if (lane_on && row + step < rows) raw = src.fetch(kFetchByRow<Src> ? row + step : in_off + in_step, col);
     radix4x2(v);  // strides 1 and 4
     float4* wrow = reinterpret_cast<float4*>(buf + L * kPitch);
 #pragma unroll
@@ -506,16 +540,16 @@ __device__ __forceinline__ void prepare_loop_body(Src src, int64_t rows, int wid
     // every wave reaches after reading this iteration's scale.
     group_lds_order();
     if (on) {
-      store_group<BITS>(out, out + out_off, row, col, width, nat, inv, valid);
-      if (grp == 0 && L == 0) scales_of<BITS>(out, rows, width, out_words)[row] = scale;
+      store_group<BITS, TILED>(out, out + out_off, row, col, width, nat, inv, valid);
+      if (grp == 0 && L == 0) (TILED ? wscales : scales_of<BITS>(out, rows, width, out_words))[row] = scale;
     }
   }
 }
 
-template <int BITS, class Src>
+template <int BITS, class Src, bool TILED>
 __global__ __launch_bounds__(256) void prepare_loop_kernel(Src src, int64_t rows, int width, int out_words,
-                                                           uint32_t* __restrict__ out) {
-  prepare_loop_body<BITS, Src>(src, rows, width, out_words, out, blockIdx.x, gridDim.x);
+                                                           uint32_t* __restrict__ out, float* __restrict__ wscales) {
+  prepare_loop_body<BITS, Src, TILED>(src, rows, width, out_words, out, wscales, blockIdx.x, gridDim.x);
 }
 
 // The router and the INT4 quantizer of the MoE input in one launch: the first
@@ -561,13 +595,13 @@ __global__ __launch_bounds__(256) void route_prepare_kernel(const void* __restri
     route_impl::route_block(logits, dtype, tokens, experts, topk, routes, blockIdx.x);
     return;
   }
-  prepare_loop_body<4, PlainSource>(src, tokens, width, out_words, out, blockIdx.x - route_blocks,
-                                    gridDim.x - route_blocks);
+  prepare_loop_body<4, PlainSource, false>(src, tokens, width, out_words, out, nullptr, blockIdx.x - route_blocks,
+                                           gridDim.x - route_blocks);
 }
 
-template <int BITS, class Src>
+template <int BITS, bool TILED = false, class Src>
 hipError_t launch_prepare_bits(const Src& src, int64_t rows, int width, int out_words,
-                               uint32_t* out, hipStream_t stream) {
+                               uint32_t* out, hipStream_t stream, float* wscales = nullptr) {
   const int G = width / 256;
   if (G <= 16 && !Src::kRowNorm) {
     const int per_block = 16 / G;
@@ -576,13 +610,13 @@ hipError_t launch_prepare_bits(const Src& src, int64_t rows, int width, int out_
     // that are walked by the grid stride.
     const unsigned grid = (unsigned)(blocks < 2048 ? blocks : 2048);
     if constexpr (!Src::kRowNorm)
-      prepare_loop_kernel<BITS, Src><<<grid, 256, 0, stream>>>(src, rows, width, out_words, out);
+      prepare_loop_kernel<BITS, Src, TILED><<<grid, 256, 0, stream>>>(src, rows, width, out_words, out, wscales);
   } else {
     const int passes = (G + 15) / 16;
     const unsigned grid = (unsigned)rows;
     switch (passes) {
 #define CLEF_PREP_CASE(N) \
-  case N: prepare_kernel<N, BITS, Src><<<grid, 256, 0, stream>>>(src, rows, width, out_words, out); break;
+  case N: prepare_kernel<N, BITS, Src, TILED><<<grid, 256, 0, stream>>>(src, rows, width, out_words, out, wscales); break;
       CLEF_PREP_CASE(2)
       CLEF_PREP_CASE(3)
       CLEF_PREP_CASE(4)
@@ -663,6 +697,22 @@ __global__ __launch_bounds__(256) void tile_permute_kernel(const uint16_t* __res
 hipError_t launch_prepare(const uint16_t* x, int64_t rows, int width, int stride, int bits,
                           uint32_t* out, hipStream_t stream) {
   return launch_prepare_src(PlainSource{x}, rows, width, stride, bits, out, stream);
+}
+
+// Weight packing: Q1 with the codes stored in the tiled layout, one pass over
+// the weight. As three passes (untile, Q1 to row-major codes, retile) plus the
+// copy of the scales, 12288 x 4096 took 28.5 + 30.8 + 10.1 + 4.6 us; this one
+// takes 33.1-36.0 from the checkpoint tiling (3.5-3.8 TB/s).
+hipError_t launch_pack_weight(const uint16_t* w, int64_t rows, int cols, int bits, bool checkpoint_tiled,
+                              uint32_t* tiled, float* scales, hipStream_t stream) {
+  if (checkpoint_tiled) {
+    const CheckpointSource src{w, cols};
+    return bits == 4 ? launch_prepare_bits<4, true>(src, rows, cols, 0, tiled, stream, scales)
+                     : launch_prepare_bits<8, true>(src, rows, cols, 0, tiled, stream, scales);
+  }
+  const PlainSource src{w};
+  return bits == 4 ? launch_prepare_bits<4, true>(src, rows, cols, 0, tiled, stream, scales)
+                   : launch_prepare_bits<8, true>(src, rows, cols, 0, tiled, stream, scales);
 }
 
 bool route_prepare_fusable(int width) { return width % 256 == 0 && width / 256 <= 16; }

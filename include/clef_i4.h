@@ -132,7 +132,8 @@ int clef_i4_prepare_norm(const uint16_t* x, const uint16_t* weight, int64_t rows
 int clef_i4_retile(const uint32_t* codes, int64_t rows, int32_t in_words, int32_t cols, int32_t bits,
                    uint32_t* tiled, clef_stream_t stream);
 
-/* Bytes of scratch clef_i4_pack_weight needs (the row-major packed staging). */
+/* Bytes of scratch clef_i4_pack_weight needs (the row-major packed staging,
+ * used when an output overlaps the weight). */
 size_t clef_i4_pack_weight_workspace_bytes(int64_t rows, int32_t cols, int32_t bits);
 
 /* bf16 weight [rows][cols] (logical row order) -> tiled codes
@@ -144,6 +145,14 @@ size_t clef_i4_pack_weight_workspace_bytes(int64_t rows, int32_t cols, int32_t b
 int clef_i4_pack_weight(const uint16_t* w, int64_t rows, int32_t cols, int32_t bits, uint32_t* tiled,
                         float* scales, void* workspace, size_t workspace_bytes,
                         clef_stream_t stream);
+
+/* The same from the rows as a checkpoint stores them: with checkpoint_tiled
+ * nonzero, w is in the 256x64-tiled layout of clef_untile_rows and is read
+ * where it stands (untile, quantize and retile in one pass, no workspace); w
+ * must not overlap the outputs. Preconditions: with checkpoint_tiled those of
+ * clef_untile_rows, then those of clef_i4_pack_weight. */
+int clef_i4_pack_checkpoint(const uint16_t* w, int64_t rows, int32_t cols, int32_t bits,
+                            int32_t checkpoint_tiled, uint32_t* tiled, float* scales, clef_stream_t stream);
 
 /* 256x64-tiled checkpoint layout [rows/256][cols/64][256][64] <-> logical
  * rows. Replace checkpoint::untile_rows / tile_rows (src/checkpoint.rs:63-106,

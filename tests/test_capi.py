@@ -74,6 +74,17 @@ def test_pack_weight_rejects():
     assert rc == -1 and msg == "workspace too small"
 
 
+@pytest.mark.parametrize("rows,cols,bits,tiled,want", [
+    (128, 256, 4, 0, "unsupported quantized weight shape"),
+    (256, 320, 4, 1, "unsupported quantized weight shape"),
+    (128, 256, 4, 1, "tiled layout requires 256-row and 64-column multiples"),
+    (256, 256, 5, 1, "unsupported rotated integer operand"),
+    (256, 33024, 8, 0, "unsupported rotated integer operand")])
+def test_pack_checkpoint_rejects(rows, cols, bits, tiled, want):
+    rc, msg = call("clef_i4_pack_checkpoint", FAKE, rows, cols, bits, tiled, FAKE, FAKE, None)
+    assert rc == -1 and msg == want
+
+
 @pytest.mark.parametrize("m,n,k,ks", [(0, 128, 256, 256), (4, 100, 256, 256), (4, 128, 300, 320),
                                       (4, 128, 256, 200), (4, 128, 256, 272)])
 def test_gemm_rejects(m, n, k, ks):

@@ -175,6 +175,43 @@ def test_pack_weight_matches_oracle():
         assert np.array_equal(qw.scales.cpu().numpy().view(np.uint32), want_scales.view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,cols", [(256, 256), (768, 1024), (512, 3840), (256, 4096), (512, 4352), (256, 12288)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_pack_checkpoint_matches_oracle(rows, cols, bits):
+    """Codes and scales of a weight read row by row and from the checkpoint
+    tiling, both quantizer kernels (rows of up to 16 groups and wider), against
+    the oracle; rows with a NaN, an infinity and zeros among them."""
+    rng = np.random.default_rng(rows + cols + bits)
+    w = randn_bf16(rng, (rows, cols), std=0.02)
+    w[3, 5] = 0x7FC0
+    w[131, cols - 1] = 0x7F80
+    w[200] = 0
+    want_codes, want_scales = oracle.pack_weight(w, bits=bits)
+    for src, tiled in ((w, False), (oracle.tile_rows(w), True)):
+        qw = clef_i4.load_quantized_weight(to_dev_bf16(src), bits=bits, tiled_checkpoint=tiled)
+        assert_same_u32(u32_host(qw.codes), want_codes, f"pack codes tiled={tiled}")
+        assert np.array_equal(qw.scales.cpu().numpy().view(np.uint32), want_scales.view(np.uint32))
+
+
+def test_pack_weight_over_its_own_input():
+    """clef_i4_pack_weight with codes that overlap the weight packs through
+    its workspace: the same codes and scales."""
+    rng = np.random.default_rng(8)
+    rows, cols = 512, 1024
+    w = randn_bf16(rng, (rows, cols), std=0.02)
+    want_codes, want_scales = oracle.pack_weight(w)
+    dev = to_dev_bf16(w)
+    scales = torch.empty(rows, dtype=torch.float32, device="cuda")
+    need = int(clef_i4.lib().clef_i4_pack_weight_workspace_bytes(rows, cols, 4))
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert clef_i4.lib().clef_i4_pack_weight(dev.data_ptr(), rows, cols, 4, dev.data_ptr(), scales.data_ptr(),
+                                             ws.data_ptr(), need, stream) == 0
+    codes = dev.view(torch.int16).view(-1)[: rows * cols // 4].view(torch.int32)
+    assert_same_u32(u32_host(codes), want_codes, "pack in place")
+    assert np.array_equal(scales.cpu().numpy().view(np.uint32), want_scales.view(np.uint32))
+
+
 def test_untile_rows_roundtrip():
     rng = np.random.default_rng(4)
     w = rng.integers(0, 1 << 16, size=(512, 192), dtype=np.uint16)
