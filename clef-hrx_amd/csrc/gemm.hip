@@ -970,10 +970,8 @@ hipError_t launch_expert_dmah(const uint32_t* a, int a_words, int64_t a_bytes, c
 // the row's 128-byte k-step, the lane -> k map of the LDS cores) with the
 // next k-step's loads in flight while the current one computes. The NW
 // partial accumulators meet in LDS by integer atomic adds (exact in any
-// order), and the G1 epilogue runs on the sums. I8: INT8 operands (k-steps of
-// 128 k, the same 64 bytes per lane; each 16-byte chunk is an MFMA operand as
-// it stands, and the accumulator is the dot product itself).
-template <int MT, int NW, bool RESID, bool I8>
+// order), and the G1 epilogue runs on the sums.
+template <int MT, int NW, bool RESID>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint32_t* __restrict__ a, int a_words,
                                                           const float* __restrict__ as, const uint32_t* __restrict__ w,
                                                           const float* __restrict__ ws, int64_t M, int N, int kb,
@@ -1014,13 +1012,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint32_t* __
   };
   auto compute = [&](auto buf) {
     constexpr int B = decltype(buf)::value;
-    if constexpr (I8) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p)
-#pragma unroll
-        for (int f = 0; f < MT; ++f) acc[f] = mfma32_i8(wr[B][p], ar[B][f][p], acc[f]);
-      return;
-    }
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
@@ -1088,9 +1079,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint32_t* __
     const int col = n0 + 8 * rq + 4 * (ln >> 5);
     const float asv = PRE ? e_as[i] : as[m];
     const float4 wsv = PRE ? e_ws[i] : *reinterpret_cast<const float4*>(ws + col);
-    constexpr int SH = I8 ? 0 : 8;
-    uint32_t p0 = g1_value<SH>(red[f][4 * rq + 0][ln], wsv.x, asv) | (g1_value<SH>(red[f][4 * rq + 1][ln], wsv.y, asv) << 16);
-    uint32_t p1 = g1_value<SH>(red[f][4 * rq + 2][ln], wsv.z, asv) | (g1_value<SH>(red[f][4 * rq + 3][ln], wsv.w, asv) << 16);
+    uint32_t p0 = g1_value<8>(red[f][4 * rq + 0][ln], wsv.x, asv) | (g1_value<8>(red[f][4 * rq + 1][ln], wsv.y, asv) << 16);
+    uint32_t p1 = g1_value<8>(red[f][4 * rq + 2][ln], wsv.z, asv) | (g1_value<8>(red[f][4 * rq + 3][ln], wsv.w, asv) << 16);
     uint16_t* dst = out + m * N + col;
     if (RESID) {
       const uint2 rv = PRE ? e_res[i] : *reinterpret_cast<const uint2*>(residual + m * N + col);
@@ -1102,30 +1092,29 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint32_t* __
 #endif
 }
 
-template <int MT, bool RESID, bool I8>
+template <int MT, bool RESID>
 hipError_t launch_skinny(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,
                          int64_t m, int n, int k, const uint16_t* residual, uint16_t* out, hipStream_t stream) {
   const int64_t groups = (m + 32 * MT - 1) / (32 * MT);
   if (groups > 65535) return hipErrorInvalidValue;
   constexpr int NW = MT == 4 ? 8 : 16;  // four row blocks need 256 VGPRs: two waves per SIMD
-  gemm_skinny_kernel<MT, NW, RESID, I8><<<dim3((unsigned)(n / 32), (unsigned)groups), NW * 64, 0, stream>>>(
-      a, a_words, as, w, ws, m, n, I8 ? k / 128 : k / 256, residual, out);
+  gemm_skinny_kernel<MT, NW, RESID><<<dim3((unsigned)(n / 32), (unsigned)groups), NW * 64, 0, stream>>>(
+      a, a_words, as, w, ws, m, n, k / 256, residual, out);
   return hipGetLastError();
 }
 
-template <bool RESID, bool I8>
+template <bool RESID>
 hipError_t launch_skinny_m(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,
                            int64_t m, int n, int k, const uint16_t* residual, uint16_t* out, hipStream_t stream) {
-  if (m <= 32) return launch_skinny<1, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  if (m <= 64) return launch_skinny<2, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  return launch_skinny<4, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (m <= 32) return launch_skinny<1, RESID>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (m <= 64) return launch_skinny<2, RESID>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  return launch_skinny<4, RESID>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
 }
 
-template <bool I8 = false>
 hipError_t launch_skinny_any(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,
                              int64_t m, int n, int k, const uint16_t* residual, uint16_t* out, hipStream_t stream) {
-  if (residual) return launch_skinny_m<true, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  return launch_skinny_m<false, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (residual) return launch_skinny_m<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  return launch_skinny_m<false>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
 }
 
 // Decode-sized G1 (M <= MR <= 8) on the VALU. v_dot8_i32_i4 multiplies eight
@@ -1279,7 +1268,8 @@ hipError_t launch_decode(const uint32_t* a, int a_words, const float* as, const 
 // wave order, and each thread runs the G1 epilogue on 8 consecutive columns of
 // one row (16-byte stores); consecutive threads take consecutive rows, so
 // their LDS reads are consecutive 16-byte slots.
-template <int MT, int NT, int NW, int NB, bool RESID>
+// I8: INT8 codes; a k-step is 128 k and a 16-byte read an MFMA operand.
+template <int MT, int NT, int NW, int NB, bool RESID, bool I8>
 __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const uint32_t* __restrict__ a, int a_words,
                                                           const float* __restrict__ as, const uint32_t* __restrict__ w,
                                                           const float* __restrict__ ws, int64_t M, int N, int kb,
@@ -1289,6 +1279,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const uint32_t* __
   constexpr int BM = 32 * MT, BN = 32 * NT;  // activation rows, weight rows of the tile
   constexpr int STAGE = (BM + BN) * 128;
   constexpr int NF = MT + NT;
+  constexpr int SHIFT = I8 ? 0 : 8;  // INT4 accumulators hold 256 x the dot product
   constexpr int CHUNKS = BM * NT * 4;        // 8-column row chunks of the tile
   constexpr int IPT = (CHUNKS + NW * 64 - 1) / (NW * 64);
   static_assert(NB * STAGE >= MT * NT * 4096, "a wave's accumulators fit its stages");
@@ -1351,11 +1342,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const uint32_t* __
 #pragma unroll
       for (int f = 0; f < NF; ++f) raw[f] = *reinterpret_cast<const uint4*>(stage + f * 4096 + off);
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
+      for (int half = 0; half < (I8 ? 1 : 2); ++half) {
         v4i u[NF];
 #pragma unroll
         for (int f = 0; f < NF; ++f)
-          u[f] = half ? unpack_pair(raw[f].z, raw[f].w) : unpack_pair(raw[f].x, raw[f].y);
+          u[f] = I8     ? __builtin_bit_cast(v4i, raw[f])
+                 : half ? unpack_pair(raw[f].z, raw[f].w)
+                        : unpack_pair(raw[f].x, raw[f].y);
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -1409,10 +1402,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const uint32_t* __
     }
     const float4 w0 = e_ws[i][0], w1 = e_ws[i][1];
     const float av = e_as[i];
-    uint32_t p[4] = {g1_value<8>(lo.x, w0.x, av) | (g1_value<8>(lo.y, w0.y, av) << 16),
-                     g1_value<8>(lo.z, w0.z, av) | (g1_value<8>(lo.w, w0.w, av) << 16),
-                     g1_value<8>(hi.x, w1.x, av) | (g1_value<8>(hi.y, w1.y, av) << 16),
-                     g1_value<8>(hi.z, w1.z, av) | (g1_value<8>(hi.w, w1.w, av) << 16)};
+    uint32_t p[4] = {g1_value<SHIFT>(lo.x, w0.x, av) | (g1_value<SHIFT>(lo.y, w0.y, av) << 16),
+                     g1_value<SHIFT>(lo.z, w0.z, av) | (g1_value<SHIFT>(lo.w, w0.w, av) << 16),
+                     g1_value<SHIFT>(hi.x, w1.x, av) | (g1_value<SHIFT>(hi.y, w1.y, av) << 16),
+                     g1_value<SHIFT>(hi.z, w1.z, av) | (g1_value<SHIFT>(hi.w, w1.w, av) << 16)};
     if (RESID) {
       const uint32_t rv[4] = {e_res[i].x, e_res[i].y, e_res[i].z, e_res[i].w};
 #pragma unroll
@@ -1423,34 +1416,37 @@ __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const uint32_t* __
 #endif
 }
 
-template <int MT, int NT, int NW, int NB>
+template <int MT, int NT, int NW, int NB, bool I8>
 hipError_t launch_ksplit_t(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,
                            int64_t m, int n, int k, const uint16_t* residual, uint16_t* out, hipStream_t stream) {
   const int64_t groups = (m + 32 * MT - 1) / (32 * MT);
   if (groups > 65535 || n % (32 * NT) != 0) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(n / (32 * NT)), (unsigned)groups);
   if (residual)
-    gemm_ksplit_kernel<MT, NT, NW, NB, true><<<grid, NW * 64, 0, stream>>>(a, a_words, as, w, ws, m, n, k / 256,
-                                                                          residual, out);
+    gemm_ksplit_kernel<MT, NT, NW, NB, true, I8>
+        <<<grid, NW * 64, 0, stream>>>(a, a_words, as, w, ws, m, n, k / (I8 ? 128 : 256), residual, out);
   else
-    gemm_ksplit_kernel<MT, NT, NW, NB, false><<<grid, NW * 64, 0, stream>>>(a, a_words, as, w, ws, m, n, k / 256,
-                                                                           residual, out);
+    gemm_ksplit_kernel<MT, NT, NW, NB, false, I8>
+        <<<grid, NW * 64, 0, stream>>>(a, a_words, as, w, ws, m, n, k / (I8 ? 128 : 256), residual, out);
   return hipGetLastError();
 }
 
+template <bool I8 = false>
 hipError_t launch_ksplit(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,
                          int64_t m, int n, int k, const uint16_t* residual, uint16_t* out, hipStream_t stream) {
-  // The largest tile that still gives about one per CU (>= 192 tiles), with
-  // 32-row tiles when m <= 32 (a 64-row tile would be half padding); else
-  // 32 x 32 tiles with two stages per wave. Measured (graph replay, us):
-  // M512 N2048 K2048 64x64 5.7 (32x64 7.2, 32x32 9.9); M16 N12288 K4096
-  // 32x64 4.7 (64x64 6.4); M64 N12288 K4096 64x64 6.9 (32x64 8.8); M64 N4096
-  // K4096 32x32 4.5 (32x64 4.8); M32 N4096 K12288 32x32 6.8 (32x64 8.7).
+  // The smallest tile that gives at most one per CU, else 64 x 64 (32 x 64 up
+  // to 32 rows, where half of a 64-row tile would be padding). Measured
+  // (graph replay, three weights in turn, us): M100 N5120 K17408 64x64 20.5
+  // (32x64, two rounds, 24.9); M37 N5120 K17408 32x64 16.0 against 32x32 18.6;
+  // M64 N4096 K4096 32x32 5.2 (32x64 5.4); M128 N4096 K4096 32x64 6.1. INT8:
+  // M64 N12288 K4096 64x64 13.1 (32x64 17.4, 32x32 20.3), M235 N4096 K4096
+  // 64x64 10.5 (13.7, 21.4), M64 N4096 K4096 32x32 7.1 (7.8, 10.2).
   auto tiles = [&](int bm, int bn) { return (m + bm - 1) / bm * (n / bn); };
-  if (m > 32 && tiles(64, 64) >= 192)
-    return launch_ksplit_t<2, 2, 8, 1>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  if (tiles(32, 64) >= 192) return launch_ksplit_t<1, 2, 8, 1>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  return launch_ksplit_t<1, 1, 8, 2>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (tiles(32, 32) <= 256)
+    return launch_ksplit_t<1, 1, 8, 2, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (m <= 32 || tiles(32, 64) <= 256)
+    return launch_ksplit_t<1, 2, 8, 1, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  return launch_ksplit_t<2, 2, 8, 1, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
 }
 
 // Grouped expert GEMM for few routed rows per expert (decode-sized batches),
@@ -2068,12 +2064,24 @@ int gemm_config_count() { return kGemmConfigs; }
 
 hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,
                           int64_t m, int n, int k, const uint16_t* residual, uint16_t* out, hipStream_t stream) {
-  // At most 8 rows: the dot-product kernel (v_dot4_i32_i8); up to 32 the skinny kernel with one 32-row
-  // block (graph replay, M1 N12288 K4096: 16.4 us against 24.2 for 128x128 tiles; at M64 the two-block
-  // form loses to 128x128 tiles, 34.1 us against 24.7, on the 50 MB INT8 weight).
-  if (m <= 8) return launch_decode<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  if (m <= 32) return launch_skinny_any<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  if (n % 256 == 0 && m >= 1024)
+  // Measured (graph replay, three weights in turn, us):
+  // At most 4 rows: the dot-product kernel (v_dot4_i32_i8; M4 N4096 K4096 5.8
+  // against 6.0 for the split-K tiles, M8 7.0 against 6.0, M8 N12288 K4096
+  // 13.2 against 10.2).
+  // Up to two rounds of 64 x 64 tiles: the split-K tiles (M16 N12288 K4096
+  // 10.3; M100 N12288 K12288 51.6 against 68.6 for the 128 x 128 ring; M400
+  // N4096 K4096 18.5 against 20.5, M620, three rounds, 26.2 against 21.2).
+  // Up to one round of 128 x 128 tiles: the ring kernel (M235 N12288 K4096
+  // 21.2 against 27.6 for the two-stage tiles, M1024 N4096 K12288 57.3
+  // against 76.2; two rounds M400 N12288 K4096 38.6 against 33.1).
+  // Else 256 x 256 tiles once there are 160 of them (M2048 N5120 K6144 75.7
+  // against 87.9 for 128 x 128; M2048 N4096 K4096, 128 tiles, 53.0 against
+  // 39.7), 128 x 128 below that.
+  auto tiles = [&](int b) { return (m + b - 1) / b * (n / b); };
+  if (m <= 4) return launch_decode<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (tiles(64) <= 512) return launch_ksplit<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (tiles(128) <= 256) return launch_gemm_i8_ring(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (n % 256 == 0 && m >= 1024 && tiles(256) >= 160)
     return launch_dma8_any<Dma256x256W8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
   return launch_dma8_any<Dma128x128>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
 }
@@ -2093,17 +2101,20 @@ hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const
     // M1 N4096 K4096 5.1 us against 17.4; M64 N12288 K4096 13.0 against
     // 17.8; M512 N2048 K2048 7.5 against 11.3; M128 N12288 K4096 29.1
     // against 18.3, where 96 tiles of 128x128 already cover most CUs).
-    // At most 8 rows: the VALU dot-product kernel (graph replay, weight in
-    // the last-level cache: M1 N12288 K4096 2.9 us against 8.4 for the
-    // skinny kernel, M8 6.6 against 8.2; M8 N2048 K2048 3.3 against 3.8).
-    // Up to 255 tiles of 128x128: the split-K tiles (M512 N2048 K2048 5.7 us
-    // against 7.4 for the skinny kernel and 11.4 for 128x128 tiles; M128
-    // N12288 K4096 12.6 against 18.3).
+    // At most 4 rows, or 8 where 32 x 32 split-K tiles would leave CUs idle:
+    // the VALU dot-product kernel (graph replay, three weights in turn: M4
+    // N12288 K4096 6.2 us against 7.6 for the split-K tiles, M8 8.2 against
+    // 7.1, M8 N5120 K17408 14.5 against 10.9; M8 N4096 K12288 7.9 against 8.7).
+    // Up to two rounds of 64 x 64 tiles, or three at K >= 8192: the split-K
+    // tiles (M400 N4096 K4096 14.2 us against 18.9 for 128 x 128 tiles, M620
+    // 20.1 against 19.0, M800 25.5 against 19.6; M128 N12288 K4096 14.9
+    // against 18.7, M256 21.9 against 19.8; three rounds at M400 N5120 K17408
+    // 52.4 against 58.7, four at M620 69.7 against 60.0).
     const int64_t tiles256 = (m + 255) / 256 * (n / 256);
-    const int64_t tiles128 = (m + 127) / 128 * (n / 128);
-    if (m <= 8)
+    const int64_t tiles64 = (m + 63) / 64 * (n / 64);
+    if (m <= 4 || (m <= 8 && n / 32 < 160))
       config = kGemmDecode;
-    else if (tiles128 < 256)
+    else if (tiles64 <= 512 || (tiles64 <= 768 && k >= 8192))
       config = kGemmKsplit;
     else
       config = (n % 256 == 0 && m >= 1024 && tiles256 >= 192) ? kGemmPersist256 : kGemmTile128;

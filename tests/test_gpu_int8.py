@@ -11,6 +11,7 @@ import oracle
 pytestmark = pytest.mark.gpu
 
 BF = oracle.f32_to_bf16
+F = oracle.bf16_to_f32
 
 
 def dev_bf16(a: np.ndarray) -> torch.Tensor:
@@ -53,6 +54,40 @@ def test_i8_gemm_residual_matches_oracle(m):
     res = BF(rng.standard_normal((m, n)).astype(np.float32))
     got, want = run(x, w, res)
     assert np.array_equal(got, want)
+
+
+# every INT8 kernel at its edges: dot products (m <= 4), split-K tiles of
+# 32 x 32, 32 x 64 and 64 x 64 (fewer k-steps than waves, uneven, two rounds),
+# the 128 x 128 ring (fewer k-steps than stages, as many, more, ragged rows),
+# 128 x 128 and 256 x 256 two-stage tiles
+@pytest.mark.parametrize("m,n,k,resid", [
+    (4, 256, 256, True), (5, 256, 256, False), (33, 1024, 1280, True), (64, 2048, 768, False),
+    (100, 4096, 512, True), (20, 12288, 512, False), (250, 4096, 2304, False), (130, 7168, 768, True),
+    (300, 8192, 256, False), (300, 8192, 512, True), (257, 8192, 768, False), (385, 6144, 1280, True),
+    (1000, 3072, 512, False), (1030, 4352, 512, True), (2100, 5120, 512, False)])
+def test_i8_gemm_every_path(m, n, k, resid):
+    """Sampled rows (block edges, a NaN row, an infinite value, the last row)
+    against the oracle; two launches agree on every row."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn((m, k), generator=g, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn((n, k), generator=g, device="cuda", dtype=torch.bfloat16) * 0.02
+    w[64:80] *= 1e-4
+    w[96:98] = 0.0
+    if m > 40:
+        x[m - 5] = float("nan")
+        x[37, 3] = float("inf")
+    res = torch.randn((m, n), generator=g, device="cuda", dtype=torch.bfloat16) if resid else None
+    q = clef_i4.load_quantized_weight(w, bits=8)
+    a = clef_i4.prepare(x, bits=8)
+    got = host_u16(clef_i4.project_prepared(a, q, residual=res))
+    assert np.array_equal(got, host_u16(clef_i4.project_prepared(a, q, residual=res)))
+    rows = sorted({0, 1 % m, m // 3, m - 1, min(37, m - 1), max(m - 5, 0), min(127, m - 1), min(128, m - 1),
+                   min(255, m - 1), min(256, m - 1), m // 128 * 128 if m % 128 else m - 1})
+    codes, scales, _ = oracle.prepare(host_u16(x[rows]), oracle.activation_stride(k, 8), 8)
+    want = oracle.gemm(codes, scales, q.codes.cpu().numpy().view(np.uint32), q.scales.cpu().numpy(), n, k, bits=8,
+                       residual=host_u16(res)[rows] if resid else None)
+    nan = np.isnan(F(want))
+    assert np.array_equal(nan, np.isnan(F(got[rows]))) and np.array_equal(got[rows][~nan], want[~nan])
 
 
 def test_i8_gemm_extreme_codes_and_nonfinite_rows():
