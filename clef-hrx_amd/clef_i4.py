@@ -37,6 +37,7 @@ SIGNATURES = {
     "clef_i4_prepare_attention_gate": (ctypes.c_int, [_P, _P, _I64, _I32, _I32, _I32, _P, _P]),
     "clef_i4_prepare_norm_words": (_I64, [_I64, _I32, _I32, _I32, _I32]),
     "clef_i4_prepare_norm": (ctypes.c_int, [_P, _P, _I64, _I32, _I32, _I32, _I32, _P, _P]),
+    "clef_i4_prepare_filled": (ctypes.c_int, [_P, _P, _I32, _I64, _I32, _I32, _I32, _P, _P]),
     "clef_i4_retile": (ctypes.c_int, [_P, _I64, _I32, _I32, _I32, _P, _P]),
     "clef_i4_pack_weight_workspace_bytes": (_SZ, [_I64, _I32, _I32]),
     "clef_i4_pack_weight": (ctypes.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _SZ, _P]),
@@ -165,14 +166,23 @@ class Prepared:
         return self.storage[start: start + self.rows].view(torch.float32)
 
 
+def _prepare_filled(producer: int, x, second, rows: int, width: int, stride: int, bits: int) -> Prepared:
+    """A new Prepared of one of the library's producers (CLEF_PRODUCER_*); the
+    kernel writes every word of it, padding as zeros."""
+    words = int(lib().clef_i4_prepared_words(rows, stride, bits))
+    out = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
+    _check(lib().clef_i4_prepare_filled(_ptr(x), _ptr(second), producer, rows, width, stride, bits, _ptr(out),
+                                        _stream()))
+    return Prepared(out, rows, width, stride, bits)
+
+
 def prepare(x: torch.Tensor, bits: int = 4, stride: int | None = None, out: torch.Tensor | None = None
             ) -> Prepared:
     """quantized::prepare (src/quantized.rs:574-686)."""
     rows, width = x.shape
     stride = activation_stride(width, bits) if stride is None else stride
-    words = int(lib().clef_i4_prepared_words(rows, stride, bits))
     if out is None:
-        out = torch.zeros(max(words, 1), dtype=torch.int32, device=x.device)
+        return _prepare_filled(0, x, None, rows, width, stride, bits)
     _check(lib().clef_i4_prepare(_ptr(x), rows, width, stride, bits, _ptr(out), _stream()))
     return Prepared(out, rows, width, stride, bits)
 
@@ -182,11 +192,7 @@ def prepare_swiglu(gate: torch.Tensor, up: torch.Tensor, bits: int = 4, stride: 
     """prepare_with_inputs([gate, up]) (src/quantized.rs:605-613)."""
     rows, width = gate.shape
     stride = activation_stride(width, bits) if stride is None else stride
-    words = int(lib().clef_i4_prepared_words(rows, stride, bits))
-    out = torch.zeros(max(words, 1), dtype=torch.int32, device=gate.device)
-    _check(lib().clef_i4_prepare_swiglu(_ptr(gate), _ptr(up), rows, width, stride, bits, _ptr(out),
-                                        _stream()))
-    return Prepared(out, rows, width, stride, bits)
+    return _prepare_filled(1, gate, up, rows, width, stride, bits)
 
 
 def prepare_attention_gate(attention: torch.Tensor, q_gate: torch.Tensor, bits: int = 4,
@@ -197,11 +203,7 @@ def prepare_attention_gate(attention: torch.Tensor, q_gate: torch.Tensor, bits: 
     if tuple(q_gate.shape) != (rows, 2 * width) or q_gate.dtype != attention.dtype:
         raise ClefError(-1, "packing input shape/dtype mismatch")
     stride = activation_stride(width, bits) if stride is None else stride
-    words = int(lib().clef_i4_prepared_words(rows, stride, bits))
-    out = torch.zeros(max(words, 1), dtype=torch.int32, device=attention.device)
-    _check(lib().clef_i4_prepare_attention_gate(_ptr(attention), _ptr(q_gate), rows, width, stride, bits,
-                                                _ptr(out), _stream()))
-    return Prepared(out, rows, width, stride, bits)
+    return _prepare_filled(2, attention, q_gate, rows, width, stride, bits)
 
 
 def prepare_norm(x: torch.Tensor, weight: torch.Tensor, bits: int = 4, stride: int | None = None,
@@ -213,14 +215,14 @@ def prepare_norm(x: torch.Tensor, weight: torch.Tensor, bits: int = 4, stride: i
     if weight.numel() != width:
         raise ClefError(-1, "unsupported normalized packing shape")
     stride = activation_stride(width, bits) if stride is None else stride
+    if not store:
+        return _prepare_filled(3, x, weight.contiguous(), rows, width, stride, bits), None
     total = int(lib().clef_i4_prepare_norm_words(rows, width, stride, bits, int(store)))
     out = torch.zeros(max(total, 1), dtype=torch.int32, device=x.device)
     _check(lib().clef_i4_prepare_norm(_ptr(x), _ptr(weight.contiguous()), rows, width, stride, bits, int(store),
                                       _ptr(out), _stream()))
-    normalized = None
-    if store:
-        first = total - rows * width // 2
-        normalized = out[first:].view(torch.bfloat16).view(rows, width)
+    first = total - rows * width // 2
+    normalized = out[first:].view(torch.bfloat16).view(rows, width)
     return Prepared(out, rows, width, stride, bits), normalized
 
 

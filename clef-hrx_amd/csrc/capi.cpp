@@ -65,6 +65,13 @@ int check_prepare(int64_t rows, int32_t width, int32_t stride, int32_t bits) {
   return CLEF_OK;
 }
 
+int check_norm(int64_t rows, int32_t width, int32_t stride, int32_t bits) {
+  if (!(width == 5120 && (bits == 4 || bits == 8) && rows >= 1 && rows <= 1048576 && stride >= width &&
+        stride <= 65536 && stride % (512 / bits) == 0))
+    return fail("unsupported normalized packing shape");
+  return CLEF_OK;
+}
+
 int check_gemm(int64_t m, int32_t n, int32_t k, int32_t k_stride) {
   if (!(m >= 1 && n >= 128 && n % 128 == 0 && k >= 256 && k % 256 == 0 && k_stride >= k &&
         k_stride % 32 == 0))
@@ -146,15 +153,42 @@ int64_t clef_i4_prepare_norm_words(int64_t rows, int32_t width, int32_t stride, 
 int clef_i4_prepare_norm(const uint16_t* x, const uint16_t* weight, int64_t rows, int32_t width,
                          int32_t stride, int32_t bits, int32_t store, uint32_t* out,
                          clef_stream_t stream) {
-  if (!(width == 5120 && (bits == 4 || bits == 8) && rows >= 1 && rows <= 1048576 && stride >= width &&
-        stride <= 65536 && stride % (512 / bits) == 0))
-    return fail("unsupported normalized packing shape");
+  if (int rc = check_norm(rows, width, stride, bits)) return rc;
   if (!aligned(x, 16) || !aligned(weight, 16) || !aligned(out, 16)) return fail(kAlign);
   uint16_t* normalized =
       store ? reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(out) + norm_offset_bytes(rows, stride, bits))
             : nullptr;
   return hip_status(
       clef::launch_prepare_norm(x, weight, rows, width, stride, bits, out, normalized, hs(stream)));
+}
+
+int clef_i4_prepare_filled(const uint16_t* x, const uint16_t* second, int32_t producer, int64_t rows, int32_t width,
+                           int32_t stride, int32_t bits, uint32_t* out, clef_stream_t stream) {
+  if (producer == CLEF_PRODUCER_NORM) {
+    if (int rc = check_norm(rows, width, stride, bits)) return rc;
+  } else if (producer == CLEF_PRODUCER_PLAIN || producer == CLEF_PRODUCER_SWIGLU ||
+             producer == CLEF_PRODUCER_ATTENTION_GATE) {
+    if (int rc = check_prepare(rows, width, stride, bits)) return rc;
+  } else {
+    return fail("unknown packing producer");
+  }
+  if (!aligned(x, 16) || (producer != CLEF_PRODUCER_PLAIN && !aligned(second, 16)) || !aligned(out, 16))
+    return fail(kAlign);
+  hipError_t e;
+  switch (producer) {
+    case CLEF_PRODUCER_SWIGLU:
+      e = clef::launch_prepare_swiglu(x, second, rows, width, stride, bits, out, hs(stream), true);
+      break;
+    case CLEF_PRODUCER_ATTENTION_GATE:
+      e = clef::launch_prepare_attention_gate(x, second, rows, width, stride, bits, out, hs(stream), true);
+      break;
+    case CLEF_PRODUCER_NORM:
+      e = clef::launch_prepare_norm(x, second, rows, width, stride, bits, out, nullptr, hs(stream), true);
+      break;
+    default:
+      e = clef::launch_prepare(x, rows, width, stride, bits, out, hs(stream), true);
+  }
+  return hip_status(e);
 }
 
 int clef_i4_retile(const uint32_t* codes, int64_t rows, int32_t in_words, int32_t cols, int32_t bits,

@@ -21,8 +21,9 @@ constexpr int64_t f6_offset(int64_t row, int64_t col, int64_t width) {
   return ((row >> 7) * (width >> 7) + (col >> 7)) * 12288 + (row & 127) * 96 + (col & 127) * 3 / 4;
 }
 
+// fill: write the padding words behind each row as zeros.
 hipError_t launch_prepare(const uint16_t* x, int64_t rows, int width, int stride, int bits,
-                          uint32_t* out, hipStream_t stream);
+                          uint32_t* out, hipStream_t stream, bool fill = false);
 // The router and the INT4 quantizer of `x` ([tokens][width], stride as
 // launch_prepare) in one launch; only for widths the grid-stride quantizer
 // takes (route_prepare_fusable).
@@ -37,11 +38,11 @@ hipError_t launch_route_prepare(const void* logits, int dtype, int64_t tokens, i
                                 hipStream_t stream, float* groups = nullptr, float* order = nullptr,
                                 int32_t* schedule = nullptr, int bm = 0, int* counts16 = nullptr);
 hipError_t launch_prepare_swiglu(const uint16_t* gate, const uint16_t* up, int64_t rows, int width,
-                                 int stride, int bits, uint32_t* out, hipStream_t stream);
+                                 int stride, int bits, uint32_t* out, hipStream_t stream, bool fill = false);
 hipError_t launch_prepare_attention_gate(const uint16_t* x, const uint16_t* q_gate, int64_t rows, int width,
-                                         int stride, int bits, uint32_t* out, hipStream_t stream);
+                                         int stride, int bits, uint32_t* out, hipStream_t stream, bool fill = false);
 hipError_t launch_prepare_norm(const uint16_t* x, const uint16_t* weight, int64_t rows, int width, int stride,
-                               int bits, uint32_t* out, uint16_t* normalized, hipStream_t stream);
+                               int bits, uint32_t* out, uint16_t* normalized, hipStream_t stream, bool fill = false);
 // Q1 of a weight (rows of a checkpoint-tiled matrix when checkpoint_tiled)
 // with the codes stored in the tiled layout, scales [rows].
 hipError_t launch_pack_weight(const uint16_t* w, int64_t rows, int cols, int bits, bool checkpoint_tiled,

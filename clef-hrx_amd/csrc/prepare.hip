@@ -297,10 +297,17 @@ __device__ __forceinline__ float* scales_of(uint32_t* out, int64_t rows, int wid
   return reinterpret_cast<float*>(out + rows * out_words);
 }
 
+// Zeros the `pad` words behind a row's codes (words lane, lane + lanes, ..).
+template <int BITS>
+__device__ __forceinline__ void zero_padding(uint32_t* out_row, int width, int pad, int lane, int lanes) {
+  for (int i = lane; i < pad; i += lanes) out_row[width / (32 / BITS) + i] = 0u;
+}
+
 // TILED: codes in the weight layout (store_group), row scales to `wscales`.
+// pad: padding words per row to write as zeros.
 template <int P, int BITS, class Src, bool TILED>
 __global__ __launch_bounds__(256) void prepare_kernel(Src src, int64_t rows, int width,
-                                                      int out_words, uint32_t* __restrict__ out,
+                                                      int out_words, int pad, uint32_t* __restrict__ out,
                                                       float* __restrict__ wscales) {
   __shared__ __align__(16) float lds[16 * kGroupLds];
   __shared__ uint32_t gmax[16];
@@ -431,6 +438,8 @@ __global__ __launch_bounds__(256) void prepare_kernel(Src src, int64_t rows, int
     group_lds_order();
     if (on) store_group<BITS, TILED>(out, out + row * out_words, row, grp * 256 + 16 * L, width, nat, inv, valid);
   }
+  if constexpr (BITS != 6 && !TILED)
+    if (pad > 0 && active) zero_padding<BITS>(out + row * out_words, width, pad, 16 * grp0 + L, P == 1 ? 16 * G : 256);
   if (active && grp0 == 0 && L == 0) (TILED ? wscales : scales_of<BITS>(out, rows, width, out_words))[row] = scale;
 }
 
@@ -440,7 +449,7 @@ __global__ __launch_bounds__(256) void prepare_kernel(Src src, int64_t rows, int
 // overlaps the work instead of being paid once per workgroup.
 // The body runs as workgroup `block` of `nblocks` walking the row blocks.
 template <int BITS, class Src, bool TILED>
-__device__ __forceinline__ void prepare_loop_body(Src src, int64_t rows, int width, int out_words,
+__device__ __forceinline__ void prepare_loop_body(Src src, int64_t rows, int width, int out_words, int pad,
                                                   uint32_t* __restrict__ out, float* __restrict__ wscales,
                                                   int64_t block, int64_t nblocks) {
   // 20 KiB: eight workgroups fill a CU's LDS. Each group's maximum goes to
@@ -541,15 +550,17 @@ __device__ __forceinline__ void prepare_loop_body(Src src, int64_t rows, int wid
     group_lds_order();
     if (on) {
       store_group<BITS, TILED>(out, out + out_off, row, col, width, nat, inv, valid);
+      if constexpr (BITS != 6 && !TILED)
+        if (pad > 0) zero_padding<BITS>(out + out_off, width, pad, 16 * grp + L, 16 * G);
       if (grp == 0 && L == 0) (TILED ? wscales : scales_of<BITS>(out, rows, width, out_words))[row] = scale;
     }
   }
 }
 
 template <int BITS, class Src, bool TILED>
-__global__ __launch_bounds__(256) void prepare_loop_kernel(Src src, int64_t rows, int width, int out_words,
+__global__ __launch_bounds__(256) void prepare_loop_kernel(Src src, int64_t rows, int width, int out_words, int pad,
                                                            uint32_t* __restrict__ out, float* __restrict__ wscales) {
-  prepare_loop_body<BITS, Src, TILED>(src, rows, width, out_words, out, wscales, blockIdx.x, gridDim.x);
+  prepare_loop_body<BITS, Src, TILED>(src, rows, width, out_words, pad, out, wscales, blockIdx.x, gridDim.x);
 }
 
 // The router and the INT4 quantizer of the MoE input in one launch: the first
@@ -595,12 +606,12 @@ __global__ __launch_bounds__(256) void route_prepare_kernel(const void* __restri
     route_impl::route_block(logits, dtype, tokens, experts, topk, routes, blockIdx.x);
     return;
   }
-  prepare_loop_body<4, PlainSource, false>(src, tokens, width, out_words, out, nullptr, blockIdx.x - route_blocks,
+  prepare_loop_body<4, PlainSource, false>(src, tokens, width, out_words, 0, out, nullptr, blockIdx.x - route_blocks,
                                            gridDim.x - route_blocks);
 }
 
 template <int BITS, bool TILED = false, class Src>
-hipError_t launch_prepare_bits(const Src& src, int64_t rows, int width, int out_words,
+hipError_t launch_prepare_bits(const Src& src, int64_t rows, int width, int out_words, int pad,
                                uint32_t* out, hipStream_t stream, float* wscales = nullptr) {
   const int G = width / 256;
   if (G <= 16 && !Src::kRowNorm) {
@@ -610,13 +621,13 @@ hipError_t launch_prepare_bits(const Src& src, int64_t rows, int width, int out_
     // that are walked by the grid stride.
     const unsigned grid = (unsigned)(blocks < 2048 ? blocks : 2048);
     if constexpr (!Src::kRowNorm)
-      prepare_loop_kernel<BITS, Src, TILED><<<grid, 256, 0, stream>>>(src, rows, width, out_words, out, wscales);
+      prepare_loop_kernel<BITS, Src, TILED><<<grid, 256, 0, stream>>>(src, rows, width, out_words, pad, out, wscales);
   } else {
     const int passes = (G + 15) / 16;
     const unsigned grid = (unsigned)rows;
     switch (passes) {
 #define CLEF_PREP_CASE(N) \
-  case N: prepare_kernel<N, BITS, Src, TILED><<<grid, 256, 0, stream>>>(src, rows, width, out_words, out, wscales); break;
+  case N: prepare_kernel<N, BITS, Src, TILED><<<grid, 256, 0, stream>>>(src, rows, width, out_words, pad, out, wscales); break;
       CLEF_PREP_CASE(2)
       CLEF_PREP_CASE(3)
       CLEF_PREP_CASE(4)
@@ -631,15 +642,17 @@ hipError_t launch_prepare_bits(const Src& src, int64_t rows, int width, int out_
   return hipGetLastError();
 }
 
-// bits 4 or 8: packed codes of `stride` columns per row; bits 6: the tiled
-// bf6 activation layout (f6_offset; stride == width).
+// bits 4 or 8: packed codes of `stride` columns per row, the padding behind
+// `width` zeroed when `fill`; bits 6: the tiled bf6 activation layout
+// (f6_offset; stride == width).
 template <class Src>
-hipError_t launch_prepare_src(const Src& src, int64_t rows, int width, int stride, int bits,
+hipError_t launch_prepare_src(const Src& src, int64_t rows, int width, int stride, int bits, bool fill,
                               uint32_t* out, hipStream_t stream) {
-  if (bits == 6) return launch_prepare_bits<6>(src, rows, width, width * 3 / 16, out, stream);
+  if (bits == 6) return launch_prepare_bits<6>(src, rows, width, width * 3 / 16, 0, out, stream);
   const int out_words = stride / (32 / bits);
-  if (bits == 4) return launch_prepare_bits<4>(src, rows, width, out_words, out, stream);
-  return launch_prepare_bits<8>(src, rows, width, out_words, out, stream);
+  const int pad = fill ? out_words - width / (32 / bits) : 0;
+  if (bits == 4) return launch_prepare_bits<4>(src, rows, width, out_words, pad, out, stream);
+  return launch_prepare_bits<8>(src, rows, width, out_words, pad, out, stream);
 }
 
 // Q2 retile: word (n, q) of the row-major codes lands at
@@ -695,8 +708,8 @@ __global__ __launch_bounds__(256) void tile_permute_kernel(const uint16_t* __res
 }  // namespace
 
 hipError_t launch_prepare(const uint16_t* x, int64_t rows, int width, int stride, int bits,
-                          uint32_t* out, hipStream_t stream) {
-  return launch_prepare_src(PlainSource{x}, rows, width, stride, bits, out, stream);
+                          uint32_t* out, hipStream_t stream, bool fill) {
+  return launch_prepare_src(PlainSource{x}, rows, width, stride, bits, fill, out, stream);
 }
 
 // Weight packing: Q1 with the codes stored in the tiled layout, one pass over
@@ -707,12 +720,12 @@ hipError_t launch_pack_weight(const uint16_t* w, int64_t rows, int cols, int bit
                               uint32_t* tiled, float* scales, hipStream_t stream) {
   if (checkpoint_tiled) {
     const CheckpointSource src{w, cols};
-    return bits == 4 ? launch_prepare_bits<4, true>(src, rows, cols, 0, tiled, stream, scales)
-                     : launch_prepare_bits<8, true>(src, rows, cols, 0, tiled, stream, scales);
+    return bits == 4 ? launch_prepare_bits<4, true>(src, rows, cols, 0, 0, tiled, stream, scales)
+                     : launch_prepare_bits<8, true>(src, rows, cols, 0, 0, tiled, stream, scales);
   }
   const PlainSource src{w};
-  return bits == 4 ? launch_prepare_bits<4, true>(src, rows, cols, 0, tiled, stream, scales)
-                   : launch_prepare_bits<8, true>(src, rows, cols, 0, tiled, stream, scales);
+  return bits == 4 ? launch_prepare_bits<4, true>(src, rows, cols, 0, 0, tiled, stream, scales)
+                   : launch_prepare_bits<8, true>(src, rows, cols, 0, 0, tiled, stream, scales);
 }
 
 bool route_prepare_fusable(int width) { return width % 256 == 0 && width / 256 <= 16; }
@@ -738,19 +751,19 @@ hipError_t launch_route_prepare(const void* logits, int dtype, int64_t tokens, i
 }
 
 hipError_t launch_prepare_swiglu(const uint16_t* gate, const uint16_t* up, int64_t rows, int width,
-                                 int stride, int bits, uint32_t* out, hipStream_t stream) {
-  return launch_prepare_src(SwigluSource{gate, up}, rows, width, stride, bits, out, stream);
+                                 int stride, int bits, uint32_t* out, hipStream_t stream, bool fill) {
+  return launch_prepare_src(SwigluSource{gate, up}, rows, width, stride, bits, fill, out, stream);
 }
 
 hipError_t launch_prepare_attention_gate(const uint16_t* x, const uint16_t* q_gate, int64_t rows, int width,
-                                         int stride, int bits, uint32_t* out, hipStream_t stream) {
-  return launch_prepare_src(AttentionGateSource{x, q_gate}, rows, width, stride, bits, out, stream);
+                                         int stride, int bits, uint32_t* out, hipStream_t stream, bool fill) {
+  return launch_prepare_src(AttentionGateSource{x, q_gate}, rows, width, stride, bits, fill, out, stream);
 }
 
 hipError_t launch_prepare_norm(const uint16_t* x, const uint16_t* weight, int64_t rows, int width, int stride,
-                               int bits, uint32_t* out, uint16_t* normalized, hipStream_t stream) {
+                               int bits, uint32_t* out, uint16_t* normalized, hipStream_t stream, bool fill) {
   if (width / 256 <= 16) return hipErrorInvalidValue;
-  return launch_prepare_src(NormSource{x, weight, normalized}, rows, width, stride, bits, out, stream);
+  return launch_prepare_src(NormSource{x, weight, normalized}, rows, width, stride, bits, fill, out, stream);
 }
 
 hipError_t launch_retile(const uint32_t* codes, int64_t rows, int in_words, int words,

@@ -124,6 +124,18 @@ int clef_i4_prepare_norm(const uint16_t* x, const uint16_t* weight, int64_t rows
                          int32_t stride, int32_t bits, int32_t store, uint32_t* out,
                          clef_stream_t stream);
 
+/* clef_i4_prepare, _swiglu (x = gate, second = up), _attention_gate (second =
+ * q_gate) or _norm without stored rows (second = weight), which also writes
+ * the padding words of each row as zeros, so `out` needs no clearing. */
+enum {
+  CLEF_PRODUCER_PLAIN = 0,
+  CLEF_PRODUCER_SWIGLU = 1,
+  CLEF_PRODUCER_ATTENTION_GATE = 2,
+  CLEF_PRODUCER_NORM = 3
+};
+int clef_i4_prepare_filled(const uint16_t* x, const uint16_t* second, int32_t producer, int64_t rows, int32_t width,
+                           int32_t stride, int32_t bits, uint32_t* out, clef_stream_t stream);
+
 /* Row-major packed codes [rows][in_words] -> tiled blocks, dropping padding.
  * Replaces quantized::retile_codes (src/quantized.rs:542-572) and
  * kernels/retile_codes.loom. Preconditions: rows % 128 == 0, words =

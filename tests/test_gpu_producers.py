@@ -124,3 +124,38 @@ def test_router_logits_integer_inputs_are_exact(tokens, hidden, experts):
     w = rng.integers(-3, 4, (experts, hidden)).astype(np.float32)
     got = host_u16(clef_i4.router_logits(dev_bf16(BF(x)), dev_bf16(BF(w))))
     assert np.array_equal(got, BF(x @ w.T))
+
+
+@pytest.mark.parametrize("producer,width,bits,extra", [
+    (0, 256, 4, 0), (0, 1024, 4, 0), (0, 768, 8, 128), (0, 4096, 8, 0), (0, 5120, 4, 1024), (0, 12288, 8, 0),
+    (1, 2048, 4, 256), (1, 17408, 4, 0), (1, 6144, 8, 0), (2, 1024, 8, 0), (2, 5120, 4, 0), (3, 5120, 4, 0),
+    (3, 5120, 8, 0)])
+def test_prepare_filled_writes_every_word(producer, width, bits, extra):
+    """clef_i4_prepare_filled on a buffer of ones bits: padding words zero,
+    codes and scales those of the entry it stands for; that entry itself
+    leaves the padding words as they were."""
+    rows = 19
+    rng = np.random.default_rng(width + bits + producer)
+    stride = clef_i4.activation_stride(width, bits) + extra
+    words, used = stride * bits // 32, width * bits // 32
+    x = dev_bf16(BF(rng.standard_normal((rows, width)).astype(np.float32)))
+    second = None if producer == 0 else dev_bf16(BF(rng.standard_normal(
+        {1: (rows, width), 2: (rows, 2 * width), 3: (width,)}[producer]).astype(np.float32)))
+    stream = torch.cuda.current_stream().cuda_stream
+    lib = clef_i4.lib()
+    filled, plain = (torch.full((rows * (words + 1),), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    p2 = None if second is None else second.data_ptr()
+    assert lib.clef_i4_prepare_filled(x.data_ptr(), p2, producer, rows, width, stride, bits, filled.data_ptr(),
+                                      stream) == 0
+    args = (rows, width, stride, bits)
+    if producer == 0:
+        rc = lib.clef_i4_prepare(x.data_ptr(), *args, plain.data_ptr(), stream)
+    elif producer == 3:
+        rc = lib.clef_i4_prepare_norm(x.data_ptr(), p2, *args, 0, plain.data_ptr(), stream)
+    else:
+        fn = lib.clef_i4_prepare_swiglu if producer == 1 else lib.clef_i4_prepare_attention_gate
+        rc = fn(x.data_ptr(), p2, *args, plain.data_ptr(), stream)
+    assert rc == 0
+    f, p = filled[: rows * words].view(rows, words), plain[: rows * words].view(rows, words)
+    assert torch.equal(f[:, :used], p[:, :used]) and torch.equal(filled[rows * words:], plain[rows * words:])
+    assert not f[:, used:].any() and bool((p[:, used:] == -1).all())
