@@ -15,6 +15,7 @@
 #include "gemm_dma.hpp"
 #include "gemm_dmah.hpp"
 #include "expert_persist.hpp"
+#include "expert_stream.hpp"
 #include "group.hpp"
 #include "kernels.hpp"
 #include "launch.hpp"
@@ -2138,11 +2139,15 @@ hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const
 }
 
 // Routed rows up to which the grouped expert GEMMs use 32-slot tiles and
-// expert_skinny_kernel (on average 16 rows per expert at 128 experts).
-constexpr int64_t kExpertSkinnyRoutes = 2048;
-constexpr int kExpertSkinnyBM = 32;
+// expert_stream_kernel (on average 32 rows per expert at 128 experts). Omni
+// MoE layer by graph replay (hidden 2048, expert width 768, top-8) against the
+// persistent 128-slot kernel: 300 tokens 86.8 against 110.8 us, 500: 109.8 /
+// 113.9, 620: 124.4 / 116.9; skewed routing 500: 106.7 / 122.0, 620: 117.1 /
+// 127.3.
+constexpr int64_t kExpertSmallRoutes = 4096;
+constexpr int kExpertSmallBM = 32;
 
-int expert_tile_rows(int64_t routes) { return routes <= kExpertSkinnyRoutes ? kExpertSkinnyBM : kExpertBM; }
+int expert_tile_rows(int64_t routes) { return routes <= kExpertSmallRoutes ? kExpertSmallBM : kExpertBM; }
 
 // Tiles of the schedule: sum over experts of ceil(count / bm) <= routes / bm
 // rounded up, plus one per expert with any route.
@@ -2152,11 +2157,12 @@ int64_t expert_max_tiles(int64_t routes) {
 }
 
 // Routed rows up to which the grouped expert GEMMs run expert_decode_kernel
-// on the 32-slot tiles: 32 tokens at top-8. Omni MoE layer by graph replay,
-// weights in the last-level cache, against expert_skinny_kernel: 1 token
-// 17.4 against 21.5 us, 2: 22.3 / 26.3, 4: 29.1 / 34.0, 8: 38.2 / 44.7, 16:
-// 52.4 / 60.1, 32: 70.8 / 77.0; equal at 48 tokens, 96.4 against 85.5 at 64.
-constexpr int64_t kExpertDecodeRoutes = 256;
+// on the 32-slot tiles: 24 tokens at top-8. Omni MoE layer by graph replay
+// against expert_stream_kernel: 16 tokens 57.3 against 56.8 us, 20: 67.0 /
+// 69.9, 24: 70.6 / 72.1, 32: 79.0 / 75.0 with evenly spread routes; with
+// skewed ones (experts of several rows, a pass each two) 24: 75.3 / 56.5, 32:
+// 86.3 / 60.1.
+constexpr int64_t kExpertDecodeRoutes = 192;
 
 namespace {
 template <bool GU, int NW, int RW, int MR>
@@ -2211,6 +2217,51 @@ hipError_t launch_expert_down_h_t(const uint16_t* h, const uint32_t* w, const fl
   return hipGetLastError();
 }
 
+template <bool GU, int NB, bool ONE>
+hipError_t launch_expert_stream_t(const uint32_t* a, int a_words, int64_t a_bytes, const float* as, const uint32_t* w,
+                                  const float* ws, const uint32_t* w2, const float* ws2, const float* groups,
+                                  const int32_t* schedule, int64_t routes, int64_t list_stride, int topk, int k, int n,
+                                  int input_routed, uint16_t* out, int spw, hipStream_t stream) {
+  const int lds = expert_stream_lds<GU, NB, ONE>(k / 256, spw);
+  static LaunchCache cache;
+  const void* kern = reinterpret_cast<const void*>(&expert_stream_kernel<GU, NB, ONE>);
+  if (hipError_t e = ensure_dynamic_lds(cache, kern, 160 * 1024)) return e;
+  const int colgroups = n / (128 * spw);
+  expert_stream_kernel<GU, NB, ONE>
+      <<<(unsigned)(expert_max_tiles(routes) * colgroups), 64 * kStreamWaves, lds, stream>>>(
+          a, a_words, (uint32_t)a_bytes, as, w, ws, w2, ws2, groups, schedule, list_stride, topk, k / 256, n,
+          input_routed, out, (uint32_t)(routes * n * 2), colgroups, spw);
+  return hipGetLastError();
+}
+
+// Most k-steps whose activation rows fit the LDS beside the rings.
+constexpr int kStreamMaxSteps = 26;
+
+// SPW, the 32-column slices per wave: up to 16 ring steps per wave (a
+// workgroup's start, three dependent loads, is paid once per about 200 KiB of
+// weights), as long as two workgroups per CU have work. Kernel time at 235
+// tokens (hidden 2048, expert width 768), against expert_skinny_kernel:
+// gate/up 50.6 -> 41.9 us (201 MB, 4.8 TB/s), down 30.0 -> 24.4 us (29.7 with
+// one slice per wave). With two or four stages per wave gate/up takes 45.6 and
+// 48.8 us (two: too little in flight; four: one workgroup per CU).
+template <bool GU>
+hipError_t launch_expert_stream(const uint32_t* a, int a_words, int64_t a_bytes, const float* as, const uint32_t* w,
+                                const float* ws, const uint32_t* w2, const float* ws2, const float* groups,
+                                const int32_t* schedule, int64_t routes, int64_t list_stride, int topk, int k, int n,
+                                int input_routed, uint16_t* out, hipStream_t stream) {
+  const int kb = k / 256;
+  int spw = 1;
+  while (spw < 4 && n % (256 * spw) == 0 && 2 * spw * kb * (GU ? 2 : 1) <= 16 &&
+         expert_max_tiles(routes) * (n / (256 * spw)) >= 512)
+    spw *= 2;
+#define CLEF_STREAM(ONE)                                                                                           \
+  return launch_expert_stream_t<GU, 3, ONE>(a, a_words, a_bytes, as, w, ws, w2, ws2, groups, schedule, routes,     \
+                                            list_stride, topk, k, n, input_routed, out, spw, stream)
+  if (spw == 1) CLEF_STREAM(true);
+  CLEF_STREAM(false);
+#undef CLEF_STREAM
+}
+
 template <bool GU>
 hipError_t launch_expert_skinny(const uint32_t* a, int a_words, int64_t a_bytes, const float* as,
                                 const uint32_t* w, const float* ws, const uint32_t* w2, const float* ws2,
@@ -2219,6 +2270,9 @@ hipError_t launch_expert_skinny(const uint32_t* a, int a_words, int64_t a_bytes,
   if (a_bytes >= ((int64_t)1 << 31) || n % 32 != 0) return hipErrorInvalidValue;
   if (routes <= kExpertDecodeRoutes)
     return launch_expert_decode<GU>(a, a_words, a_bytes, as, w, ws, w2, ws2, groups, schedule, routes, list_stride,
+                                    topk, k, n, input_routed, out, stream);
+  if (n % 128 == 0 && k / 256 <= kStreamMaxSteps && routes * n * 2 < ((int64_t)1 << 31))
+    return launch_expert_stream<GU>(a, a_words, a_bytes, as, w, ws, w2, ws2, groups, schedule, routes, list_stride,
                                     topk, k, n, input_routed, out, stream);
   const int slices = n / 32;
   const int64_t blocks = expert_max_tiles(routes) * slices;
@@ -2298,7 +2352,7 @@ hipError_t launch_expert_gate_up(const uint32_t* a, int a_words, const float* as
   const int64_t routes = tokens * topk;
   if (list_stride <= 0) list_stride = tokens + 1;
   if (a_bytes >= ((int64_t)1 << 31) || n % 128 != 0) return hipErrorInvalidValue;
-  if (expert_tile_rows(routes) == kExpertSkinnyBM)
+  if (expert_tile_rows(routes) == kExpertSmallBM)
     return launch_expert_skinny<true>(a, a_words, a_bytes, as, gate_w, gate_s, up_w, up_s, groups, schedule, routes,
                                       list_stride, topk, k, n, 0, h, stream);
   if (use_expert_persist<true>(k, n, routes))
@@ -2421,7 +2475,7 @@ hipError_t launch_expert_i4(const uint32_t* a, int a_words, const float* as, con
   const int64_t a_rows = input_routed ? routes : tokens;
   const int64_t a_bytes = a_rows * a_words * 4;
   if (list_stride <= 0) list_stride = tokens + 1;
-  if (expert_tile_rows(routes) == kExpertSkinnyBM)
+  if (expert_tile_rows(routes) == kExpertSmallBM)
     return launch_expert_skinny<false>(a, a_words, a_bytes, as, w, ws, w, ws, groups, schedule, routes, list_stride,
                                        topk, k, n, input_routed, out, stream);
   // The callers reject activation operands of 2 GiB or more and n % 256 != 0.

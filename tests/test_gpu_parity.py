@@ -734,6 +734,50 @@ def test_expert_gate_up_persistent_matches_oracle(tokens, k, n, skew):
     assert torch.equal(again.view(torch.int16), got.view(torch.int16))
 
 
+# (tokens, k, n, topk, skew): expert_stream_kernel at its edges: one, two,
+# three, eight and the most k-steps its LDS takes (and one more: the kernel
+# for wider rows), one, two and four slices per wave, tiles with one slot and
+# full ones, experts of several tiles, both ends of its range of routed rows
+# and one token count past it.
+STREAM_CASES = [(25, 256, 256, 8, 0.0), (40, 512, 768, 8, 2.0), (300, 512, 2048, 8, 0.0), (300, 256, 1024, 8, 3.0),
+                (512, 768, 512, 8, 1.0), (513, 768, 512, 8, 1.0), (100, 2048, 256, 4, 2.0), (60, 2304, 256, 8, 0.0),
+                (30, 6656, 256, 8, 1.0), (30, 6912, 256, 8, 1.0), (260, 1024, 768, 6, 4.0)]
+
+
+def _stream_operands(tokens, k, n, topk, skew, weights, rows):
+    g = torch.Generator(device="cuda").manual_seed(tokens + k + n)
+    rng = np.random.default_rng(tokens + k + n)
+    routes = random_routes(rng, tokens, topk=topk, skew=skew)
+    groups, _ = oracle.group_routes(routes, topk=topk)
+    x = torch.randn((rows, k), generator=g, device="cuda", dtype=torch.bfloat16)
+    x[rows // 2] = float("nan")
+    x[rows - 1, 3] = 0.0
+    qs = [clef_i4.load_quantized_weight(torch.randn((128 * n, k), generator=g, device="cuda", dtype=torch.bfloat16)
+                                        * 0.02) for _ in range(weights)]
+    codes, scales, _ = oracle.prepare(bf16_host(x), oracle.activation_stride(k))
+    return groups, clef_i4.prepare(x), qs, codes, scales, [(u32_host(q.codes), q.scales.cpu().numpy()) for q in qs]
+
+
+@pytest.mark.parametrize("tokens,k,n,topk,skew", STREAM_CASES)
+@pytest.mark.parametrize("routed", [False, True])
+def test_expert_stream_matches_oracle(tokens, k, n, topk, skew, routed):
+    groups, a, (q,), codes, scales, host = _stream_operands(tokens, k, n, topk, skew, 1,
+                                                            tokens * topk if routed else tokens)
+    want = oracle.expert_i4(codes, scales, *host[0], groups, tokens, topk, k, n, routed)
+    for _ in range(2):
+        got = clef_i4.omni_expert(a, q, to_dev_f32(groups), tokens, topk, routed)
+        assert_same_bf16_nan_aware(bf16_host(got), want, f"expert stream t={tokens} k={k} n={n} routed={routed}")
+
+
+@pytest.mark.parametrize("tokens,k,n,topk,skew", STREAM_CASES)
+def test_expert_gate_up_stream_matches_oracle(tokens, k, n, topk, skew):
+    groups, a, (qg, qu), codes, scales, host = _stream_operands(tokens, k, n, topk, skew, 2, tokens)
+    want = oracle.swiglu(*(oracle.expert_i4(codes, scales, *h, groups, tokens, topk, k, n, False) for h in host))
+    for _ in range(2):
+        got = clef_i4.omni_gate_up(a, qg, qu, to_dev_f32(groups), tokens, topk)
+        assert_same_bf16_nan_aware(bf16_host(got), want, f"gate/up stream t={tokens} k={k} n={n}")
+
+
 def test_swiglu_every_bf16_gate():
     """swiglu_preserves_materialized_rounding (src/ops.rs:482-520) over all
     65536 gate bit patterns."""
