@@ -14,6 +14,7 @@
 #include "gemm_dma.hpp"
 #include "kernels.hpp"
 #include "group.hpp"
+#include "launch.hpp"
 #include "route.hpp"
 
 namespace clef {
@@ -776,10 +777,127 @@ __global__ __launch_bounds__(64) void router_gate_kernel(const uint16_t* __restr
 #endif
 }
 
+// The same logits for few tokens: a workgroup of four waves takes 16 tokens x
+// 8 experts, so that at one token 16 CUs share the weight rows instead of four,
+// loads all of their hidden dimension into LDS at once (3 KiB per 64-k step)
+// and runs the chain on wave 0, in four phases that start as their quarter of
+// the steps has landed. What is left is a launch, one memory round trip and
+// the chain. Lanes of MFMA rows 16.. and columns 8.. repeat the first ones;
+// their results are not stored. Same chain, same bits as router_gate_kernel.
+constexpr int kRouterSmallTokens = 16, kRouterSmallExperts = 8;
+constexpr int kRouterSmallHidden = 2048;  // two steps per wave and phase
+constexpr int kRouterSmallStage = (kRouterSmallTokens + kRouterSmallExperts) * 128;
+[[maybe_unused]] constexpr int kRouterSmallInst = kRouterSmallStage / 1024;
+__global__ __launch_bounds__(256) void router_gate_small_kernel(const uint16_t* __restrict__ x,
+                                                                const uint16_t* __restrict__ w, int64_t tokens,
+                                                                int hidden, int experts, uint16_t* __restrict__ out) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __align__(16) char lds[];
+  const int groups = experts / kRouterSmallExperts;
+  const int e0 = (int)(blockIdx.x % groups) * kRouterSmallExperts;
+  const int64_t t0 = (int64_t)(blockIdx.x / groups) * kRouterSmallTokens;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // DMA instruction q of a step moves rows 8q .. 8q+7 of x (q < 2) or the
+  // expert rows: lane -> row lane / 8, stored chunk lane % 8 = logical chunk
+  // (lane % 8) ^ ((row >> 1) & 7). Rows past the last token re-read it.
+  const char* src[kRouterSmallInst];
+#pragma unroll
+  for (int q = 0; q < kRouterSmallInst; ++q) {
+    const int row = 8 * (q & 1) + (lane >> 3);
+    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
+    const int64_t t = t0 + row < tokens ? t0 + row : tokens - 1;
+    src[q] = reinterpret_cast<const char*>(q < 2 ? x + t * hidden : w + (int64_t)(e0 + (lane >> 3)) * hidden) +
+             16 * chunk;
+  }
+  const int steps = hidden / 64;
+  const int per = (steps + 15) / 16;  // steps per wave and phase
+  // wave w loads steps (4 p + w) per .. of phase p; a phase's instructions are
+  // the same number for every wave (steps past the last repeat it, into its
+  // own stage: the same bytes)
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+    for (int i = 0; i < per; ++i) {
+      const int step = (4 * p + wave) * per + i;
+      const int kt = step < steps ? step : steps - 1;
+#pragma unroll
+      for (int q = 0; q < kRouterSmallInst; ++q)
+        __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src[q] + (int64_t)kt * 128),
+                                         (lds_ptr_t)(lds + kt * kRouterSmallStage + q * 1024), 16, 0, 0);
+    }
+  const int h = lane >> 5, xr = lane & 15, wr = lane & 7;
+  v16f acc = {};
+  auto phase = [&](int p, auto behind_tag) {
+    constexpr int BEHIND = decltype(behind_tag)::value;
+    // at most the later phases' instructions outstanding (per is 1 or 2: the
+    // launcher's limit on hidden)
+    if (per == 1)
+      wait_vmcnt<BEHIND * kRouterSmallInst>();
+    else
+      wait_vmcnt<BEHIND * 2 * kRouterSmallInst>();
+    asm volatile("s_barrier" ::: "memory");
+    if (wave != 0) return;
+    const int k1 = 4 * (p + 1) * per < steps ? 4 * (p + 1) * per : steps;
+    auto read = [&](int kt, u4 (&a)[4], u4 (&b)[4]) {
+      const char* st = lds + kt * kRouterSmallStage;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        a[s] = *reinterpret_cast<const u4*>(st + xr * 128 + (((2 * s + h) ^ ((xr >> 1) & 7)) << 4));
+        b[s] = *reinterpret_cast<const u4*>(st + 2048 + wr * 128 + (((2 * s + h) ^ ((wr >> 1) & 7)) << 4));
+      }
+    };
+    auto mma = [&](const u4 (&a)[4], const u4 (&b)[4]) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
+                                                      __builtin_bit_cast(bf16x8_t, b[s]), acc, 0, 0, 0);
+    };
+    // a step's operands are read under the MFMAs of the step before
+    const int k0 = 4 * p * per;
+    if (k0 >= k1) return;
+    u4 a0[4], b0[4], a1[4], b1[4];
+    read(k0, a0, b0);
+    for (int kt = k0; kt < k1; kt += 2) {
+      if (kt + 1 < k1) read(kt + 1, a1, b1);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(a0, b0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kt + 1 >= k1) break;
+      if (kt + 2 < k1) read(kt + 2, a0, b0);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(a1, b1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  phase(0, std::integral_constant<int, 3>{});
+  phase(1, std::integral_constant<int, 2>{});
+  phase(2, std::integral_constant<int, 1>{});
+  phase(3, std::integral_constant<int, 0>{});
+  if (wave != 0 || (lane & 31) >= kRouterSmallExperts) return;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {  // rows 8 (i / 4) + 4 h + i % 4 < 16
+    const int64_t t = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
+    if (t < tokens) out[t * experts + e0 + (lane & 31)] = (uint16_t)f32_to_bf16(acc[i]);
+  }
+#endif
+}
+
 hipError_t launch_router_gate(const uint16_t* x, const uint16_t* w, int64_t tokens, int hidden, int experts,
                               uint16_t* out, hipStream_t stream) {
   const int64_t blocks = (tokens + 31) / 32;
   if (blocks == 0) return hipSuccess;
+  // Up to 256 tokens: one workgroup per CU. 1 token 8.2 -> 7.0 us, 33: 8.6 ->
+  // 7.3, 235: 8.7 -> 7.8 (hidden 2048, 128 experts, graph replay).
+  if (tokens <= 256 && hidden <= kRouterSmallHidden) {
+    const int lds = hidden / 64 * kRouterSmallStage;
+    static LaunchCache cache;
+    const void* kern = reinterpret_cast<const void*>(&router_gate_small_kernel);
+    if (hipError_t e = ensure_dynamic_lds(cache, kern, kRouterSmallHidden / 64 * kRouterSmallStage)) return e;
+    const unsigned grid = (unsigned)((tokens + kRouterSmallTokens - 1) / kRouterSmallTokens) *
+                          (experts / kRouterSmallExperts);
+    router_gate_small_kernel<<<grid, 256, lds, stream>>>(x, w, tokens, hidden, experts, out);
+    return hipGetLastError();
+  }
   const int64_t grid = (blocks + 7) / 8 * 8 * (experts / 32);
   router_gate_kernel<<<(unsigned)grid, 64, 0, stream>>>(x, w, tokens, hidden, experts, out);
   return hipGetLastError();

@@ -126,6 +126,23 @@ def test_router_logits_integer_inputs_are_exact(tokens, hidden, experts):
     assert np.array_equal(got, BF(x @ w.T))
 
 
+@pytest.mark.parametrize("hidden,experts", [(64, 32), (448, 96), (960, 64), (1024, 128), (1088, 32), (1984, 128),
+                                            (2048, 128)])
+def test_router_logits_few_tokens_equal_many(hidden, experts):
+    """The kernel for up to 256 tokens runs the same MFMA chain as the one for
+    more: its logits equal the first rows of a 300-token call bit for bit, and
+    those lie within the f32 summation bound of float64."""
+    g = torch.Generator(device="cuda").manual_seed(hidden + experts)
+    x = torch.randn((300, hidden), generator=g, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn((experts, hidden), generator=g, device="cuda", dtype=torch.bfloat16)
+    many = clef_i4.router_logits(x, w).view(torch.int16)
+    for n in (1, 15, 16, 17, 240, 256):
+        assert torch.equal(clef_i4.router_logits(x[:n].contiguous(), w).view(torch.int16), many[:n]), n
+    xd, wd = x.double(), w.double()
+    bound = hidden * 2.0 ** -23 * (xd.abs() @ wd.abs().t()) + 2.0 ** -8 * (xd @ wd.t()).abs() + 1e-30
+    assert bool(((many.view(torch.bfloat16).double() - xd @ wd.t()).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("producer,width,bits,extra", [
     (0, 256, 4, 0), (0, 1024, 4, 0), (0, 768, 8, 128), (0, 4096, 8, 0), (0, 5120, 4, 1024), (0, 12288, 8, 0),
     (1, 2048, 4, 256), (1, 17408, 4, 0), (1, 6144, 8, 0), (2, 1024, 8, 0), (2, 5120, 4, 0), (3, 5120, 4, 0),
