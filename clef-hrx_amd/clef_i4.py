@@ -12,6 +12,9 @@ path.
 from __future__ import annotations
 
 import ctypes
+import functools
+import importlib.machinery
+import importlib.util
 import os
 from dataclasses import dataclass
 
@@ -19,6 +22,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libclef_i4.so")
+HOST_PATH = os.path.join(_HERE, "lib", "clef_host.so")
 
 _P = ctypes.c_void_p
 _I64 = ctypes.c_int64
@@ -119,25 +123,33 @@ def _check(rc: int) -> None:
         raise ClefError(rc, lib().clef_last_error().decode())
 
 
-def _ptr(t):
-    if t is None:
-        return None
-    if isinstance(t, int):
-        return t
-    assert t.is_cuda and t.is_contiguous(), "device tensors must be contiguous CUDA tensors"
-    return t.data_ptr()
+class _Native:
+    """The call module (csrc/host_call.cpp: launch, value, pointer, empty) and
+    the address of every entry point, as attributes; filled on first use."""
+
+    def __getattr__(self, name):
+        handle = lib()
+        loader = importlib.machinery.ExtensionFileLoader("clef_host", HOST_PATH)
+        host = importlib.util.module_from_spec(importlib.util.spec_from_loader("clef_host", loader))
+        loader.exec_module(host)
+        built = handle.clef_build_id().decode()
+        if host.build_id != built:
+            raise ImportError(f"{HOST_PATH} was built from other sources (module {host.build_id}, library {built})")
+        host.set_check(_check)
+        found = {entry: ctypes.cast(getattr(handle, entry), ctypes.c_void_p).value for entry in SIGNATURES}
+        found.update(launch=host.launch, value=host.value, pointer=host.pointer, empty=host.empty)
+        if name not in found:
+            raise AttributeError(name)
+        self.__dict__.update(found)
+        return found[name]
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
-
-
-def _empty(shape, dtype, device):
-    return torch.empty(shape, dtype=dtype, device=device)
+_n = _Native()
 
 
 # ---------------------------------------------------------------- Q1 / Q2
 
+@functools.lru_cache(maxsize=256)
 def activation_stride(width: int, bits: int = 4) -> int:
     """src/quantized.rs:161-166."""
     return int(lib().clef_i4_activation_stride(width, bits))
@@ -165,14 +177,20 @@ class Prepared:
         start = self.rows * self.words
         return self.storage[start: start + self.rows].view(torch.float32)
 
+    def scales_arg(self):
+        """scales as a call argument: its address, without slicing a view."""
+        start = self.rows * self.words
+        if self.storage.dtype != torch.int32 or self.storage.numel() < start + self.rows:
+            return self.scales
+        return _n.pointer(self.storage) + 4 * start
+
 
 def _prepare_filled(producer: int, x, second, rows: int, width: int, stride: int, bits: int) -> Prepared:
     """A new Prepared of one of the library's producers (CLEF_PRODUCER_*); the
     kernel writes every word of it, padding as zeros."""
-    words = int(lib().clef_i4_prepared_words(rows, stride, bits))
-    out = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
-    _check(lib().clef_i4_prepare_filled(_ptr(x), _ptr(second), producer, rows, width, stride, bits, _ptr(out),
-                                        _stream()))
+    words = _n.value(_n.clef_i4_prepared_words, rows, stride, bits)
+    out = _n.empty(x, torch.int32, max(words, 1))
+    _n.launch(_n.clef_i4_prepare_filled, x, second, producer, rows, width, stride, bits, out)
     return Prepared(out, rows, width, stride, bits)
 
 
@@ -183,7 +201,7 @@ def prepare(x: torch.Tensor, bits: int = 4, stride: int | None = None, out: torc
     stride = activation_stride(width, bits) if stride is None else stride
     if out is None:
         return _prepare_filled(0, x, None, rows, width, stride, bits)
-    _check(lib().clef_i4_prepare(_ptr(x), rows, width, stride, bits, _ptr(out), _stream()))
+    _n.launch(_n.clef_i4_prepare, x, rows, width, stride, bits, out)
     return Prepared(out, rows, width, stride, bits)
 
 
@@ -219,8 +237,7 @@ def prepare_norm(x: torch.Tensor, weight: torch.Tensor, bits: int = 4, stride: i
         return _prepare_filled(3, x, weight.contiguous(), rows, width, stride, bits), None
     total = int(lib().clef_i4_prepare_norm_words(rows, width, stride, bits, int(store)))
     out = torch.zeros(max(total, 1), dtype=torch.int32, device=x.device)
-    _check(lib().clef_i4_prepare_norm(_ptr(x), _ptr(weight.contiguous()), rows, width, stride, bits, int(store),
-                                      _ptr(out), _stream()))
+    _n.launch(_n.clef_i4_prepare_norm, x, weight.contiguous(), rows, width, stride, bits, int(store), out)
     first = total - rows * width // 2
     normalized = out[first:].view(torch.bfloat16).view(rows, width)
     return Prepared(out, rows, width, stride, bits), normalized
@@ -230,8 +247,7 @@ def retile_codes(codes: torch.Tensor, rows: int, cols: int, bits: int = 4) -> to
     """quantized::retile_codes (src/quantized.rs:542-572); codes [rows][in_words]."""
     in_words = codes.shape[1]
     tiled = torch.empty(rows * cols // (32 // bits), dtype=torch.int32, device=codes.device)
-    _check(lib().clef_i4_retile(_ptr(codes.contiguous()), rows, in_words, cols, bits, _ptr(tiled),
-                                _stream()))
+    _n.launch(_n.clef_i4_retile, codes.contiguous(), rows, in_words, cols, bits, tiled)
     return tiled
 
 
@@ -414,8 +430,7 @@ def _pack(w: torch.Tensor, bits: int, tiled_checkpoint: bool) -> QuantizedWeight
     rows, cols = w.shape
     codes = torch.empty(rows * cols // (32 // bits), dtype=torch.int32, device=w.device)
     scales = torch.empty(rows, dtype=torch.float32, device=w.device)
-    _check(lib().clef_i4_pack_checkpoint(_ptr(w), rows, cols, bits, int(tiled_checkpoint), _ptr(codes), _ptr(scales),
-                                         _stream()))
+    _n.launch(_n.clef_i4_pack_checkpoint, w, rows, cols, bits, int(tiled_checkpoint), codes, scales)
     return QuantizedWeight(codes, scales, rows, cols, activation_stride(cols, bits), bits)
 
 
@@ -438,14 +453,14 @@ def load_expert_layer(experts: list[torch.Tensor], rows: int, cols: int, bits: i
 def untile_rows(tiled: torch.Tensor) -> torch.Tensor:
     rows, cols = tiled.shape
     out = torch.empty_like(tiled)
-    _check(lib().clef_untile_rows(_ptr(tiled), rows, cols, _ptr(out), _stream()))
+    _n.launch(_n.clef_untile_rows, tiled, rows, cols, out)
     return out
 
 
 def tile_rows(dense: torch.Tensor) -> torch.Tensor:
     rows, cols = dense.shape
     out = torch.empty_like(dense)
-    _check(lib().clef_tile_rows(_ptr(dense), rows, cols, _ptr(out), _stream()))
+    _n.launch(_n.clef_tile_rows, dense, rows, cols, out)
     return out
 
 
@@ -459,16 +474,15 @@ def project_prepared(a: Prepared, w: QuantizedWeight, residual: torch.Tensor | N
                      config: int = -1, out: torch.Tensor | None = None) -> torch.Tensor:
     """Engine::project_prepared (src/quantized.rs:470-537)."""
     if out is None:
-        out = _empty((a.rows, w.rows), torch.bfloat16, a.storage.device)
+        out = _n.empty(a.storage, torch.bfloat16, a.rows, w.rows)
     if a.bits != w.bits:
         raise ClefError(-1, "unsupported integer projection shape")
     if w.bits == 8:  # h3_gemm_i8_256
-        _check(lib().clef_i8_gemm(_ptr(a.storage), a.stride, _ptr(a.scales), _ptr(w.codes), _ptr(w.scales),
-                                  a.rows, w.rows, w.cols, _ptr(residual), _ptr(out), _stream()))
+        _n.launch(_n.clef_i8_gemm, a.storage, a.stride, a.scales_arg(), w.codes, w.scales, a.rows, w.rows, w.cols,
+                  residual, out)
         return out
-    _check(lib().clef_i4_gemm_config(_ptr(a.storage), a.stride, _ptr(a.scales), _ptr(w.codes),
-                                     _ptr(w.scales), a.rows, w.rows, w.cols, _ptr(residual), _ptr(out),
-                                     config, _stream()))
+    _n.launch(_n.clef_i4_gemm_config, a.storage, a.stride, a.scales_arg(), w.codes, w.scales, a.rows, w.rows, w.cols,
+              residual, out, config)
     return out
 
 
@@ -487,7 +501,7 @@ def f6_weight(w: QuantizedWeight) -> F6Weight:
     if w.bits != 4:
         raise ClefError(-1, "unsupported integer projection shape")
     codes = torch.empty(w.rows * w.cols * 3 // 4, dtype=torch.uint8, device=w.codes.device)
-    _check(lib().clef_i4_f6_weight(_ptr(w.codes), w.rows, w.cols, _ptr(codes), _stream()))
+    _n.launch(_n.clef_i4_f6_weight, w.codes, w.rows, w.cols, codes)
     return F6Weight(codes, w.scales, w.rows, w.cols)
 
 
@@ -507,7 +521,7 @@ def f6_activation(a: Prepared, out: torch.Tensor | None = None) -> torch.Tensor:
         out = torch.empty(nbytes, dtype=torch.uint8, device=a.storage.device)
     elif out.dtype != torch.uint8 or out.numel() < nbytes:
         raise ClefError(-1, "bf6 activation buffer too small")
-    _check(lib().clef_i4_f6_activation(_ptr(a.storage), a.stride, a.rows, a.width, _ptr(out), _stream()))
+    _n.launch(_n.clef_i4_f6_activation, a.storage, a.stride, a.rows, a.width, out)
     return out
 
 
@@ -519,9 +533,8 @@ def gemm_f6(a_f6: torch.Tensor, a_scales: torch.Tensor, w: F6Weight, residual: t
     if a_f6.numel() < f6_codes_bytes(rows, w.cols):
         raise ClefError(-1, "bf6 activation buffer too small")
     if out is None:
-        out = _empty((rows, w.rows), torch.bfloat16, a_f6.device)
-    _check(lib().clef_i4_gemm_f6(_ptr(a_f6), _ptr(a_scales), _ptr(w.codes), _ptr(w.scales), rows, w.rows, w.cols,
-                                 _ptr(residual), _ptr(out), _stream()))
+        out = _n.empty(a_f6, torch.bfloat16, rows, w.rows)
+    _n.launch(_n.clef_i4_gemm_f6, a_f6, a_scales, w.codes, w.scales, rows, w.rows, w.cols, residual, out)
     return out
 
 
@@ -543,11 +556,19 @@ class PreparedF6:
         start = f6_codes_bytes(self.rows, self.width)
         return self.storage[start: start + 4 * self.rows].view(torch.float32)
 
+    def call_args(self):
+        """codes and scales as call arguments: addresses, without slicing views."""
+        start = f6_codes_bytes(self.rows, self.width)
+        if self.storage.dtype != torch.uint8 or self.storage.numel() < start + 4 * self.rows:
+            return self.codes, self.scales
+        base = _n.pointer(self.storage)
+        return base, base + start
 
-def _prepared_f6_storage(rows: int, width: int, device, out: torch.Tensor | None) -> torch.Tensor:
-    nbytes = int(lib().clef_i4_f6_prepared_bytes(rows, width))
+
+def _prepared_f6_storage(rows: int, width: int, x: torch.Tensor, out: torch.Tensor | None) -> torch.Tensor:
+    nbytes = _n.value(_n.clef_i4_f6_prepared_bytes, rows, width)
     if out is None:
-        return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+        return _n.empty(x, torch.uint8, max(nbytes, 1))
     if out.dtype != torch.uint8 or out.numel() < nbytes:
         raise ClefError(-1, "bf6 activation buffer too small")
     return out
@@ -557,16 +578,16 @@ def prepare_f6(x: torch.Tensor, out: torch.Tensor | None = None) -> PreparedF6:
     """prepare (bits 4) with the codes written as bf6: the same codes and
     scales as prepare followed by f6_activation, in one pass."""
     rows, width = x.shape
-    out = _prepared_f6_storage(rows, width, x.device, out)
-    _check(lib().clef_i4_prepare_f6(_ptr(x), rows, width, _ptr(out), _stream()))
+    out = _prepared_f6_storage(rows, width, x, out)
+    _n.launch(_n.clef_i4_prepare_f6, x, rows, width, out)
     return PreparedF6(out, rows, width)
 
 
 def prepare_swiglu_f6(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None) -> PreparedF6:
     """prepare_swiglu (bits 4) with the codes written as bf6."""
     rows, width = gate.shape
-    out = _prepared_f6_storage(rows, width, gate.device, out)
-    _check(lib().clef_i4_prepare_swiglu_f6(_ptr(gate), _ptr(up), rows, width, _ptr(out), _stream()))
+    out = _prepared_f6_storage(rows, width, gate, out)
+    _n.launch(_n.clef_i4_prepare_swiglu_f6, gate, up, rows, width, out)
     return PreparedF6(out, rows, width)
 
 
@@ -576,7 +597,13 @@ def project_f6(a: PreparedF6, w: F6Weight, residual: torch.Tensor | None = None,
     project_prepared(prepare(x), w) for the weight w came from."""
     if a.width != w.cols:
         raise ClefError(-1, "unsupported integer projection shape")
-    return gemm_f6(a.codes, a.scales, w, residual, out)
+    codes, scales = a.call_args()
+    if not isinstance(codes, int):
+        return gemm_f6(codes, scales, w, residual, out)
+    if out is None:
+        out = _n.empty(a.storage, torch.bfloat16, a.rows, w.rows)
+    _n.launch(_n.clef_i4_gemm_f6, codes, scales, w.codes, w.scales, a.rows, w.rows, w.cols, residual, out)
+    return out
 
 
 def project_gate_up_f6(a: PreparedF6, gate: F6Weight, up: F6Weight, out: torch.Tensor | None = None
@@ -588,10 +615,10 @@ def project_gate_up_f6(a: PreparedF6, gate: F6Weight, up: F6Weight, out: torch.T
     if a.width != gate.cols or gate.cols != up.cols or gate.rows != up.rows:
         raise ClefError(-1, "unsupported integer projection shape")
     if out is None:
-        out = _empty((a.rows, gate.rows), torch.bfloat16, a.storage.device)
-    _check(lib().clef_i4_gemm_f6_gate_up(_ptr(a.codes), _ptr(a.scales), _ptr(gate.codes), _ptr(gate.scales),
-                                         _ptr(up.codes), _ptr(up.scales), a.rows, gate.rows, gate.cols, _ptr(out),
-                                         _stream()))
+        out = _n.empty(a.storage, torch.bfloat16, a.rows, gate.rows)
+    codes, scales = a.call_args()
+    _n.launch(_n.clef_i4_gemm_f6_gate_up, codes, scales, gate.codes, gate.scales, up.codes, up.scales, a.rows,
+              gate.rows, gate.cols, out)
     return out
 
 
@@ -602,11 +629,10 @@ def project_quantized_f6(x: torch.Tensor, w: F6Weight, residual: torch.Tensor | 
     GEMM. Same output as project_quantized(x, the 4-bit weight)."""
     m, k = x.shape
     if out is None:
-        out = _empty((m, w.rows), torch.bfloat16, x.device)
-    nbytes = int(lib().clef_i4_project_f6_workspace_bytes(m, k))
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
-    _check(lib().clef_i4_project_f6(_ptr(x), m, k, _ptr(w.codes), _ptr(w.scales), w.rows, _ptr(residual), _ptr(out),
-                                    _ptr(ws), nbytes, _stream()))
+        out = _n.empty(x, torch.bfloat16, m, w.rows)
+    nbytes = _n.value(_n.clef_i4_project_f6_workspace_bytes, m, k)
+    ws = _n.empty(x, torch.uint8, max(nbytes, 1))
+    _n.launch(_n.clef_i4_project_f6, x, m, k, w.codes, w.scales, w.rows, residual, out, ws, nbytes)
     return out
 
 
@@ -622,11 +648,10 @@ def project_quantized(x: torch.Tensor, w: QuantizedWeight, residual: torch.Tenso
                       ) -> torch.Tensor:
     """Engine::project_quantized[_with_residual] (src/quantized.rs:235-303)."""
     m, k = x.shape
-    out = _empty((m, w.rows), torch.bfloat16, x.device)
-    ws_bytes = int(lib().clef_i4_project_workspace_bytes(m, k))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=x.device)
-    _check(lib().clef_i4_project(_ptr(x), m, k, _ptr(w.codes), _ptr(w.scales), w.rows, _ptr(residual),
-                                 _ptr(out), _ptr(ws), ws_bytes, _stream()))
+    out = _n.empty(x, torch.bfloat16, m, w.rows)
+    ws_bytes = _n.value(_n.clef_i4_project_workspace_bytes, m, k)
+    ws = _n.empty(x, torch.uint8, max(ws_bytes, 16))
+    _n.launch(_n.clef_i4_project, x, m, k, w.codes, w.scales, w.rows, residual, out, ws, ws_bytes)
     return out
 
 
@@ -649,9 +674,8 @@ def router_logits(x: torch.Tensor, gate_w: torch.Tensor) -> torch.Tensor:
     experts = gate_w.shape[0]
     if gate_w.shape[1] != hidden or x.dtype != torch.bfloat16 or gate_w.dtype != torch.bfloat16:
         raise ClefError(-1, "linear shape/dtype mismatch")
-    out = _empty((tokens, experts), torch.bfloat16, x.device)
-    _check(lib().clef_moe_router_logits(_ptr(x.contiguous()), _ptr(gate_w.contiguous()), tokens, hidden, experts,
-                                        _ptr(out), _stream()))
+    out = _n.empty(x, torch.bfloat16, tokens, experts)
+    _n.launch(_n.clef_moe_router_logits, x.contiguous(), gate_w.contiguous(), tokens, hidden, experts, out)
     return out
 
 
@@ -659,8 +683,8 @@ def omni_route(logits: torch.Tensor, topk: int = 8) -> torch.Tensor:
     """Engine::omni_route (src/omni.rs:170-190)."""
     tokens, experts = logits.shape
     dtype = 0 if logits.dtype == torch.bfloat16 else 1
-    routes = _empty((tokens, 2 * topk), torch.float32, logits.device)
-    _check(lib().clef_moe_route(_ptr(logits), dtype, tokens, experts, topk, _ptr(routes), _stream()))
+    routes = _n.empty(logits, torch.float32, tokens, 2 * topk)
+    _n.launch(_n.clef_moe_route, logits, dtype, tokens, experts, topk, routes)
     return routes
 
 
@@ -670,10 +694,9 @@ def omni_group_routes(routes: torch.Tensor, ordered: bool = True):
     topk = routes.shape[1] // 2
     groups = torch.zeros((128, tokens + 1), dtype=torch.float32, device=routes.device)
     order = torch.zeros((tokens, topk), dtype=torch.float32, device=routes.device) if ordered else None
-    ws_bytes = int(lib().clef_moe_group_workspace_bytes(tokens))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=routes.device)
-    _check(lib().clef_moe_group_routes(_ptr(routes), tokens, topk, _ptr(groups), _ptr(order), _ptr(ws),
-                                       ws_bytes, _stream()))
+    ws_bytes = _n.value(_n.clef_moe_group_workspace_bytes, tokens)
+    ws = _n.empty(routes, torch.uint8, max(ws_bytes, 16))
+    _n.launch(_n.clef_moe_group_routes, routes, tokens, topk, groups, order, ws, ws_bytes)
     return groups, order
 
 
@@ -682,7 +705,7 @@ def omni_expert_tasks(groups: torch.Tensor, topk: int = 8) -> torch.Tensor:
     tokens = groups.shape[1] - 1
     tasks = torch.zeros(1 + 2 * ((tokens * topk + 15) // 16 + 127), dtype=torch.float32,
                         device=groups.device)
-    _check(lib().clef_moe_expert_tasks(_ptr(groups), tokens, _ptr(tasks), _stream()))
+    _n.launch(_n.clef_moe_expert_tasks, groups, tokens, tasks)
     return tasks
 
 
@@ -691,11 +714,10 @@ def omni_expert(a: Prepared, w: QuantizedWeight, groups: torch.Tensor, tokens: i
     """Engine::omni_expert_impl (src/omni.rs:289-534); w holds 128 experts' rows."""
     n = w.rows // 128
     out = torch.zeros((tokens * topk, n), dtype=torch.bfloat16, device=groups.device)
-    ws_bytes = int(lib().clef_moe_expert_workspace_bytes(tokens, topk))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=groups.device)
-    _check(lib().clef_moe_expert_i4(_ptr(a.storage), a.stride, _ptr(a.scales), _ptr(w.codes),
-                                    _ptr(w.scales), _ptr(groups), tokens, topk, w.cols, n,
-                                    int(input_routed), _ptr(out), _ptr(ws), ws_bytes, _stream()))
+    ws_bytes = _n.value(_n.clef_moe_expert_workspace_bytes, tokens, topk)
+    ws = _n.empty(groups, torch.uint8, max(ws_bytes, 16))
+    _n.launch(_n.clef_moe_expert_i4, a.storage, a.stride, a.scales_arg(), w.codes, w.scales, groups, tokens, topk,
+              w.cols, n, int(input_routed), out, ws, ws_bytes)
     return out
 
 
@@ -708,11 +730,10 @@ def omni_expert_ungrouped(a: Prepared, w: QuantizedWeight, routes: torch.Tensor,
     topk = routes.shape[1] // 2
     n = w.rows // 128
     out = torch.zeros((tokens * topk, n), dtype=torch.bfloat16, device=routes.device)
-    ws_bytes = int(lib().clef_moe_expert_ungrouped_workspace_bytes(tokens, topk))
-    ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=routes.device)
-    _check(lib().clef_moe_expert_i4_ungrouped(_ptr(a.storage), a.stride, _ptr(a.scales), _ptr(w.codes),
-                                              _ptr(w.scales), _ptr(routes), tokens, topk, w.cols, n,
-                                              int(input_routed), _ptr(out), _ptr(ws), ws_bytes, _stream()))
+    ws_bytes = _n.value(_n.clef_moe_expert_ungrouped_workspace_bytes, tokens, topk)
+    ws = _n.empty(routes, torch.uint8, max(ws_bytes, 256))
+    _n.launch(_n.clef_moe_expert_i4_ungrouped, a.storage, a.stride, a.scales_arg(), w.codes, w.scales, routes, tokens,
+              topk, w.cols, n, int(input_routed), out, ws, ws_bytes)
     return out
 
 
@@ -722,11 +743,10 @@ def omni_gate_up(a: Prepared, gate: QuantizedWeight, up: QuantizedWeight, groups
     and SwiGLU over the routed rows; h bf16 [tokens * topk][n]."""
     n = gate.rows // 128
     h = torch.zeros((tokens * topk, n), dtype=torch.bfloat16, device=groups.device)
-    ws_bytes = int(lib().clef_moe_expert_workspace_bytes(tokens, topk))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=groups.device)
-    _check(lib().clef_moe_expert_gate_up_i4(_ptr(a.storage), a.stride, _ptr(a.scales), _ptr(gate.codes),
-                                            _ptr(gate.scales), _ptr(up.codes), _ptr(up.scales), _ptr(groups),
-                                            tokens, topk, gate.cols, n, _ptr(h), _ptr(ws), ws_bytes, _stream()))
+    ws_bytes = _n.value(_n.clef_moe_expert_workspace_bytes, tokens, topk)
+    ws = _n.empty(groups, torch.uint8, max(ws_bytes, 16))
+    _n.launch(_n.clef_moe_expert_gate_up_i4, a.storage, a.stride, a.scales_arg(), gate.codes, gate.scales, up.codes,
+              up.scales, groups, tokens, topk, gate.cols, n, h, ws, ws_bytes)
     return h
 
 
@@ -735,7 +755,7 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     if gate.shape != up.shape:
         raise ClefError(-1, "SwiGLU shape/dtype mismatch")
     h = torch.empty_like(gate)
-    _check(lib().clef_swiglu(_ptr(gate), _ptr(up), gate.numel(), _ptr(h), _stream()))
+    _n.launch(_n.clef_swiglu, gate, up, gate.numel(), h)
     return h
 
 
@@ -745,9 +765,8 @@ def omni_combine(values: torch.Tensor, routes: torch.Tensor, order: torch.Tensor
     tokens = routes.shape[0]
     topk = routes.shape[1] // 2
     width = values.shape[1]
-    out = _empty((tokens, width), torch.bfloat16, values.device)
-    _check(lib().clef_moe_combine(_ptr(values), _ptr(routes), _ptr(order), tokens, width, topk, _ptr(out),
-                                  _stream()))
+    out = _n.empty(values, torch.bfloat16, tokens, width)
+    _n.launch(_n.clef_moe_combine, values, routes, order, tokens, width, topk, out)
     return out
 
 
@@ -768,7 +787,7 @@ class MoeLayer:
 
     def workspace(self, tokens: int, device) -> torch.Tensor:
         if self._ws_tokens != tokens:
-            nbytes = int(lib().clef_moe_layer_workspace_bytes(tokens, self.hidden, self.inter, self.topk))
+            nbytes = _n.value(_n.clef_moe_layer_workspace_bytes, tokens, self.hidden, self.inter, self.topk)
             self._ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
             self._ws_tokens = tokens
         return self._ws
@@ -781,12 +800,10 @@ class MoeLayer:
                 raise ClefError(-1, "MoE layer needs router logits or a router gate weight")
             logits = router_logits(x, self.router)  # e.project(norm, "mlp.gate"), src/omni.rs:764
         if out is None:
-            out = _empty((tokens, self.hidden), torch.bfloat16, x.device)
+            out = _n.empty(x, torch.bfloat16, tokens, self.hidden)
         ws = self.workspace(tokens, x.device)
         dtype = 0 if logits.dtype == torch.bfloat16 else 1
-        _check(lib().clef_moe_layer(_ptr(x), _ptr(logits), dtype, tokens, self.hidden, self.inter, 128,
-                                    self.topk, _ptr(self.gate.codes), _ptr(self.gate.scales),
-                                    _ptr(self.up.codes), _ptr(self.up.scales), _ptr(self.down.codes),
-                                    _ptr(self.down.scales), _ptr(routes_out), _ptr(out), _ptr(ws),
-                                    ws.numel(), _stream()))
+        _n.launch(_n.clef_moe_layer, x, logits, dtype, tokens, self.hidden, self.inter, 128, self.topk,
+                  self.gate.codes, self.gate.scales, self.up.codes, self.up.scales, self.down.codes, self.down.scales,
+                  routes_out, out, ws, ws.numel())
         return out

@@ -407,3 +407,28 @@ def test_resident_bytes_count_the_kept_weight_forms():
         clef_i4.QuantizedProjections(bits=4, forms=("int4", "fp8"))
     with pytest.raises(ValueError):
         clef_i4.QuantizedProjections(bits=4, forms=())
+
+
+def test_call_module_converts_and_checks_arguments():
+    """The binding's call module: size functions as through ctypes, the device
+    and contiguity check on tensor arguments, allocation like torch.empty,
+    and errors for what is neither tensor, integer nor None."""
+    import torch
+
+    n = clef_i4._n
+    for rows, stride, bits in [(3, 256, 4), (7, 1088, 8), (1 << 20, 65536, 4), (5, 256, 3)]:
+        assert n.value(n.clef_i4_prepared_words, rows, stride, bits) == \
+            clef_i4.lib().clef_i4_prepared_words(rows, stride, bits)
+    cpu = torch.zeros(4)
+    with pytest.raises(AssertionError, match="contiguous CUDA tensors"):
+        n.launch(n.clef_swiglu, cpu, cpu, 4, cpu)
+    with pytest.raises(AssertionError, match="contiguous CUDA tensors"):
+        n.pointer(cpu)
+    with pytest.raises(TypeError, match="unsupported argument type float"):
+        n.value(n.clef_i4_prepared_words, 1.5, 256, 4)
+    e = n.empty(cpu, torch.bfloat16, 2, 3)
+    assert e.shape == (2, 3) and e.dtype == torch.bfloat16 and e.device == cpu.device
+    with pytest.raises(RuntimeError):
+        n.empty(cpu, torch.float32, -1)
+    with pytest.raises(AttributeError):
+        n.no_such_entry
