@@ -185,7 +185,6 @@ template <int BITS>
 __device__ __forceinline__ uint32_t pack_codes(const float* v, float inv, bool valid) {
   constexpr int per = 32 / BITS;
   constexpr float qmax = BITS == 8 ? 127.0f : 7.0f;
-  constexpr uint32_t mask = BITS == 8 ? 0xffu : 0xfu;
   // Round to nearest even by adding 1.5 * 2^23: when valid, |v * inv| <= qmax
   // (times 1 + 2^-22), so the sum lies in [2^23, 2^24), where the f32 spacing is
   // 1 and the addend is even; the add then rounds exactly as rint does, and
@@ -193,13 +192,20 @@ __device__ __forceinline__ uint32_t pack_codes(const float* v, float inv, bool v
   // mantissa is 0x400000). Clamping the biased value to magic +- qmax is the
   // clamp of n.
   constexpr float magic = 12582912.0f;
-  uint32_t word = 0;
+  // The biased bit patterns are summed with their shifts: sum (B + n_p) 2^(BITS p)
+  // mod 2^32, B the addend's bits. With half the field's range added to each
+  // n_p no field borrows from the next, and flipping each field's top bit
+  // takes the half off again in two's complement: one shift-add per code and
+  // two operations per word.
+  constexpr uint32_t ones = BITS == 8 ? 0x01010101u : 0x11111111u, half = BITS == 8 ? 0x80u : 0x8u;
+  uint32_t word = 0u - 0x4B400000u * ones + half * ones;
 #pragma unroll
   for (int p = 0; p < per; ++p) {
     float t = v[p] * inv + magic;
     t = __builtin_fminf(__builtin_fmaxf(t, magic - qmax), magic + qmax);
-    word |= (as_uint(t) & mask) << (p * BITS);
+    word += as_uint(t) << (p * BITS);
   }
+  word ^= half * ones;
   return valid ? word : 0u;
 }
 
