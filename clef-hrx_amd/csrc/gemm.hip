@@ -1634,8 +1634,8 @@ __device__ __forceinline__ void q1_rows_lds(RowFn row, int G, float (*qbuf)[16 *
     for (int i = 0; i < 16; ++i) v[i] = 0.0f;
   }
   float* buf = qbuf[m < MR ? m * QG + g : 0];
-  radix4x2(v);  // strides 1 and 4
-  if (m < MR) {
+  if (m < MR) {  // waves past the rows skip the work between the barriers
+    radix4x2(v);  // strides 1 and 4
     float4* wrow = reinterpret_cast<float4*>(buf + L * 20);
 #pragma unroll
     for (int c = 0; c < 4; ++c) wrow[c] = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
@@ -1646,18 +1646,18 @@ __device__ __forceinline__ void q1_rows_lds(RowFn row, int G, float (*qbuf)[16 *
     for (int k = 0; k < 16; ++k) v[k] = buf[k * 20 + L];
   }
   __syncthreads();
-  radix4x2(v);  // strides 16 and 64 (value k holds index L + 16 k)
-  uint32_t mbits = 0;
-  if (on) {
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const uint32_t a = as_uint(v[k]) & 0x7fffffffu;
-      mbits = mbits > a ? mbits : a;
-    }
-  }
-  mbits = group_max16(mbits);
-  if (m < MR && L == 0) qmax_s[m * QG + g] = mbits;
   if (m < MR) {
+    radix4x2(v);  // strides 16 and 64 (value k holds index L + 16 k)
+    uint32_t mbits = 0;
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const uint32_t a = as_uint(v[k]) & 0x7fffffffu;
+        mbits = mbits > a ? mbits : a;
+      }
+    }
+    mbits = group_max16(mbits);
+    if (L == 0) qmax_s[m * QG + g] = mbits;
 #pragma unroll
     for (int k = 0; k < 16; ++k) buf[k * 20 + L] = v[k];
   }
@@ -2053,6 +2053,116 @@ __global__ __launch_bounds__(512) void moe_down_combine_kernel(
 #endif
 }
 
+// project_quantized for a token or a few: Q1(x) and the dot-product G1 in one
+// launch. Every workgroup quantizes the rows itself into LDS (q1_rows_lds: the
+// codes and scales clef_i4_prepare writes) while its weight loads, issued
+// first and all of them at once (one round: U k-steps per wave), are in
+// flight; the sums and the epilogue are gemm_decode_kernel's. The quantizer's
+// launch, its write and the gap after it cost more than repeating it (graph
+// replay, three weights in turn): 1 x 12288 x 4096 8.9 -> 7.2 us, 1 x 2048 x
+// 2048 5.2 -> 3.5, 2 x 4096 x 4096 5.9 -> 4.6, 4 x 1024 x 1024 5.6 -> 4.4.
+template <int MR, int QG, int RW, bool RESID>
+__global__ __launch_bounds__(512) void gemm_decode_q_kernel(const uint16_t* __restrict__ x,
+                                                            const uint32_t* __restrict__ w,
+                                                            const float* __restrict__ ws, int M, int N, int kb,
+                                                            const uint16_t* __restrict__ residual,
+                                                            uint16_t* __restrict__ out) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int NW = 8, J = RW / 8, U = QG / NW;
+  static_assert(MR * QG * 16 <= NW * 64 && QG % NW == 0 && MR * RW <= NW * 64, "one thread per 16 values");
+  asm volatile("" ::"s"(x), "s"(w), "s"(ws), "s"(residual), "s"(out), "s"(M), "s"(N), "s"(kb));
+  __shared__ __align__(16) float qbuf[MR * QG][16 * 20];
+  __shared__ uint32_t qmax_s[MR * QG];
+  __shared__ __align__(16) uint32_t qcodes[MR][QG * 32];
+  __shared__ float qscale[MR][2];
+  __shared__ int red[NW][MR][RW];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int seg = lane & 7, r8 = lane >> 3;
+  const int n0 = blockIdx.x * RW;
+  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(w + (int64_t)(n0 / 128) * kb * 4096, (uint32_t)(kb * 16384));
+  const int w_voff = ((n0 % 128) + r8) * 128 + 16 * seg;
+  v4i wv[U][J];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int j = 0; j < J; ++j)  // k-steps past kb leave the resource (read 0)
+      wv[u][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_voff + 1024 * j, (wave + NW * u) * 16384, 0);
+  const int em = threadIdx.x / RW, er = threadIdx.x % RW;
+  const bool epi = threadIdx.x < MR * RW && em < M;
+  float e_ws = 0.0f;
+  uint32_t e_res = 0;
+  if (epi) {
+    e_ws = ws[n0 + er];
+    if (RESID) e_res = residual[(int64_t)em * N + n0 + er];
+  }
+  q1_rows_lds<MR, QG>([&](int m) -> const uint16_t* { return m < M ? x + (int64_t)m * (kb * 256) : nullptr; }, kb, qbuf,
+                      qmax_s, qcodes, qscale);
+  int acc[J][MR];
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int m = 0; m < MR; ++m) acc[j][m] = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int kt = wave + NW * u;
+    if (kt >= kb) break;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+      const v4i av = m < M ? *reinterpret_cast<const v4i*>(&qcodes[m][kt * 32 + 4 * seg]) : v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[j][m] = __builtin_amdgcn_sdot8(wv[u][j][c], av[c], acc[j][m], false);
+    }
+  }
+  // the eight segments of a row, then the waves (as gemm_decode_kernel)
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+      int v = acc[j][m];
+      v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
+      v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
+      v += __builtin_amdgcn_ds_swizzle(v, 0x101F);
+      if (seg == 0) red[wave][m][r8 + 8 * j] = v;
+    }
+  __syncthreads();
+  if (epi) {
+    int sum = 0;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) sum += red[q][em][er];
+    uint32_t v = g1_value<0>(sum, e_ws, qscale[em][0]);
+    if (RESID) v = f32_to_bf16(bf16_lo(e_res) + bf16_lo(v));
+    out[(int64_t)em * N + n0 + er] = (uint16_t)v;
+  }
+#endif
+}
+
+template <int MR, int QG>
+hipError_t launch_decode_q(const uint16_t* x, const uint32_t* w, const float* ws, int64_t m, int n, int k,
+                           const uint16_t* residual, uint16_t* out, hipStream_t stream) {
+  // 32 columns per workgroup where that still gives 160 of them (1 x 5120 x
+  // 8192 7.3 us against 8.0 with 16, 2 x 12288 x 2048 6.1 / 6.5; 1 x 4096 x
+  // 4096 4.1 / 4.0, 4 x 2048 x 2048 5.1 / 4.5).
+#define CLEF_DECQ(RW, RESID)                                                                                         \
+  gemm_decode_q_kernel<MR, QG, RW, RESID><<<(unsigned)(n / RW), 512, 0, stream>>>(x, w, ws, (int)m, n, k / 256,      \
+                                                                                  residual, out)
+  if (n / 32 >= 160) {
+    if (residual)
+      CLEF_DECQ(32, true);
+    else
+      CLEF_DECQ(32, false);
+  } else {
+    if (residual)
+      CLEF_DECQ(16, true);
+    else
+      CLEF_DECQ(16, false);
+  }
+#undef CLEF_DECQ
+  return hipGetLastError();
+}
+
 template <bool GU>
 hipError_t launch_expert_skinny(const uint32_t* a, int a_words, int64_t a_bytes, const float* as,
                                 const uint32_t* w, const float* ws, const uint32_t* w2, const float* ws2,
@@ -2085,6 +2195,25 @@ hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const
   if (n % 256 == 0 && m >= 1024 && tiles(256) >= 160)
     return launch_dma8_any<Dma256x256W8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
   return launch_dma8_any<Dma128x128>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+}
+
+bool project_fusable(int64_t m, int k) {
+  // one workgroup's 512 threads hold 16 values each
+  return m <= 4 && k / 256 <= (m == 1 ? 32 : m == 2 ? 16 : 8);
+}
+
+hipError_t launch_project_i4(const uint16_t* x, const uint32_t* w, const float* ws, int64_t m, int n, int k,
+                             const uint16_t* residual, uint16_t* out, hipStream_t stream) {
+  if (!project_fusable(m, k)) return hipErrorInvalidValue;
+  const int kb = k / 256;
+  if (m == 1) {
+    if (kb <= 8) return launch_decode_q<1, 8>(x, w, ws, m, n, k, residual, out, stream);
+    if (kb <= 16) return launch_decode_q<1, 16>(x, w, ws, m, n, k, residual, out, stream);
+    return launch_decode_q<1, 32>(x, w, ws, m, n, k, residual, out, stream);
+  }
+  if (m == 2 && kb > 8) return launch_decode_q<2, 16>(x, w, ws, m, n, k, residual, out, stream);
+  if (m == 2) return launch_decode_q<2, 8>(x, w, ws, m, n, k, residual, out, stream);
+  return launch_decode_q<4, 8>(x, w, ws, m, n, k, residual, out, stream);
 }
 
 hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const uint32_t* w,

@@ -1346,6 +1346,28 @@ def test_gemm_f6_gate_up_rejects():
         clef_i4.project_gate_up_f6(a, fw, fw)  # 192 columns: not whole 128-column panels
 
 
+@pytest.mark.parametrize("n,k", [(256, 256), (768, 2048), (256, 2304), (1024, 4096), (256, 4352), (5120, 1024),
+                                 (5376, 4096), (512, 8192), (5120, 8192), (256, 8448)])
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
+def test_project_quantized_few_rows_matches_oracle(m, n, k):
+    """Q1(x) and G1 in one launch (up to 4 rows, by K) and in two, 16 and 32
+    columns per workgroup, fewer groups than the workgroup holds: the oracle's
+    quantizer and G1, with and without the residual, on plain and exceptional
+    rows (NaN, infinity, zeros, one denormal)."""
+    rng = np.random.default_rng(m * 3 + n + k)
+    x = randn_bf16(rng, (m, k), std=2.0)
+    odd = exceptional_rows(k)[[0, 1, 3, 6, 7]][:m]
+    qw = clef_i4.load_quantized_weight(to_dev_bf16(randn_bf16(rng, (n, k), std=0.02)))
+    host = u32_host(qw.codes), qw.scales.cpu().numpy()
+    res = randn_bf16(rng, (m, n), std=2.0)
+    for rows in (x, odd):
+        codes, scales, _ = oracle.prepare(rows, oracle.activation_stride(k))
+        for r in (None, res):
+            want = oracle.gemm(codes, scales, *host, n, k, residual=r)
+            got = bf16_host(clef_i4.project_quantized(to_dev_bf16(rows), qw, None if r is None else to_dev_bf16(r)))
+            assert_same_bf16_nan_aware(got, want, f"project_quantized m={m} n={n} k={k} resid={r is not None}")
+
+
 # ---------------------------------------------------------------- decode-sized G1
 # Configuration 4: v_dot8_i32_i4 on the packed codes for m <= 8.
 
