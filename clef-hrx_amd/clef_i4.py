@@ -51,6 +51,8 @@ SIGNATURES = {
     "clef_i4_gemm": (ctypes.c_int, [_P, _I32, _P, _P, _P, _I64, _I32, _I32, _P, _P, _P]),
     "clef_i4_gemm_config": (ctypes.c_int, [_P, _I32, _P, _P, _P, _I64, _I32, _I32, _P, _P, _I32, _P]),
     "clef_i4_gemm_configs": (ctypes.c_int, []),
+    "clef_i4_gemm_workspace_bytes": (_SZ, [_I64, _I32, _I32]),
+    "clef_i4_gemm_ws": (ctypes.c_int, [_P, _I32, _P, _P, _P, _I64, _I32, _I32, _P, _P, _P, _SZ, _P]),
     "clef_i8_gemm": (ctypes.c_int, [_P, _I32, _P, _P, _P, _I64, _I32, _I32, _P, _P, _P]),
     "clef_i4_f6_activation": (ctypes.c_int, [_P, _I32, _I64, _I32, _P, _P]),
     "clef_i4_f6_weight": (ctypes.c_int, [_P, _I64, _I32, _P, _P]),
@@ -470,6 +472,14 @@ def gemm_configs() -> int:
     return int(lib().clef_i4_gemm_configs())
 
 
+def _scratch(like: torch.Tensor, nbytes: int) -> torch.Tensor | None:
+    """Scratch that a call does without where memory is short."""
+    try:
+        return _n.empty(like, torch.uint8, nbytes)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def project_prepared(a: Prepared, w: QuantizedWeight, residual: torch.Tensor | None = None,
                      config: int = -1, out: torch.Tensor | None = None) -> torch.Tensor:
     """Engine::project_prepared (src/quantized.rs:470-537)."""
@@ -480,6 +490,12 @@ def project_prepared(a: Prepared, w: QuantizedWeight, residual: torch.Tensor | N
     if w.bits == 8:  # h3_gemm_i8_256
         _n.launch(_n.clef_i8_gemm, a.storage, a.stride, a.scales_arg(), w.codes, w.scales, a.rows, w.rows, w.cols,
                   residual, out)
+        return out
+    ws_bytes = _n.value(_n.clef_i4_gemm_workspace_bytes, a.rows, w.rows, w.cols) if config == -1 else 0
+    ws = _scratch(a.storage, ws_bytes) if ws_bytes > 0 else None
+    if ws is not None:
+        _n.launch(_n.clef_i4_gemm_ws, a.storage, a.stride, a.scales_arg(), w.codes, w.scales, a.rows, w.rows, w.cols,
+                  residual, out, ws, ws_bytes)
         return out
     _n.launch(_n.clef_i4_gemm_config, a.storage, a.stride, a.scales_arg(), w.codes, w.scales, a.rows, w.rows, w.cols,
               residual, out, config)
@@ -648,6 +664,8 @@ def project_quantized(x: torch.Tensor, w: QuantizedWeight, residual: torch.Tenso
                       ) -> torch.Tensor:
     """Engine::project_quantized[_with_residual] (src/quantized.rs:235-303)."""
     m, k = x.shape
+    if m >= 1024 and _n.value(_n.clef_i4_gemm_workspace_bytes, m, w.rows, k) > 0:
+        return project_prepared(prepare(x), w, residual)
     out = _n.empty(x, torch.bfloat16, m, w.rows)
     ws_bytes = _n.value(_n.clef_i4_project_workspace_bytes, m, k)
     ws = _n.empty(x, torch.uint8, max(ws_bytes, 16))

@@ -283,6 +283,27 @@ int clef_i4_gemm(const uint32_t* a, int32_t k_stride, const float* a_scales, con
                              stream);
 }
 
+size_t clef_i4_gemm_workspace_bytes(int64_t m, int32_t n, int32_t k) {
+  if (check_gemm(m, n, k, k) != CLEF_OK || !clef::gemm_i4_via_f6(m, n, k)) return 0;
+  return align256((size_t)clef::f6_codes_bytes(m, k)) + (size_t)n * k * 3 / 4;
+}
+
+int clef_i4_gemm_ws(const uint32_t* a, int32_t k_stride, const float* a_scales, const uint32_t* w_tiled,
+                    const float* w_scales, int64_t m, int32_t n, int32_t k, const uint16_t* residual, uint16_t* out,
+                    void* workspace, size_t workspace_bytes, clef_stream_t stream) {
+  if (int rc = check_gemm(m, n, k, k_stride)) return rc;
+  const size_t need = clef_i4_gemm_workspace_bytes(m, n, k);
+  if (need == 0 || workspace == nullptr || workspace_bytes < need)
+    return clef_i4_gemm(a, k_stride, a_scales, w_tiled, w_scales, m, n, k, residual, out, stream);
+  if (!aligned(a, 16) || !aligned(a_scales, 4) || !aligned(w_tiled, 16) || !aligned(w_scales, 16) ||
+      !aligned(out, 16) || (residual && !aligned(residual, 16)) || !aligned(workspace, 16))
+    return fail(kAlign);
+  uint8_t* a6 = static_cast<uint8_t*>(workspace);
+  uint8_t* w6 = a6 + align256((size_t)clef::f6_codes_bytes(m, k));
+  if (int rc = hip_status(clef::launch_f6_convert(w_tiled, n, w6, a, k_stride / 8, m, a6, k, hs(stream)))) return rc;
+  return hip_status(clef::launch_gemm_f6(a6, a_scales, w6, w_scales, m, n, k, residual, out, hs(stream)));
+}
+
 int clef_i8_gemm(const uint32_t* a, int32_t k_stride, const float* a_scales, const uint32_t* w_tiled,
                  const float* w_scales, int64_t m, int32_t n, int32_t k, const uint16_t* residual,
                  uint16_t* out, clef_stream_t stream) {

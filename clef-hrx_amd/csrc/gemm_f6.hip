@@ -83,46 +83,46 @@ __device__ __forceinline__ void f6_pack32(const uint32_t (&w)[4], uint32_t (&out
   }
 }
 
-// Packed activation (k_stride words per row) -> the bf6 activation layout
-// (f6_offset); one thread per 32 codes.
-__global__ __launch_bounds__(256) void f6_rows_kernel(const uint32_t* __restrict__ a, int a_words, int64_t rows,
-                                                      int k, uint8_t* __restrict__ out) {
-  const int groups = k / 32;
-  const int64_t total = rows * groups;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = t / groups;
-    const int g = (int)(t - r * groups);
-    const uint4 in = *reinterpret_cast<const uint4*>(a + r * a_words + 4 * g);
-    const uint32_t w[4] = {in.x, in.y, in.z, in.w};
-    uint32_t o[6];
-    f6_pack32(w, o);
-    v2u* dst = reinterpret_cast<v2u*>(out + f6_offset(r, 32 * g, k));
-    dst[0] = v2u{o[0], o[1]};
-    dst[1] = v2u{o[2], o[3]};
-    dst[2] = v2u{o[4], o[5]};
+// 32 codes (four packed words) -> bytes 24 (g % 4) .. + 23 of the 96-byte row at
+// `row`, chunks stored at chunk ^ s.
+__device__ __forceinline__ void f6_store32(uint4 in, uint8_t* row, int g, int s) {
+  const uint32_t wv[4] = {in.x, in.y, in.z, in.w};
+  uint32_t o[6];
+  f6_pack32(wv, o);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    const int off = 24 * (g % 4) + 8 * p;  // logical byte offset in the row
+    *reinterpret_cast<v2u*>(row + (((off >> 4) ^ s) << 4) + (off & 15)) = v2u{o[2 * p], o[2 * p + 1]};
   }
 }
 
-// Tiled INT4 weight (the reference layout: 128-row x 256-k blocks of 32 words
-// per row) -> bf6 tiled weight (header comment); one thread per 32 codes, in
-// the order of the INT4 weight, so that a wave reads one KiB and writes two
-// runs of 768 bytes (8 rows of each 128-k block). Codes through byte-permute
-// tables: 12288 x 4096 23.5 -> 13.9 us.
-__global__ __launch_bounds__(256) void f6_tiled_kernel(const uint32_t* __restrict__ w, int64_t total,
-                                                       uint8_t* __restrict__ out) {
+// Operands re-encoded as bf6, one thread per 32 codes, a wave per 8 rows x 256
+// k (so it reads eight 128-byte row pieces, one contiguous KiB of a weight, and
+// writes two runs of 768 bytes, 8 rows of each 128-k block). The first
+// `wtotal` threads take the tiled INT4 weight (the reference layout: 128-row x
+// 256-k blocks of 32 words per row) to the bf6 tiled weight, the others the
+// packed activation (a_words per row) to the bf6 activation layout; either may
+// be absent. Codes through byte-permute tables: weight 12288 x 4096 23.5 ->
+// 13.4 us, activation 8192 x 17408 54.4 -> 43.3.
+__global__ __launch_bounds__(256) void f6_convert_kernel(const uint32_t* __restrict__ w, int64_t wtotal,
+                                                         uint8_t* __restrict__ w_out, const uint32_t* __restrict__ a,
+                                                         int a_words, int64_t rows, int kb4, int64_t total,
+                                                         uint8_t* __restrict__ a_out) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const uint4 in = reinterpret_cast<const uint4*>(w)[t];
-    const int g = (int)(t & 7), r = (int)(t >> 3) & 127;
-    const int64_t block = t >> 10;  // panel * kb4 + 256-k block: its two 128-k blocks are 2 block, 2 block + 1
-    const uint32_t wv[4] = {in.x, in.y, in.z, in.w};
-    uint32_t o[6];
-    f6_pack32(wv, o);
-    uint8_t* blk = out + (2 * block + (g >> 2)) * 12288 + r * 96;
-    const int s = (r >> 3) & 1;
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      const int off = 24 * (g % 4) + 8 * p;  // logical byte offset in the 96-byte row
-      *reinterpret_cast<v2u*>(blk + ((((off >> 4) ^ s)) << 4) + (off & 15)) = v2u{o[2 * p], o[2 * p + 1]};
+    if (t < wtotal) {  // whole waves: wtotal is a multiple of 1024
+      const int g = (int)(t & 7), r = (int)(t >> 3) & 127;
+      const int64_t block = t >> 10;  // panel * kb4 + 256-k block: its two 128-k blocks are 2 block, 2 block + 1
+      f6_store32(reinterpret_cast<const uint4*>(w)[t], w_out + (2 * block + (g >> 2)) * 12288 + r * 96, g,
+                 (r >> 3) & 1);
+    } else {
+      const int64_t u = t - wtotal;
+      const int g = (int)(u & 7), r8 = (int)(u >> 3) & 7;
+      const int64_t unit = u >> 6, rg = unit / kb4;
+      const int kt = (int)(unit - rg * kb4);
+      const int64_t row = rg * 8 + r8;
+      if (row >= rows) continue;
+      const uint4 in = *reinterpret_cast<const uint4*>(a + row * a_words + kt * 32 + 4 * g);
+      f6_store32(in, a_out + ((row >> 7) * (2 * kb4) + 2 * kt + (g >> 2)) * 12288 + (row & 127) * 96, g, 0);
     }
   }
 }
@@ -496,7 +496,32 @@ hipError_t launch_gemm_f6_impl(const RingArgs& x, hipStream_t stream) {
 
 }  // namespace
 
+// Packed activation rows (k % 128 == 0) -> bf6 activation, for widths that are
+// not whole 256-k blocks.
+__global__ __launch_bounds__(256) void f6_rows_kernel(const uint32_t* __restrict__ a, int a_words, int64_t rows,
+                                                      int k, uint8_t* __restrict__ out) {
+  const int groups = k / 32;
+  const int64_t total = rows * groups;
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = t / groups;
+    const int g = (int)(t - r * groups);
+    f6_store32(*reinterpret_cast<const uint4*>(a + r * a_words + 4 * g),
+               out + ((r >> 7) * (k / 128) + (g >> 2)) * 12288 + (r & 127) * 96, g, 0);
+  }
+}
+
+hipError_t launch_f6_convert(const uint32_t* w_tiled, int64_t n, uint8_t* w_out, const uint32_t* a, int a_words,
+                             int64_t rows, uint8_t* a_out, int k, hipStream_t stream) {
+  const int64_t wtotal = n * (k / 32);
+  const int64_t total = wtotal + (rows + 7) / 8 * 64 * (k / 256);
+  const int64_t blocks = (total + 255) / 256;
+  f6_convert_kernel<<<(unsigned)(blocks < 8192 ? blocks : 8192), 256, 0, stream>>>(w_tiled, wtotal, w_out, a, a_words,
+                                                                                  rows, k / 256, total, a_out);
+  return hipGetLastError();
+}
+
 hipError_t launch_f6_rows(const uint32_t* a, int a_words, int64_t rows, int k, uint8_t* out, hipStream_t stream) {
+  if (k % 256 == 0) return launch_f6_convert(nullptr, 0, nullptr, a, a_words, rows, out, k, stream);
   const int64_t total = rows * (k / 32);
   const int64_t blocks = (total + 255) / 256;
   f6_rows_kernel<<<(unsigned)(blocks < 8192 ? blocks : 8192), 256, 0, stream>>>(a, a_words, rows, k, out);
@@ -504,10 +529,24 @@ hipError_t launch_f6_rows(const uint32_t* a, int a_words, int64_t rows, int k, u
 }
 
 hipError_t launch_f6_tiled(const uint32_t* w_tiled, int64_t n, int k, uint8_t* out, hipStream_t stream) {
-  const int64_t total = n * (k / 32);
-  const int64_t blocks = (total + 255) / 256;
-  f6_tiled_kernel<<<(unsigned)(blocks < 8192 ? blocks : 8192), 256, 0, stream>>>(w_tiled, total, out);
-  return hipGetLastError();
+  return launch_f6_convert(w_tiled, n, out, nullptr, 0, 0, nullptr, k, stream);
+}
+
+// The bf6 GEMM is a quarter faster than the INT4 one on the same tiles (twice
+// the MFMA rate, no unpacking), and re-encoding both operands costs one pass
+// over them. Whole calls (graph replay, three weights in turn, us, INT4 / via
+// bf6): 2729 x 17408 x 5120 173 / 159, 4096 x 12288 x 4096 147 / 127, 8192 x
+// 5120 x 17408 499 / 431, 1500 x 6144 x 5120 53.1 / 47.0, 2048 x 12288 x 2048
+// 52.0 / 50.0. Few rows do not pay for the weight (1024 x 12288 x 4096 47.3 /
+// 48.8), few tiles leave CUs idle either way (1500 x 4096 x 4096, 96 tiles,
+// 31.2 / 38.0), short K is stores and launches (2729 x 12288 x 1024 45.2 / 50.4).
+bool gemm_i4_via_f6(int64_t m, int n, int k) {
+  // clef_i4_gemm_f6's limits
+  if (n % 256 != 0 || k > 32768 || n >= (1 << 22) || m > ((int64_t)1 << 29)) return false;
+  const int64_t tiles = (m + 255) / 256 * (n / 256);
+  if (tiles > kMaxTiles / 4) return false;  // tiles of 128 x 128 are indexed in 32 bits
+  if (k >= 4096) return tiles > 256 || (m >= 1500 && tiles >= 144);
+  return k >= 2048 && tiles > 320;
 }
 
 hipError_t launch_gemm_f6(const uint8_t* a, const float* as, const uint8_t* w, const float* ws, int64_t m, int n,

@@ -69,6 +69,11 @@ hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const
 // rows of k * 3/4 bytes; tiled INT4 weight -> bf6 tiled weight; the GEMM on
 // them (k % 128 == 0, n % 256 == 0).
 hipError_t launch_f6_rows(const uint32_t* a, int a_words, int64_t rows, int k, uint8_t* out, hipStream_t stream);
+// Both at once (k % 256 == 0).
+hipError_t launch_f6_convert(const uint32_t* w_tiled, int64_t n, uint8_t* w_out, const uint32_t* a, int a_words,
+                             int64_t rows, uint8_t* a_out, int k, hipStream_t stream);
+// Whether G1 on INT4 operands is faster by re-encoding both as bf6 first.
+bool gemm_i4_via_f6(int64_t m, int n, int k);
 hipError_t launch_f6_tiled(const uint32_t* w_tiled, int64_t n, int k, uint8_t* out, hipStream_t stream);
 hipError_t launch_gemm_f6(const uint8_t* a, const float* as, const uint8_t* w, const float* ws, int64_t m, int n,
                           int k, const uint16_t* residual, uint16_t* out, hipStream_t stream);

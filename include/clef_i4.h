@@ -190,6 +190,16 @@ int clef_i4_gemm(const uint32_t* a, int32_t k_stride, const float* a_scales, con
                  const float* w_scales, int64_t m, int32_t n, int32_t k, const uint16_t* residual,
                  uint16_t* out, clef_stream_t stream);
 
+/* clef_i4_gemm with scratch: for shapes of many tiles the operands are first
+ * re-encoded as bf6 in the workspace (clef_i4_f6_activation,
+ * clef_i4_f6_weight) and multiplied by clef_i4_gemm_f6, the same bits in less
+ * time. workspace_bytes gives 0 for every other shape; with less workspace
+ * than it asks for (or NULL) the call is clef_i4_gemm. */
+size_t clef_i4_gemm_workspace_bytes(int64_t m, int32_t n, int32_t k);
+int clef_i4_gemm_ws(const uint32_t* a, int32_t k_stride, const float* a_scales, const uint32_t* w_tiled,
+                    const float* w_scales, int64_t m, int32_t n, int32_t k, const uint16_t* residual, uint16_t* out,
+                    void* workspace, size_t workspace_bytes, clef_stream_t stream);
+
 /* INT8 x INT8 -> i32 dense GEMM with the same epilogue, for INT8-packed
  * activations (clef_i4_prepare with bits 8: 4 codes per word, row pitch
  * k_stride/4 words) and INT8 weights (clef_i4_pack_weight with bits 8).

@@ -1346,6 +1346,29 @@ def test_gemm_f6_gate_up_rejects():
         clef_i4.project_gate_up_f6(a, fw, fw)  # 192 columns: not whole 128-column panels
 
 
+@pytest.mark.parametrize("m,n,k", [(1537, 6144, 4096), (1500, 6144, 4352), (1030, 16640, 4096), (2049, 9216, 2048)])
+@pytest.mark.parametrize("resid", [False, True])
+def test_gemm_through_bf6_matches_direct(m, n, k, resid):
+    """Shapes that project_prepared re-encodes as bf6: all rows bit-equal to
+    the INT4-operand kernel (also what a call without enough workspace runs),
+    sampled rows to the oracle; project_quantized gives the same."""
+    assert clef_i4._n.value(clef_i4._n.clef_i4_gemm_workspace_bytes, m, n, k) > 0
+    x, (q,), rows, a_codes, a_scales, host = _f6_path_operands(m, n, k, 1)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    res = torch.randn((m, n), generator=g, device="cuda", dtype=torch.bfloat16) if resid else None
+    a = clef_i4.prepare(x)
+    want = bf16_host(clef_i4.project_prepared(a, q, residual=res, config=2))
+    assert_same_bf16_nan_aware(bf16_host(clef_i4.project_prepared(a, q, residual=res)), want, "through bf6")
+    assert_same_bf16_nan_aware(bf16_host(clef_i4.project_quantized(x, q, res)), want, "project_quantized")
+    out = torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+    ws = torch.empty(4096, dtype=torch.uint8, device="cuda")
+    clef_i4._n.launch(clef_i4._n.clef_i4_gemm_ws, a.storage, a.stride, a.scales, q.codes, q.scales, m, n, k, res, out,
+                      ws, 4096)
+    assert_same_bf16_nan_aware(bf16_host(out), want, "too little workspace")
+    sub = oracle.gemm(a_codes, a_scales, *host[0], n, k, residual=bf16_host(res)[rows] if resid else None)
+    assert_same_bf16_nan_aware(want[rows], sub, "sampled rows vs oracle")
+
+
 @pytest.mark.parametrize("n,k", [(256, 256), (768, 2048), (256, 2304), (1024, 4096), (256, 4352), (5120, 1024),
                                  (5376, 4096), (512, 8192), (5120, 8192), (256, 8448)])
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
