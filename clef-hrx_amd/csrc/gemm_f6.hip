@@ -139,7 +139,7 @@ struct F6Op {
   // read (mf 1) at the lane's swizzled chunk offsets.
   struct Reader {
     int c0, c1, c2;  // byte offsets of logical chunks 3h, 3h+1, 3h+2 in the row
-    __device__ __forceinline__ Reader() {
+    __device__ __forceinline__ explicit Reader(int = 0) {
       const int lane = threadIdx.x & 63;
       const int h = lane >> 5, s = ((lane & 31) >> 3) & 1;
       c0 = ((3 * h) ^ s) << 4;

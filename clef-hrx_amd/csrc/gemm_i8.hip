@@ -14,16 +14,17 @@ struct I8Op {
   static constexpr int kStep = 64;
   [[maybe_unused]] static constexpr float kDotPerStep = 16384.0f * kStep;  // |dot| per k-step, codes of magnitude 128
 
-  // Row r's logical 16-byte chunk c (of four) is stored at c ^ ((r >> 2) & 3):
-  // 16 consecutive rows of one chunk cover the 64 banks once. Round s takes
-  // chunk 2 s + h.
+  // A stage row is 128 bytes, both groups' k-steps (one row of a weight block);
+  // row r's logical 16-byte chunk c is stored at c ^ ((r >> 1) & 7): 16
+  // consecutive rows of one chunk cover the 64 banks once. Round s of group kg
+  // takes chunk 4 kg + 2 s + h.
   struct Reader {
     int c[2];
-    __device__ __forceinline__ Reader() {
+    __device__ __forceinline__ explicit Reader(int kg) {
       const int lane = threadIdx.x & 63;
-      const int h = lane >> 5, g = ((lane & 31) >> 2) & 3;
-      c[0] = (h ^ g) << 4;
-      c[1] = ((2 + h) ^ g) << 4;
+      const int h = lane >> 5, g = ((lane & 31) >> 1) & 7;
+      c[0] = ((4 * kg + h) ^ g) << 4;
+      c[1] = ((4 * kg + 2 + h) ^ g) << 4;
     }
     __device__ __forceinline__ v4i operand(const char* row, int s) const {
       return *reinterpret_cast<const v4i*>(row + c[s]);
@@ -32,10 +33,13 @@ struct I8Op {
 
   __device__ __forceinline__ static v16i mfma(v4i w, v4i a, v16i c) { return mfma32_i8(w, a, c); }
 
-  // DMA instruction q moves 16 rows of one k-step, lane -> row 16 (q % ..) +
-  // lane / 4, stored chunk lane % 4. Activation rows are a_row_bytes apart;
-  // weight rows are the 128 bytes of a tiled block, the k-step one half of
-  // them; the stage's two k-steps (KG 2) are the two halves.
+  // DMA instruction q moves 8 whole 128-byte rows, lane -> row 8 q + lane / 8,
+  // stored chunk lane % 8. Activation rows are a_row_bytes apart, weight rows
+  // those of a tiled block. Whole lines per instruction: with each group's 64
+  // bytes in rows of their own, 16 half lines an instruction, every line was
+  // requested twice (m x n x k, graph replay, three runs of each in turn:
+  // 235 x 12288 x 4096 21.8 -> 20.5 us, 620 x 4096 x 12288 49.5 -> 46.5,
+  // 620 x 5120 x 6144 29.8 -> 27.8, 1000 x 12288 x 4096 69.2 -> 67.5).
   template <class T>
   __device__ __forceinline__ static void offsets(int, int a_row_bytes, int (&voff)[T::SLOTS]) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -43,16 +47,15 @@ struct I8Op {
     for (int slot = 0; slot < T::SLOTS; ++slot) {
       const int q = wave + T::NW * slot;
       const bool is_a = T::NW * slot < T::A_QS;
-      const int per = (is_a ? T::BM : T::BN) / 16, i = is_a ? q : q - T::A_QS;
-      const int row = 16 * (i % per) + (lane >> 2), g = i / per;
-      voff[slot] = (is_a ? row * a_row_bytes : (row & 127) * 128) + 64 * g + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+      const int row = 8 * (is_a ? q : q - T::A_QS) + (lane >> 3);
+      voff[slot] = (is_a ? row * a_row_bytes : row * 128) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
     }
   }
 
   template <class T, bool GU>
   __device__ __forceinline__ static void issue_slot(char* stage, const RingTiles& x, const int (&voff)[T::SLOTS],
                                                     int, int kt, int slot) {
-    static_assert(!GU && T::A_QS % T::NW == 0 && T::QS % T::NW == 0 && T::KG == 2 && T::BN == 128, "whole slots");
+    static_assert(!GU && T::A_QS % T::NW == 0 && T::QS % T::NW == 0 && T::KG == 2 && T::SPLIT && T::BN == 128, "whole slots");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = wave + T::NW * slot;
     const lds_ptr_t dst = (lds_ptr_t)(stage + q * 1024);
@@ -82,8 +85,8 @@ struct I8Op {
   }
 };
 
-// 128 x 128 tiles, 32 KiB stages: the two halves of a 128-byte weight block row
-using I8Tile128 = RingTile<64, 64, 64, 2, 2, 2, 4>;
+// 128 x 128 tiles, 32 KiB stages of 128-byte rows (the two groups split each row)
+using I8Tile128 = RingTile<128, 64, 64, 2, 2, 2, 4, true>;
 
 }  // namespace
 

@@ -23,7 +23,9 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 // Tile shape: KG groups of WAVES_M x WAVES_N waves, each wave
 // WM rows x WN weight rows; a stage holds KG k-steps and group g contracts
 // the g-th of them.
-template <int ROW_, int WM_, int WN_, int WAVES_M_, int WAVES_N_, int KG_, int NST_>
+// SPLIT: a row of a stage holds the groups' k-steps side by side (ROW bytes in
+// all); otherwise each group has its own rows.
+template <int ROW_, int WM_, int WN_, int WAVES_M_, int WAVES_N_, int KG_, int NST_, bool SPLIT_ = false>
 struct RingTile {
   static constexpr int WM = WM_, WN = WN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, KG = KG_;
   static constexpr int NST = NST_;                              // LDS stages
@@ -34,7 +36,8 @@ struct RingTile {
   static constexpr int EM = TM / KG;                            // row fragments a wave takes through the epilogue
   static constexpr int ROW = ROW_;                              // bytes per row per k-step
   static constexpr int A_STEP = BM * ROW, B_STEP = BN * ROW;    // bytes of one k-step
-  static constexpr int A_BYTES = KG * A_STEP, B_BYTES = KG * B_STEP;
+  static constexpr bool SPLIT = SPLIT_;
+  static constexpr int A_BYTES = (SPLIT ? 1 : KG) * A_STEP, B_BYTES = (SPLIT ? 1 : KG) * B_STEP;
   static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
   static constexpr int A_QS = A_BYTES / 1024, QS = STAGE_BYTES / 1024;  // DMA instructions per stage
   static constexpr int SLOTS = (QS + NW - 1) / NW;              // and per wave, at most
@@ -455,9 +458,9 @@ __global__ __launch_bounds__(T::THREADS) void gemm_ring_kernel(
   const int ksteps = kb / T::KG;  // k-steps (of KG) per tile
   int voff[T::SLOTS];
   Op::template offsets<T>(kb, a_row_bytes, voff);
-  const typename Op::Reader o;
-  const int a_base = kg * T::A_STEP + (wm * T::WM + lr) * T::ROW;
-  const int b_base = T::A_BYTES + kg * T::B_STEP + ((GU ? wn * (T::WN / 2) : wn * T::WN) + lr) * T::ROW;
+  const typename Op::Reader o(kg);
+  const int a_base = (T::SPLIT ? 0 : kg * T::A_STEP) + (wm * T::WM + lr) * T::ROW;
+  const int b_base = T::A_BYTES + (T::SPLIT ? 0 : kg * T::B_STEP) + ((GU ? wn * (T::WN / 2) : wn * T::WN) + lr) * T::ROW;
   const int b_step = (GU ? T::BN / 2 : 32) * T::ROW;  // weight fragment 1: the up rows (GU)
   auto st = [&](int i) { return lds + i * T::STAGE_BYTES; };
   char* sc = lds + NST * T::STAGE_BYTES + wave * T::SCALE_WAVE;
