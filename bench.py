@@ -34,7 +34,7 @@ M=4096 on one MI355X.
                experts take most rows, eight none).
   moe_small_t  the MoE layer at 1, 16 and 256 tokens: GPU time per layer by
                graph replay (weights from HBM, and cache-resident), and the
-               HBM rate of the skinny expert GEMMs over the routed experts'
+               HBM rate of the expert GEMMs over the routed experts'
                codes.
   roofline     the GEMM kernel against the peak of the MFMA it runs on (fp6
                dense, 10.1 POP/s); pct_int8_peak is the metric's own ratio.
@@ -428,7 +428,7 @@ def moe_small_leg(args):
     """The Omni MoE layer at decode-sized token counts (1, 16 and 256 tokens;
     hidden 2048, 128 experts, top-8, intermediate 768): GPU time per layer by
     HIP graph replay, and the HBM rate of the two expert GEMMs alone (the
-    skinny 32-slot kernels; each call also runs its small tile-schedule
+    32-slot kernels; each call also runs its small tile-schedule
     kernel), over the codes and scales of the experts the tokens route to.
     `us` and the GEMM figures cycle through 14 copies of the layer's packed
     weights, so each call reads its experts from HBM as a multi-layer decode

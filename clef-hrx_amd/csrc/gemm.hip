@@ -2183,7 +2183,7 @@ hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const
   // 10.3; M100 N12288 K12288 51.6 against 68.6 for the 128 x 128 ring; M400
   // N4096 K4096 18.5 against 20.5, M620, three rounds, 26.2 against 21.2).
   // Up to one round of 128 x 128 tiles: the ring kernel (M235 N12288 K4096
-  // 21.2 against 27.6 for the two-stage tiles, M1024 N4096 K12288 57.3
+  // 20.5 against 27.6 for the two-stage tiles, M1024 N4096 K12288 57.3
   // against 76.2; two rounds M400 N12288 K4096 38.6 against 33.1).
   // Else 256 x 256 tiles once there are 160 of them (M2048 N5120 K6144 75.7
   // against 87.9 for 128 x 128; M2048 N4096 K4096, 128 tiles, 53.0 against
@@ -2226,11 +2226,6 @@ hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const
     // each next tile's first k-steps under the current tile's last one
     // (M4096 N12288 K4096: 154 us against 160 us with one workgroup per
     // tile); 128x128 tiles otherwise.
-    // Few rows: the weight stream dominates and 128x128 tiles give too few
-    // workgroups, so the K-split skinny kernel (GPU time, graph replay:
-    // M1 N4096 K4096 5.1 us against 17.4; M64 N12288 K4096 13.0 against
-    // 17.8; M512 N2048 K2048 7.5 against 11.3; M128 N12288 K4096 29.1
-    // against 18.3, where 96 tiles of 128x128 already cover most CUs).
     // At most 4 rows, or 8 where 32 x 32 split-K tiles would leave CUs idle:
     // the VALU dot-product kernel (graph replay, three weights in turn: M4
     // N12288 K4096 6.2 us against 7.6 for the split-K tiles, M8 8.2 against
