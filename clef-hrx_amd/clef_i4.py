@@ -664,11 +664,14 @@ def project_quantized(x: torch.Tensor, w: QuantizedWeight, residual: torch.Tenso
                       ) -> torch.Tensor:
     """Engine::project_quantized[_with_residual] (src/quantized.rs:235-303)."""
     m, k = x.shape
-    if m >= 1024 and _n.value(_n.clef_i4_gemm_workspace_bytes, m, w.rows, k) > 0:
-        return project_prepared(prepare(x), w, residual)
     out = _n.empty(x, torch.bfloat16, m, w.rows)
     ws_bytes = _n.value(_n.clef_i4_project_workspace_bytes, m, k)
-    ws = _n.empty(x, torch.uint8, max(ws_bytes, 16))
+    more = _n.value(_n.clef_i4_gemm_workspace_bytes, m, w.rows, k)
+    ws = _scratch(x, ws_bytes + more) if more > 0 else None
+    if ws is None:
+        ws = _n.empty(x, torch.uint8, max(ws_bytes, 16))
+    else:
+        ws_bytes += more
     _n.launch(_n.clef_i4_project, x, m, k, w.codes, w.scales, w.rows, residual, out, ws, ws_bytes)
     return out
 

@@ -420,8 +420,9 @@ int clef_i4_project(const uint16_t* x, int64_t m, int32_t k, const uint32_t* w_t
   uint32_t* packed = static_cast<uint32_t*>(workspace);
   if (int rc = hip_status(clef::launch_prepare(x, m, k, stride, 4, packed, hs(stream)))) return rc;
   const float* a_scales = reinterpret_cast<const float*>(packed + m * (stride / 8));
-  return hip_status(clef::launch_gemm_i4(packed, stride / 8, a_scales, w_tiled, w_scales, m, n, k,
-                                         residual, out, -1, hs(stream)));
+  const size_t used = clef_i4_project_workspace_bytes(m, k);
+  return clef_i4_gemm_ws(packed, stride, a_scales, w_tiled, w_scales, m, n, k, residual, out,
+                         static_cast<char*>(workspace) + used, workspace_bytes - used, stream);
 }
 
 int clef_moe_route(const void* logits, int32_t logits_dtype, int64_t tokens, int32_t experts,

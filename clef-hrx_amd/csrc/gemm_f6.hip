@@ -534,19 +534,28 @@ hipError_t launch_f6_tiled(const uint32_t* w_tiled, int64_t n, int k, uint8_t* o
 
 // The bf6 GEMM is a quarter faster than the INT4 one on the same tiles (twice
 // the MFMA rate, no unpacking), and re-encoding both operands costs one pass
-// over them. Whole calls (graph replay, three weights in turn, us, INT4 / via
-// bf6): 2729 x 17408 x 5120 173 / 159, 4096 x 12288 x 4096 147 / 127, 8192 x
-// 5120 x 17408 499 / 431, 1500 x 6144 x 5120 53.1 / 47.0, 2048 x 12288 x 2048
-// 52.0 / 50.0. Few rows do not pay for the weight (1024 x 12288 x 4096 47.3 /
-// 48.8), few tiles leave CUs idle either way (1500 x 4096 x 4096, 96 tiles,
-// 31.2 / 38.0), short K is stores and launches (2729 x 12288 x 1024 45.2 / 50.4).
+// over them. Per 1024 k a round of 256 x 256 tiles (one per CU) saves about
+// 3 us, and the pass takes about 0.32 us per 1024 rows of either operand: it
+// pays while the rounds exceed (m + n) / 9500, at K below 4096, where a round's
+// start and stores weigh more, (m + n) / 7500. Whole calls (graph replay, three
+// weights in turn, m x n x k, us, INT4 / via bf6): 1024 x 17408 x 5120 105 /
+// 94, 2729: 171 / 158; 33024 x 4096 at 1280 rows 137 / 140, at 1400 172 / 169;
+// 65536 x 6144 at 1536 433 / 456, at 2729 762 / 711; 98304 x 2048 at 2048 330 /
+// 344, at 2729 456 / 443; 128256 x 4096 at 1536 574 / 599, at one row 46 / 256.
+// One round: 1500 x 6144 x 5120 53.1 / 47.0; fewer tiles leave CUs idle either
+// way (1500 x 4096 x 4096, 96 tiles, 31.2 / 38.0). Below 1024 rows the INT4
+// GEMM runs smaller tiles, whose last round is fuller (769 x 17408 x 5120 71 /
+// 86). Below K 2048 a call is stores and launches (2729 x 12288 x 1024 45.2 /
+// 50.4).
 bool gemm_i4_via_f6(int64_t m, int n, int k) {
   // clef_i4_gemm_f6's limits
   if (n % 256 != 0 || k > 32768 || n >= (1 << 22) || m > ((int64_t)1 << 29)) return false;
   const int64_t tiles = (m + 255) / 256 * (n / 256);
   if (tiles > kMaxTiles / 4) return false;  // tiles of 128 x 128 are indexed in 32 bits
-  if (k >= 4096) return tiles > 256 || (m >= 1500 && tiles >= 144);
-  return k >= 2048 && tiles > 320;
+  if (m < 1024 || k < 2048) return false;
+  const int64_t rounds = (tiles + 255) / 256;
+  if (k < 4096) return tiles > 320 && 7500 * rounds > m + n;
+  return (rounds > 1 || (m >= 1500 && tiles >= 144)) && 9500 * rounds > m + n;
 }
 
 hipError_t launch_gemm_f6(const uint8_t* a, const float* as, const uint8_t* w, const float* ws, int64_t m, int n,

@@ -282,7 +282,8 @@ int clef_i4_gemm_f6_gate_up(const uint8_t* a_f6, const float* a_scales, const ui
                             const float* gate_scales, const uint8_t* up_f6, const float* up_scales, int64_t m,
                             int32_t n, int32_t k, uint16_t* h, clef_stream_t stream);
 
-/* Bytes of scratch clef_i4_project needs (the packed activation). */
+/* Bytes of scratch clef_i4_project needs (the packed activation). With
+ * clef_i4_gemm_workspace_bytes(m, n, k) more, the GEMM is clef_i4_gemm_ws's. */
 size_t clef_i4_project_workspace_bytes(int64_t m, int32_t k);
 
 /* Quantize x [m][k] with the weight's stride (clef_i4_activation_stride(k,

@@ -354,6 +354,17 @@ def test_gemm_f6_bounds_k_to_quantizer_width(k, ok):
     assert msg == ("device pointer is NULL or not 16-byte aligned" if ok else "unsupported integer projection shape")
 
 
+@pytest.mark.parametrize("n,k", [(66048, 4096), (98304, 2048), (128256, 4096), (152064, 5120), (4194048, 4096)])
+def test_gemm_workspace_is_for_many_rows(n, k):
+    """Re-encoding a weight costs a pass over it, whatever the rows: a
+    vocabulary-sized projection of few rows asks for no scratch, so nothing
+    re-encodes it; many rows against the same k do."""
+    size = clef_i4.lib().clef_i4_gemm_workspace_bytes
+    for m in (1, 4, 8, 64, 256, 300, 512, 769, 1023):
+        assert size(m, n, k) == 0, (m, n, k)
+    assert size(4096, 12288, k) >= 4096 * k * 3 // 4 + 12288 * k * 3 // 4
+
+
 @pytest.mark.parametrize("rows,width", [(1, 256), (127, 768), (128, 4096), (129, 4096), (4096, 12288)])
 def test_f6_prepared_bytes_pad_rows_to_whole_blocks(rows, width):
     """A bf6-prepared activation holds its codes in 128-row blocks (the last
