@@ -2179,9 +2179,11 @@ hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const
   // At most 4 rows: the dot-product kernel (v_dot4_i32_i8; M4 N4096 K4096 5.8
   // against 6.0 for the split-K tiles, M8 7.0 against 6.0, M8 N12288 K4096
   // 13.2 against 10.2).
-  // Up to two rounds of 64 x 64 tiles: the split-K tiles (M16 N12288 K4096
-  // 10.3; M100 N12288 K12288 51.6 against 68.6 for the 128 x 128 ring; M400
-  // N4096 K4096 18.5 against 20.5, M620, three rounds, 26.2 against 21.2).
+  // Up to 32 rows, and up to two rounds of 64 x 64 tiles: the split-K tiles
+  // (M16 N12288 K4096 10.3; M100 N12288 K12288 51.6 against 68.6 for the 128 x
+  // 128 ring; M400 N4096 K4096 18.5 against 20.5, M620, three rounds, 26.2
+  // against 21.2; M8 N33024 K4096 33.2 against 41.3 for 128 x 128 tiles, mostly
+  // padding there, and 38.6 for the dot-product kernel).
   // Up to one round of 128 x 128 tiles: the ring kernel (M235 N12288 K4096
   // 20.5 against 27.6 for the two-stage tiles, M1024 N4096 K12288 57.3
   // against 76.2; two rounds M400 N12288 K4096 38.6 against 33.1).
@@ -2190,7 +2192,7 @@ hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const
   // 39.7), 128 x 128 below that.
   auto tiles = [&](int b) { return (m + b - 1) / b * (n / b); };
   if (m <= 4) return launch_decode<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  if (tiles(64) <= 512) return launch_ksplit<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if (m <= 32 || tiles(64) <= 512) return launch_ksplit<true>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
   if (tiles(128) <= 256) return launch_gemm_i8_ring(a, a_words, as, w, ws, m, n, k, residual, out, stream);
   if (n % 256 == 0 && m >= 1024 && tiles(256) >= 160)
     return launch_dma8_any<Dma256x256W8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
@@ -2230,6 +2232,9 @@ hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const
     // the VALU dot-product kernel (graph replay, three weights in turn: M4
     // N12288 K4096 6.2 us against 7.6 for the split-K tiles, M8 8.2 against
     // 7.1, M8 N5120 K17408 14.5 against 10.9; M8 N4096 K12288 7.9 against 8.7).
+    // Up to 32 rows: the split-K tiles, however wide N (M8 N33024 K4096 21.7
+    // against 29.4 for 128 x 128 tiles, mostly padding there, and 22.4 for the
+    // dot-product kernel; M32 N128256 K4096 62.6 against 63.4).
     // Up to two rounds of 64 x 64 tiles, or three at K >= 8192: the split-K
     // tiles (M400 N4096 K4096 14.2 us against 18.9 for 128 x 128 tiles, M620
     // 20.1 against 19.0, M800 25.5 against 19.6; M128 N12288 K4096 14.9
@@ -2239,7 +2244,7 @@ hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const
     const int64_t tiles64 = (m + 63) / 64 * (n / 64);
     if (m <= 4 || (m <= 8 && n / 32 < 160))
       config = kGemmDecode;
-    else if (tiles64 <= 512 || (tiles64 <= 768 && k >= 8192))
+    else if (m <= 32 || tiles64 <= 512 || (tiles64 <= 768 && k >= 8192))
       config = kGemmKsplit;
     else
       config = (n % 256 == 0 && m >= 1024 && tiles256 >= 192) ? kGemmPersist256 : kGemmTile128;

@@ -64,7 +64,8 @@ def test_i8_gemm_residual_matches_oracle(m):
     (4, 256, 256, True), (5, 256, 256, False), (33, 1024, 1280, True), (64, 2048, 768, False),
     (100, 4096, 512, True), (20, 12288, 512, False), (250, 4096, 2304, False), (130, 7168, 768, True),
     (300, 8192, 256, False), (300, 8192, 512, True), (257, 8192, 768, False), (385, 6144, 1280, True),
-    (1000, 3072, 512, False), (1030, 4352, 512, True), (2100, 5120, 512, False)])
+    (1000, 3072, 512, False), (1030, 4352, 512, True), (2100, 5120, 512, False),
+    (8, 33024, 256, True), (32, 33024, 256, False), (33, 33024, 256, False)])  # wide N: 32 x 64, then 128 x 128
 def test_i8_gemm_every_path(m, n, k, resid):
     """Sampled rows (block edges, a NaN row, an infinite value, the last row)
     against the oracle; two launches agree on every row."""

@@ -1450,6 +1450,9 @@ def test_gemm_decode_extreme_codes_and_scales(m):
     (20, 12288, 2304),    # 32x64 tiles (m <= 32), 9 k-steps
     (40, 1024, 12544),    # 32x32 tiles, two stages per wave, 49 k-steps
     (9, 128, 256),        # one k-step, one tile column
+    (8, 33024, 256),      # wide N: 32x64 tiles up to 32 rows, 128x128 ones above (the automatic choice)
+    (32, 33024, 256),
+    (33, 33024, 256),
     (300, 384, 1024),
 ])
 def test_gemm_ksplit_matches_oracle(m, n, k):
