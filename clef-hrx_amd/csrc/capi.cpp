@@ -415,7 +415,7 @@ int clef_i4_project(const uint16_t* x, int64_t m, int32_t k, const uint32_t* w_t
   if (workspace_bytes < clef_i4_project_workspace_bytes(m, k)) return fail(kWorkspace);
   // a few rows in one launch, unless the output overlaps the input that every
   // workgroup of that launch reads
-  if (clef::project_fusable(m, k) && !overlap(x, (size_t)m * k * 2, out, (size_t)m * n * 2))
+  if (clef::project_fusable(m, n, k) && !overlap(x, (size_t)m * k * 2, out, (size_t)m * n * 2))
     return hip_status(clef::launch_project_i4(x, w_tiled, w_scales, m, n, k, residual, out, hs(stream)));
   uint32_t* packed = static_cast<uint32_t*>(workspace);
   if (int rc = hip_status(clef::launch_prepare(x, m, k, stride, 4, packed, hs(stream)))) return rc;

@@ -2199,14 +2199,24 @@ hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const
   return launch_dma8_any<Dma128x128>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
 }
 
-bool project_fusable(int64_t m, int k) {
+bool project_fusable(int64_t m, int n, int k) {
   // one workgroup's 512 threads hold 16 values each
-  return m <= 4 && k / 256 <= (m == 1 ? 32 : m == 2 ? 16 : 8);
+  if (m > 4 || k / 256 > (m == 1 ? 32 : m == 2 ? 16 : 8)) return false;
+  // Every workgroup quantizes the rows, so wide outputs repeat it more often
+  // than a launch costs; the sooner, the more rows and the shorter the weight
+  // rows that hide it. In one launch / in two (graph replay, three weights in
+  // turn, us): 4 x 12288 x 2048 8.9 / 8.9, 4 x 17408 x 2048 10.3 / 9.7, 4 x
+  // 33024 x 2048 14.1 / 11.7; 2 x 32768 x 1024 8.2 / 9.3, 2 x 98304 x 1024
+  // 15.4 / 14.0, 2 x 98304 x 2048 20.3 / 21.4; 1 x 98304 x 512 11.7 / 12.0, 1 x
+  // 152064 x 512 16.3 / 14.5, 1 x 152064 x 2048 30.6 / 30.8.
+  if (m == 1) return n <= 98304 || k >= 1536;
+  if (m == 2) return n <= 32768 || k >= 2048;
+  return n <= 12288;
 }
 
 hipError_t launch_project_i4(const uint16_t* x, const uint32_t* w, const float* ws, int64_t m, int n, int k,
                              const uint16_t* residual, uint16_t* out, hipStream_t stream) {
-  if (!project_fusable(m, k)) return hipErrorInvalidValue;
+  if (!project_fusable(m, n, k)) return hipErrorInvalidValue;
   const int kb = k / 256;
   if (m == 1) {
     if (kb <= 8) return launch_decode_q<1, 8>(x, w, ws, m, n, k, residual, out, stream);

@@ -1370,10 +1370,11 @@ def test_gemm_through_bf6_matches_direct(m, n, k, resid):
 
 
 @pytest.mark.parametrize("n,k", [(256, 256), (768, 2048), (256, 2304), (1024, 4096), (256, 4352), (5120, 1024),
-                                 (5376, 4096), (512, 8192), (5120, 8192), (256, 8448)])
+                                 (5376, 4096), (512, 8192), (5120, 8192), (256, 8448), (12544, 256), (33024, 256),
+                                 (98560, 256)])
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
 def test_project_quantized_few_rows_matches_oracle(m, n, k):
-    """Q1(x) and G1 in one launch (up to 4 rows, by K) and in two, 16 and 32
+    """Q1(x) and G1 in one launch (up to 4 rows, by K and N) and in two, 16 and 32
     columns per workgroup, fewer groups than the workgroup holds: the oracle's
     quantizer and G1, with and without the residual, on plain and exceptional
     rows (NaN, infinity, zeros, one denormal)."""
