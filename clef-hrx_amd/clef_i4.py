@@ -127,7 +127,7 @@ def _check(rc: int) -> None:
 
 class _Native:
     """The call module (csrc/host_call.cpp: launch, value, pointer, empty) and
-    the address of every entry point, as attributes; filled on first use."""
+    its handle of every entry point, as attributes; filled on first use."""
 
     def __getattr__(self, name):
         handle = lib()
@@ -138,7 +138,9 @@ class _Native:
         if host.build_id != built:
             raise ImportError(f"{HOST_PATH} was built from other sources (module {host.build_id}, library {built})")
         host.set_check(_check)
-        found = {entry: ctypes.cast(getattr(handle, entry), ctypes.c_void_p).value for entry in SIGNATURES}
+        found = {entry: host.entry(ctypes.cast(getattr(handle, entry), ctypes.c_void_p).value,
+                                   "".join("p" if a is _P else "i" for a in args))
+                 for entry, (_, args) in SIGNATURES.items()}
         found.update(launch=host.launch, value=host.value, pointer=host.pointer, empty=host.empty)
         if name not in found:
             raise AttributeError(name)

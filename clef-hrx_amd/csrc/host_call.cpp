@@ -1,12 +1,15 @@
-// Calls from the Python binding into the C ABI: an extension module of four
-// functions that do in C++ what the binding did per call in Python (argument
+// Calls from the Python binding into the C ABI: an extension module whose
+// functions do in C++ what the binding did per call in Python (argument
 // conversion with the device and contiguity checks, the current stream, output
 // allocation, the status check). A small projection is two launches of about
 // 3 us each; the Python side of it took longer than the GPU.
 //
-//   launch(entry, *args): entry(args.., current stream); a tensor argument is
-//     its device pointer, None is NULL, integers are themselves. A nonzero
-//     status goes to the function given to set_check, which raises.
+//   entry(address, kinds): a handle for launch and value; kinds has one
+//     letter per parameter, 'p' pointer or 'i' integer.
+//   launch(entry, *args): entry(args.., current stream). A pointer argument is
+//     a tensor (its device pointer), None (NULL) or an int address; an integer
+//     is anything with __index__, as through ctypes. A nonzero status goes to
+//     the function given to set_check, which raises.
 //   value(entry, *args): entry(args..) as int64 (size functions).
 //   pointer(tensor): its device pointer, checked as an argument is.
 //   empty(like, dtype, *sizes): torch.empty on like's device.
@@ -21,6 +24,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
+#include <deque>
 #include <utility>
 
 #include "build_id.inc"  // CLEF_BUILD_ID, generated by the Makefile
@@ -28,6 +32,13 @@
 namespace {
 
 constexpr int kMaxArgs = 24;
+
+struct Entry {
+  void* f;
+  uint32_t pointers;  // bit i: parameter i is a pointer
+  int args;
+};
+std::deque<Entry> g_entries;  // handles are addresses of its elements; kept for the process
 
 PyObject* g_check = nullptr;       // called with a nonzero status
 PyObject* g_device = nullptr;      // torch._C._cuda_getDevice
@@ -58,53 +69,83 @@ bool tensor_pointer(PyObject* o, int64_t& out) {
   return true;
 }
 
-bool convert(PyObject* o, int64_t& out) {
-  if (o == Py_None) {
-    out = 0;
-    return true;
-  }
+bool convert(PyObject* o, bool pointer, int64_t& out) {
   if (PyLong_Check(o)) {
     // device addresses and sizes below 2^64
     out = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(o));
     return !PyErr_Occurred();
   }
-  if (THPVariable_Check(o)) return tensor_pointer(o, out);
+  if (pointer && o == Py_None) {
+    out = 0;
+    return true;
+  }
+  if (pointer && THPVariable_Check(o)) return tensor_pointer(o, out);
+  if (!pointer && PyIndex_Check(o)) {
+    PyObject* i = PyNumber_Index(o);
+    if (i == nullptr) return false;
+    out = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(i));
+    Py_DECREF(i);
+    return !PyErr_Occurred();
+  }
   PyErr_Format(PyExc_TypeError, "unsupported argument type %s", Py_TYPE(o)->tp_name);
   return false;
 }
 
-bool arguments(PyObject* const* args, Py_ssize_t n, void*& entry, int64_t* v) {
-  if (n < 1 || n > kMaxArgs) {
-    PyErr_SetString(PyExc_TypeError, "entry address and at most 23 arguments expected");
-    return false;
-  }
-  entry = PyLong_AsVoidPtr(args[0]);
+// The handle args[0] and the arguments behind it, `missing` fewer than the
+// entry has.
+bool arguments(PyObject* const* args, Py_ssize_t n, int missing, const Entry*& entry, int64_t* v) {
+  entry = n < 1 ? nullptr : static_cast<const Entry*>(PyLong_AsVoidPtr(args[0]));
   if (entry == nullptr) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "no entry");
     return false;
   }
+  if (n - 1 != entry->args - missing) {
+    PyErr_Format(PyExc_TypeError, "entry takes %d arguments (%zd given)", entry->args - missing, n - 1);
+    return false;
+  }
   for (Py_ssize_t i = 1; i < n; ++i)
-    if (!convert(args[i], v[i - 1])) return false;
+    if (!convert(args[i], (entry->pointers >> (i - 1)) & 1, v[i - 1])) return false;
   return true;
+}
+
+PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 2) {
+    PyErr_SetString(PyExc_TypeError, "entry(address, kinds) expected");
+    return nullptr;
+  }
+  Entry e{PyLong_AsVoidPtr(args[0]), 0, 0};
+  Py_ssize_t count = 0;
+  const char* kinds = PyErr_Occurred() ? nullptr : PyUnicode_AsUTF8AndSize(args[1], &count);
+  if (kinds == nullptr) return nullptr;
+  if (e.f == nullptr || count > kMaxArgs) {
+    PyErr_SetString(PyExc_ValueError, "no entry, or more than 24 parameters");
+    return nullptr;
+  }
+  e.args = static_cast<int>(count);
+  for (int i = 0; i < e.args; ++i) e.pointers |= static_cast<uint32_t>(kinds[i] == 'p') << i;
+  g_entries.push_back(e);
+  return PyLong_FromVoidPtr(&g_entries.back());
+  END_HANDLE_TH_ERRORS
 }
 
 PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  void* entry;
+  const Entry* entry;
   int64_t v[kMaxArgs];
-  if (!arguments(args, n, entry, v)) return nullptr;
+  if (!arguments(args, n, 1, entry, v)) return nullptr;
   PyObject* device = PyObject_CallNoArgs(g_device);
   if (device == nullptr) return nullptr;
   PyObject* stream = PyObject_CallOneArg(g_raw_stream, device);
   Py_DECREF(device);
   if (stream == nullptr) return nullptr;
-  const bool ok = convert(stream, v[n - 1]);
+  const bool ok = convert(stream, true, v[n - 1]);
   Py_DECREF(stream);
   if (!ok) return nullptr;
   const Invoker call = pick(static_cast<size_t>(n), std::make_index_sequence<kMaxArgs + 1>{});
   int32_t rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = static_cast<int32_t>(call(entry, v));
+  rc = static_cast<int32_t>(call(entry->f, v));
   Py_END_ALLOW_THREADS
   if (rc != 0) {
     PyObject* r = PyObject_CallFunction(g_check, "i", rc);
@@ -117,10 +158,10 @@ PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 PyObject* value(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  void* entry;
+  const Entry* entry;
   int64_t v[kMaxArgs];
-  if (!arguments(args, n, entry, v)) return nullptr;
-  return PyLong_FromLongLong(pick(static_cast<size_t>(n - 1), std::make_index_sequence<kMaxArgs + 1>{})(entry, v));
+  if (!arguments(args, n, 0, entry, v)) return nullptr;
+  return PyLong_FromLongLong(pick(static_cast<size_t>(n - 1), std::make_index_sequence<kMaxArgs + 1>{})(entry->f, v));
   END_HANDLE_TH_ERRORS
 }
 
@@ -166,6 +207,7 @@ PyObject* set_check(PyObject*, PyObject* o) {
 }
 
 PyMethodDef methods[] = {
+    {"entry", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry)), METH_FASTCALL, nullptr},
     {"launch", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&launch)), METH_FASTCALL, nullptr},
     {"value", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&value)), METH_FASTCALL, nullptr},
     {"pointer", &pointer, METH_O, nullptr},

@@ -443,3 +443,28 @@ def test_call_module_converts_and_checks_arguments():
         n.empty(cpu, torch.float32, -1)
     with pytest.raises(AttributeError):
         n.no_such_entry
+
+
+@pytest.mark.parametrize("make", [int, bool, "numpy", "tensor"])
+def test_call_module_takes_integers_as_ctypes_does(make):
+    """Integer arguments are anything with __index__ (a numpy integer, a
+    one-element integer tensor), as through ctypes; None and floats are not,
+    and None is a pointer argument's NULL only."""
+    import numpy as np
+    import torch
+
+    n, lib = clef_i4._n, clef_i4.lib()
+    make = {"numpy": np.int64, "tensor": torch.tensor}.get(make, make)
+    for rows, stride, bits in [(3, 256, 4), (1, 512, 8)]:
+        rows, stride, bits = (make(1) if make is bool else make(rows)), int(stride), int(bits)
+        assert n.value(n.clef_i4_prepared_words, rows, stride, bits) == lib.clef_i4_prepared_words(rows, stride, bits)
+    for bad in (None, 1.0, "1", torch.tensor(1.5), torch.tensor([1, 2])):
+        with pytest.raises(Exception):  # ctypes.ArgumentError
+            lib.clef_i4_prepared_words(3, 256, bad)
+        with pytest.raises(TypeError):
+            n.value(n.clef_i4_prepared_words, 3, 256, bad)
+    with pytest.raises(TypeError, match="3 arguments"):
+        n.value(n.clef_i4_prepared_words, 3, 256)
+    for bad in (np.int64(FAKE), 1.0, "1"):
+        with pytest.raises(TypeError, match="unsupported argument type"):
+            n.launch(n.clef_swiglu, bad, None, 0, None)
