@@ -153,7 +153,7 @@ _n = _Native()
 
 # ---------------------------------------------------------------- Q1 / Q2
 
-@functools.lru_cache(maxsize=256)
+@functools.lru_cache(maxsize=256, typed=True)  # 4096.0 is refused whether or not 4096 is held
 def activation_stride(width: int, bits: int = 4) -> int:
     """src/quantized.rs:161-166."""
     return int(lib().clef_i4_activation_stride(width, bits))

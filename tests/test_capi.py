@@ -45,6 +45,13 @@ def test_abi_version_and_stride_rule():
     assert clef_i4.lib().clef_i4_prepared_words(3, 2176, 4) == 3 * 273
 
 
+def test_activation_stride_refuses_floats_held_or_not():
+    clef_i4.activation_stride(4096, 4)
+    for width, bits in [(4096.0, 4), (4096, 4.0), (4352.0, 4)]:
+        with pytest.raises(ctypes.ArgumentError):
+            clef_i4.activation_stride(width, bits)
+
+
 @pytest.mark.parametrize("rows,width,stride,bits", [
     (4, 255, 256, 4), (4, 300, 384, 4), (0, 256, 256, 4), (1048577, 256, 256, 4),
     (4, 256, 200, 4), (4, 256, 65664, 4), (4, 256, 320, 4), (4, 256, 256, 5), (4, 32768 + 256, 33024, 4),
