@@ -470,7 +470,7 @@ int clef_moe_expert_tasks(const float* groups, int64_t tokens, float* tasks, cle
 
 size_t clef_moe_expert_workspace_bytes(int64_t tokens, int32_t topk) {
   if (tokens < 1 || topk < 1) return 0;
-  return align256(clef::expert_schedule_bytes(tokens * topk));
+  return align256(clef::expert_schedule_bytes(tokens * topk, clef::expert_tile_rows(tokens * topk, 256)));
 }
 
 int clef_moe_expert_i4(const uint32_t* a, int32_t stride, const float* a_scales,
@@ -490,8 +490,9 @@ int clef_moe_expert_i4(const uint32_t* a, int32_t stride, const float* a_scales,
     return fail(kAlign);
   if (workspace_bytes < clef_moe_expert_workspace_bytes(tokens, topk)) return fail(kWorkspace);
   int32_t* schedule = static_cast<int32_t*>(workspace);
-  if (int rc = hip_status(clef::launch_expert_schedule(groups, tokens, topk, schedule, hs(stream)))) return rc;
-  return hip_status(clef::launch_expert_i4(a, stride / 8, a_scales, w_tiled, w_scales, groups, schedule,
+  const int bm = clef::expert_tile_rows(tokens * topk, k);
+  if (int rc = hip_status(clef::launch_expert_schedule(groups, tokens, bm, schedule, hs(stream)))) return rc;
+  return hip_status(clef::launch_expert_i4(a, stride / 8, a_scales, w_tiled, w_scales, groups, schedule, bm,
                                            tokens, topk, k, n, input_routed ? 1 : 0, out, hs(stream)));
 }
 
@@ -514,7 +515,7 @@ UngroupedLayout ungrouped_layout(int64_t tokens, int32_t topk) {
   l.slots = take((size_t)routes * 2 * 4);
   l.groups = take((size_t)128 * (routes + 1) * 4);
   l.group_ws = take(clef::group_workspace_bytes(routes));
-  l.schedule = take(clef::expert_schedule_bytes(routes));
+  l.schedule = take(clef::expert_schedule_bytes(routes, clef::expert_tile_rows(routes, 256)));
   l.total = at;
   return l;
 }
@@ -549,11 +550,12 @@ int clef_moe_expert_i4_ungrouped(const uint32_t* a, int32_t stride, const float*
   // Each route slot is grouped as a token of its own (topk 1), so every slot
   // naming an expert is listed, duplicates included, under its ordinal
   // t * topk + r; E1 then reads the lists with that row pitch.
+  const int bm = clef::expert_tile_rows(routed, k);
   if (int rc = hip_status(clef::launch_route_slots(routes, tokens, topk, slots, s))) return rc;
   if (int rc = hip_status(clef::launch_group_routes(slots, routed, 1, groups, nullptr, ws + l.group_ws, s, schedule,
-                                                    clef::expert_tile_rows(routed))))
+                                                    bm)))
     return rc;
-  return hip_status(clef::launch_expert_i4(a, stride / 8, a_scales, w_tiled, w_scales, groups, schedule, tokens,
+  return hip_status(clef::launch_expert_i4(a, stride / 8, a_scales, w_tiled, w_scales, groups, schedule, bm, tokens,
                                            topk, k, n, input_routed ? 1 : 0, out, s, routed + 1));
 }
 
@@ -574,9 +576,10 @@ int clef_moe_expert_gate_up_i4(const uint32_t* a, int32_t stride, const float* a
     return fail(kAlign);
   if (workspace_bytes < clef_moe_expert_workspace_bytes(tokens, topk)) return fail(kWorkspace);
   int32_t* schedule = static_cast<int32_t*>(workspace);
-  if (int rc = hip_status(clef::launch_expert_schedule(groups, tokens, topk, schedule, hs(stream)))) return rc;
+  const int bm = clef::expert_tile_rows(tokens * topk, k);
+  if (int rc = hip_status(clef::launch_expert_schedule(groups, tokens, bm, schedule, hs(stream)))) return rc;
   return hip_status(clef::launch_expert_gate_up(a, stride / 8, a_scales, gate_w, gate_s, up_w, up_s, groups,
-                                                schedule, tokens, topk, k, n, h, hs(stream)));
+                                                schedule, bm, tokens, topk, k, n, h, hs(stream)));
 }
 
 int clef_swiglu(const uint16_t* gate, const uint16_t* up, int64_t n, uint16_t* h, clef_stream_t stream) {
@@ -603,6 +606,7 @@ namespace {
 
 // Workspace carve-up of the MoE block; offsets are 256-byte aligned.
 struct MoeLayout {
+  int bm;  // slots per expert tile
   size_t routes, groups, order, group_ws, schedule, ax, h, ah, values, total;
 };
 
@@ -621,7 +625,8 @@ MoeLayout moe_layout(int64_t tokens, int32_t hidden, int32_t inter, int32_t topk
   const size_t grouping = clef::group_workspace_bytes(tokens);
   const size_t counted = clef::group_counted_fusable(tokens, topk) ? clef::group_counted_bytes(tokens) : 0;
   l.group_ws = take(grouping > counted ? grouping : counted);  // the three-pass grouping's or the router's counts
-  l.schedule = take(clef::expert_schedule_bytes(routed));
+  l.bm = clef::expert_tile_rows(routed, hidden > inter ? hidden : inter);
+  l.schedule = take(clef::expert_schedule_bytes(routed, l.bm));
   l.ax = take((size_t)prepared_words(tokens, stride_for(hidden, 4), 4) * 4);
   l.h = take((size_t)routed * inter * 2);
   l.ah = take((size_t)prepared_words(routed, stride_for(inter, 4), 4) * 4);
@@ -702,7 +707,7 @@ int moe_layer_run(const uint16_t* x, const void* logits, int32_t logits_dtype, i
   if (clef::route_prepare_fusable(hidden) && clef::route_group_fusable(tokens, topk)) {
     // at most 16 tokens: the routing workgroup also groups them
     CLEF_STEP(clef::launch_route_prepare(logits, logits_dtype, tokens, experts, topk, routes, x, hidden, sx, ax, s,
-                                         groups, order, schedule, clef::expert_tile_rows(routed)));
+                                         groups, order, schedule, l.bm));
   } else if (clef::route_prepare_fusable(hidden) && clef::group_counted_fusable(tokens, topk)) {
     // the router also counts each 16-token block's routes per expert; one
     // launch then scans the counts and lists the routes
@@ -710,22 +715,22 @@ int moe_layer_run(const uint16_t* x, const void* logits, int32_t logits_dtype, i
     CLEF_STEP(clef::launch_route_prepare(logits, logits_dtype, tokens, experts, topk, routes, x, hidden, sx, ax, s,
                                          nullptr, nullptr, nullptr, 0, counts16));
     CLEF_STEP(clef::launch_group_counted(routes, tokens, counts16, groups, order, schedule,
-                                         clef::expert_tile_rows(routed), s));
+                                         l.bm, s));
   } else if (clef::route_prepare_fusable(hidden)) {  // router and the quantizer of x side by side
     CLEF_STEP(clef::launch_route_prepare(logits, logits_dtype, tokens, experts, topk, routes, x, hidden, sx, ax, s));
     CLEF_STEP(clef::launch_group_routes(routes, tokens, topk, groups, order, ws + l.group_ws, s, schedule,
-                                        clef::expert_tile_rows(routed)));
+                                        l.bm));
   } else {
     CLEF_STEP(clef::launch_route(logits, logits_dtype, tokens, experts, topk, routes, s));
     CLEF_STEP(clef::launch_group_routes(routes, tokens, topk, groups, order, ws + l.group_ws, s, schedule,
-                                        clef::expert_tile_rows(routed)));
+                                        l.bm));
     CLEF_STEP(clef::launch_prepare(x, tokens, hidden, sx, 4, ax, s));
   }
   // Gate and up share one pass over the gathered x rows and SwiGLU runs in
   // their epilogue; h is then quantized per routed row. Bit-equal to the
   // separate gate, up, swiglu and prepare (each lane applies the same E1
   // rounding and S1 to the same bf16 values).
-  CLEF_STEP(clef::launch_expert_gate_up(ax, sx / 8, axs, gate_w, gate_s, up_w, up_s, groups, schedule, tokens,
+  CLEF_STEP(clef::launch_expert_gate_up(ax, sx / 8, axs, gate_w, gate_s, up_w, up_s, groups, schedule, l.bm, tokens,
                                         topk, hidden, inter, h, s));
   if (clef::down_combine_fusable(tokens, topk, inter, hidden)) {
     // a few tokens: down projection, its quantizer and combine in one launch
@@ -737,7 +742,7 @@ int moe_layer_run(const uint16_t* x, const void* logits, int32_t logits_dtype, i
     CLEF_STEP(clef::launch_expert_down_h(h, down_w, down_s, groups, schedule, tokens, topk, inter, hidden, values, s));
   } else {
     CLEF_STEP(clef::launch_prepare(h, routed, inter, sh, 4, ah, s));
-    CLEF_STEP(clef::launch_expert_i4(ah, sh / 8, ahs, down_w, down_s, groups, schedule, tokens, topk,
+    CLEF_STEP(clef::launch_expert_i4(ah, sh / 8, ahs, down_w, down_s, groups, schedule, l.bm, tokens, topk,
                                      inter, hidden, 1, values, s));
   }
   CLEF_STEP(clef::launch_combine(values, routes, order, tokens, hidden, topk, out, s));

@@ -2285,13 +2285,23 @@ hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const
 // 127.3.
 constexpr int64_t kExpertSmallRoutes = 4096;
 constexpr int kExpertSmallBM = 32;
+// K too deep for expert_stream_kernel (kStreamMaxSteps) leaves the 32-slot
+// tiles to expert_skinny_kernel, which re-reads the weights per tile: up to
+// half as many rows (gate/up of 128 experts 2048 wide, K 7168: 256 tokens at
+// top-8 588 us, 257 on 128-slot tiles 378 against 585, 512: 385 against 813).
+constexpr int64_t kExpertSkinnyRoutes = 2048;
+// Most k-steps whose activation rows fit the LDS beside the rings of
+// expert_stream_kernel.
+constexpr int kStreamMaxSteps = 26;
 
-int expert_tile_rows(int64_t routes) { return routes <= kExpertSmallRoutes ? kExpertSmallBM : kExpertBM; }
+int expert_tile_rows(int64_t routes, int depth) {
+  return routes <= (depth / 256 <= kStreamMaxSteps ? kExpertSmallRoutes : kExpertSkinnyRoutes) ? kExpertSmallBM
+                                                                                              : kExpertBM;
+}
 
 // Tiles of the schedule: sum over experts of ceil(count / bm) <= routes / bm
 // rounded up, plus one per expert with any route.
-int64_t expert_max_tiles(int64_t routes) {
-  const int bm = expert_tile_rows(routes);
+int64_t expert_max_tiles(int64_t routes, int bm) {
   return (routes + bm - 1) / bm + (routes < 128 ? routes : 128);
 }
 
@@ -2300,8 +2310,10 @@ int64_t expert_max_tiles(int64_t routes) {
 // against expert_stream_kernel: 16 tokens 57.3 against 56.8 us, 20: 67.0 /
 // 69.9, 24: 70.6 / 72.1, 32: 79.0 / 75.0 with evenly spread routes; with
 // skewed ones (experts of several rows, a pass each two) 24: 75.3 / 56.5, 32:
-// 86.3 / 60.1.
-constexpr int64_t kExpertDecodeRoutes = 192;
+// 86.3 / 60.1. Where K is too deep for that kernel, against
+// expert_skinny_kernel: 32 tokens (gate/up 7168 x 2048 of 128 experts: 25
+// tokens 295 / 408 us, 32: 344 / 425, skewed 327 / 293).
+constexpr int64_t kExpertDecodeRoutes = 192, kExpertDecodeDeepRoutes = 256;
 
 namespace {
 template <bool GU, int NW, int RW, int MR>
@@ -2311,7 +2323,7 @@ hipError_t launch_expert_decode_t(const uint32_t* a, int a_words, int64_t a_byte
                                   int topk, int k, int n, int input_routed, uint16_t* out, hipStream_t stream) {
   if (a_bytes >= ((int64_t)1 << 31) || n % RW != 0) return hipErrorInvalidValue;
   const int slices = n / RW;
-  const int64_t blocks = expert_max_tiles(routes) * slices;
+  const int64_t blocks = expert_max_tiles(routes, kExpertSmallBM) * slices;
   expert_decode_kernel<GU, NW, RW, MR><<<(unsigned)blocks, NW * 64, 0, stream>>>(
       a, a_words, (uint32_t)a_bytes, as, w, ws, w2, ws2, groups, schedule, list_stride, topk, k / 256, n,
       input_routed, out, slices);
@@ -2350,7 +2362,7 @@ hipError_t launch_expert_down_h_t(const uint16_t* h, const uint32_t* w, const fl
                                   uint16_t* out, hipStream_t stream) {
   constexpr int RW = 32;
   const int slices = n / RW;
-  const int64_t blocks = expert_max_tiles(routes) * slices;
+  const int64_t blocks = expert_max_tiles(routes, kExpertSmallBM) * slices;
   expert_decode_kernel<false, NW, RW, MR, true><<<(unsigned)blocks, NW * 64, 0, stream>>>(
       nullptr, 0, 0u, nullptr, w, ws, w, ws, groups, schedule, list_stride, topk, k / 256, n, 1, out, slices, h);
   return hipGetLastError();
@@ -2367,14 +2379,11 @@ hipError_t launch_expert_stream_t(const uint32_t* a, int a_words, int64_t a_byte
   if (hipError_t e = ensure_dynamic_lds(cache, kern, 160 * 1024)) return e;
   const int colgroups = n / (128 * spw);
   expert_stream_kernel<GU, NB, ONE>
-      <<<(unsigned)(expert_max_tiles(routes) * colgroups), 64 * kStreamWaves, lds, stream>>>(
+      <<<(unsigned)(expert_max_tiles(routes, kExpertSmallBM) * colgroups), 64 * kStreamWaves, lds, stream>>>(
           a, a_words, (uint32_t)a_bytes, as, w, ws, w2, ws2, groups, schedule, list_stride, topk, k / 256, n,
           input_routed, out, (uint32_t)(routes * n * 2), colgroups, spw);
   return hipGetLastError();
 }
-
-// Most k-steps whose activation rows fit the LDS beside the rings.
-constexpr int kStreamMaxSteps = 26;
 
 // SPW, the 32-column slices per wave: up to 16 ring steps per wave (a
 // workgroup's start, three dependent loads, is paid once per about 200 KiB of
@@ -2391,7 +2400,7 @@ hipError_t launch_expert_stream(const uint32_t* a, int a_words, int64_t a_bytes,
   const int kb = k / 256;
   int spw = 1;
   while (spw < 4 && n % (256 * spw) == 0 && 2 * spw * kb * (GU ? 2 : 1) <= 16 &&
-         expert_max_tiles(routes) * (n / (256 * spw)) >= 512)
+         expert_max_tiles(routes, kExpertSmallBM) * (n / (256 * spw)) >= 512)
     spw *= 2;
 #define CLEF_STREAM(ONE)                                                                                           \
   return launch_expert_stream_t<GU, 3, ONE>(a, a_words, a_bytes, as, w, ws, w2, ws2, groups, schedule, routes,     \
@@ -2407,14 +2416,14 @@ hipError_t launch_expert_skinny(const uint32_t* a, int a_words, int64_t a_bytes,
                                 const float* groups, const int32_t* schedule, int64_t routes, int64_t list_stride,
                                 int topk, int k, int n, int input_routed, uint16_t* out, hipStream_t stream) {
   if (a_bytes >= ((int64_t)1 << 31) || n % 32 != 0) return hipErrorInvalidValue;
-  if (routes <= kExpertDecodeRoutes)
+  if (routes <= (k / 256 <= kStreamMaxSteps ? kExpertDecodeRoutes : kExpertDecodeDeepRoutes))
     return launch_expert_decode<GU>(a, a_words, a_bytes, as, w, ws, w2, ws2, groups, schedule, routes, list_stride,
                                     topk, k, n, input_routed, out, stream);
   if (n % 128 == 0 && k / 256 <= kStreamMaxSteps && routes * n * 2 < ((int64_t)1 << 31))
     return launch_expert_stream<GU>(a, a_words, a_bytes, as, w, ws, w2, ws2, groups, schedule, routes, list_stride,
                                     topk, k, n, input_routed, out, stream);
   const int slices = n / 32;
-  const int64_t blocks = expert_max_tiles(routes) * slices;
+  const int64_t blocks = expert_max_tiles(routes, kExpertSmallBM) * slices;
   const int waves = k / 256 < 16 ? k / 256 : 16;  // one k-step per wave at most needs no more waves
   expert_skinny_kernel<GU><<<(unsigned)blocks, 64 * waves, 0, stream>>>(a, a_words, (uint32_t)a_bytes, as, w, ws, w2,
                                                                    ws2, groups, schedule, list_stride, topk, k / 256,
@@ -2433,7 +2442,7 @@ hipError_t launch_expert_dmah(const uint32_t* a, int a_words, int64_t a_bytes, c
   const void* kern = reinterpret_cast<const void*>(&expert_dmah_kernel<T, GU>);
   if (hipError_t e = ensure_dynamic_lds(cache, kern, expert_lds_bytes<T, GU>())) return e;
   const int tiles_n = n / (GU ? T::BN / 2 : T::BN);
-  const int64_t blocks = 8 * ((expert_max_tiles(routes) * tiles_n + 7) / 8);
+  const int64_t blocks = 8 * ((expert_max_tiles(routes, kExpertBM) * tiles_n + 7) / 8);
   expert_dmah_kernel<T, GU><<<(unsigned)blocks, T::THREADS, expert_lds_bytes<T, GU>(), stream>>>(
       a, a_words, (uint32_t)a_bytes, as, w, ws, w2, ws2, groups, schedule, list_stride, topk, k / 256, n, input_routed,
       out, tiles_n);
@@ -2479,19 +2488,19 @@ bool use_expert_persist(int k, int n, int64_t routes) {
   using P = ExpertPersist<GU, kExpertWaves>;
   return k / 256 * 2 >= P::MIN_HALF_STEPS && n % P::COLS == 0 &&
          routes * n * 2 <= ((int64_t)1 << 31) &&  // 32-bit store offsets
-         expert_max_tiles(routes) * (n / P::COLS) < ((int64_t)1 << 31);  // 32-bit item indices
+         expert_max_tiles(routes, kExpertBM) * (n / P::COLS) < ((int64_t)1 << 31);  // 32-bit item indices
 }
 }  // namespace
 
 hipError_t launch_expert_gate_up(const uint32_t* a, int a_words, const float* as, const uint32_t* gate_w,
                                  const float* gate_s, const uint32_t* up_w, const float* up_s, const float* groups,
-                                 const int32_t* schedule, int64_t tokens, int topk, int k, int n, uint16_t* h,
+                                 const int32_t* schedule, int bm, int64_t tokens, int topk, int k, int n, uint16_t* h,
                                  hipStream_t stream, int64_t list_stride) {
   const int64_t a_bytes = tokens * a_words * 4;
   const int64_t routes = tokens * topk;
   if (list_stride <= 0) list_stride = tokens + 1;
   if (a_bytes >= ((int64_t)1 << 31) || n % 128 != 0) return hipErrorInvalidValue;
-  if (expert_tile_rows(routes) == kExpertSmallBM)
+  if (bm == kExpertSmallBM)
     return launch_expert_skinny<true>(a, a_words, a_bytes, as, gate_w, gate_s, up_w, up_s, groups, schedule, routes,
                                       list_stride, topk, k, n, 0, h, stream);
   if (use_expert_persist<true>(k, n, routes))
@@ -2501,14 +2510,12 @@ hipError_t launch_expert_gate_up(const uint32_t* a, int a_words, const float* as
                                                 schedule, routes, list_stride, topk, k, n, 0, h, stream);
 }
 
-size_t expert_schedule_bytes(int64_t routes) {
-  return (size_t)(kSchedEntries + 2 * expert_max_tiles(routes)) * sizeof(int32_t);
+size_t expert_schedule_bytes(int64_t routes, int bm) {
+  return (size_t)(kSchedEntries + 2 * expert_max_tiles(routes, bm)) * sizeof(int32_t);
 }
 
-hipError_t launch_expert_schedule(const float* groups, int64_t tokens, int topk, int32_t* schedule,
-                                  hipStream_t stream) {
-  tile_list_kernel<int32_t, kSchedEntries><<<1, 128, 0, stream>>>(groups, tokens, expert_tile_rows(tokens * topk),
-                                                                  schedule);
+hipError_t launch_expert_schedule(const float* groups, int64_t tokens, int bm, int32_t* schedule, hipStream_t stream) {
+  tile_list_kernel<int32_t, kSchedEntries><<<1, 128, 0, stream>>>(groups, tokens, bm, schedule);
   return hipGetLastError();
 }
 
@@ -2607,14 +2614,14 @@ hipError_t launch_expert_down_h(const uint16_t* h, const uint32_t* w, const floa
 }
 
 hipError_t launch_expert_i4(const uint32_t* a, int a_words, const float* as, const uint32_t* w,
-                            const float* ws, const float* groups, const int32_t* schedule,
+                            const float* ws, const float* groups, const int32_t* schedule, int bm,
                             int64_t tokens, int topk, int k, int n, int input_routed, uint16_t* out,
                             hipStream_t stream, int64_t list_stride) {
   const int64_t routes = tokens * topk;
   const int64_t a_rows = input_routed ? routes : tokens;
   const int64_t a_bytes = a_rows * a_words * 4;
   if (list_stride <= 0) list_stride = tokens + 1;
-  if (expert_tile_rows(routes) == kExpertSmallBM)
+  if (bm == kExpertSmallBM)
     return launch_expert_skinny<false>(a, a_words, a_bytes, as, w, ws, w, ws, groups, schedule, routes, list_stride,
                                        topk, k, n, input_routed, out, stream);
   // The callers reject activation operands of 2 GiB or more and n % 256 != 0.

@@ -119,21 +119,20 @@ hipError_t launch_expert_tasks(const float* groups, int64_t tokens, float* tasks
                                hipStream_t stream);
 
 // Tile schedule of the grouped expert GEMM: int32 [kSchedEntries + 2 *
-// max_tiles], tiles of expert_tile_rows(routes) slots for `routes` routed rows
-// (tokens * topk): 32-slot tiles for few routed rows, 128-slot tiles
-// otherwise. The expert GEMM launches pick their kernel by the same rule, so a
-// schedule must be built for the routes count the GEMMs are launched with.
+// max_tiles], tiles of `bm` slots (expert_tile_rows): 32 for few routed rows
+// (tokens * topk), 128 otherwise. The expert GEMM launches pick their kernel by
+// `bm`, which must be that of the schedule they are given. `depth` is the
+// largest K of the GEMMs that share the schedule.
 // Layout: [0] the tile count; [kSchedClaims, +16) the work counters of the
 // persistent expert kernels (eight per launch, one per XCD: the fused gate/up
 // kernel uses the first eight, the other the second eight), zeroed by every
 // writer of [0]; tile t's expert and first slot at [kSchedEntries + 2t] and
 // [kSchedEntries + 2t + 1].
 constexpr int kSchedClaims = 1, kSchedEntries = 17;
-int expert_tile_rows(int64_t routes);
-int64_t expert_max_tiles(int64_t routes);
-size_t expert_schedule_bytes(int64_t routes);
-hipError_t launch_expert_schedule(const float* groups, int64_t tokens, int topk, int32_t* schedule,
-                                  hipStream_t stream);
+int expert_tile_rows(int64_t routes, int depth);
+int64_t expert_max_tiles(int64_t routes, int bm);
+size_t expert_schedule_bytes(int64_t routes, int bm);
+hipError_t launch_expert_schedule(const float* groups, int64_t tokens, int bm, int32_t* schedule, hipStream_t stream);
 // `list_stride` is the row pitch of `groups` in floats: tokens + 1 for the
 // reference's table (0 selects it), more for a table that lists every route
 // slot (ungrouped, duplicates included).
@@ -166,14 +165,14 @@ hipError_t launch_expert_down_h(const uint16_t* h, const uint32_t* w, const floa
                                 hipStream_t stream);
 hipError_t launch_expert_i4(const uint32_t* a, int a_words, const float* a_scales,
                             const uint32_t* w_tiled, const float* w_scales, const float* groups,
-                            const int32_t* schedule, int64_t tokens, int topk, int k, int n,
+                            const int32_t* schedule, int bm, int64_t tokens, int topk, int k, int n,
                             int input_routed, uint16_t* out, hipStream_t stream, int64_t list_stride = 0);
 
 // Fused gate/up expert GEMMs with SwiGLU: h[route][c] = S1(E1(gate), E1(up)),
 // routed rows gathered from `a` by route / topk; n % 128 == 0.
 hipError_t launch_expert_gate_up(const uint32_t* a, int a_words, const float* as, const uint32_t* gate_w,
                                  const float* gate_s, const uint32_t* up_w, const float* up_s, const float* groups,
-                                 const int32_t* schedule, int64_t tokens, int topk, int k, int n, uint16_t* h,
+                                 const int32_t* schedule, int bm, int64_t tokens, int topk, int k, int n, uint16_t* h,
                                  hipStream_t stream, int64_t list_stride = 0);
 
 // Every route slot of `routes` ([tokens][2 * topk]) as a one-slot token:
