@@ -2284,6 +2284,13 @@ hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* as, const
 // 113.9, 620: 124.4 / 116.9; skewed routing 500: 106.7 / 122.0, 620: 117.1 /
 // 127.3.
 constexpr int64_t kExpertSmallRoutes = 4096;
+// Above K 2048 its workgroups fill more than half of a CU's LDS, one per CU
+// instead of two, and the 128-slot kernel is ahead sooner: gate/up + down, us,
+// 32-slot / 128-slot tiles: 4096 x 1536 448 tokens 290.6 / 295.2, 512: 312.0 /
+// 296.7; 2560 x 1024 448: 134.5 / 135.2, 480: 146.3 / 135.5; 6656 x 2048 448:
+// 558.4 / 568.9, 512: 605.7 / 574.0.
+constexpr int64_t kExpertSmallDeepRoutes = 3584;
+constexpr int kExpertSmallDepth = 2048;
 constexpr int kExpertSmallBM = 32;
 // K too deep for expert_stream_kernel (kStreamMaxSteps) leaves the 32-slot
 // tiles to expert_skinny_kernel, which re-reads the weights per tile: up to
@@ -2295,8 +2302,10 @@ constexpr int64_t kExpertSkinnyRoutes = 2048;
 constexpr int kStreamMaxSteps = 26;
 
 int expert_tile_rows(int64_t routes, int depth) {
-  return routes <= (depth / 256 <= kStreamMaxSteps ? kExpertSmallRoutes : kExpertSkinnyRoutes) ? kExpertSmallBM
-                                                                                              : kExpertBM;
+  const int64_t small = depth <= kExpertSmallDepth        ? kExpertSmallRoutes
+                        : depth / 256 <= kStreamMaxSteps ? kExpertSmallDeepRoutes
+                                                         : kExpertSkinnyRoutes;
+  return routes <= small ? kExpertSmallBM : kExpertBM;
 }
 
 // Tiles of the schedule: sum over experts of ceil(count / bm) <= routes / bm

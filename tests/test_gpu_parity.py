@@ -738,12 +738,13 @@ def test_expert_gate_up_persistent_matches_oracle(tokens, k, n, skew):
 # three, eight and the most k-steps its LDS takes (and one more: the kernel
 # for wider rows), one, two and four slices per wave, tiles with one slot and
 # full ones, experts of several tiles, both ends of its range of routed rows
-# and one token count past it. K 6912 (a k-step too many for its LDS): the
+# (K to 2048 and above it) and one token count past it. K 6912 (a k-step too many for its LDS): the
 # dot-product kernel to 256 routed rows, the skinny one to 2048, 128-slot tiles.
 STREAM_CASES = [(25, 256, 256, 8, 0.0), (40, 512, 768, 8, 2.0), (300, 512, 2048, 8, 0.0), (300, 256, 1024, 8, 3.0),
                 (512, 768, 512, 8, 1.0), (513, 768, 512, 8, 1.0), (100, 2048, 256, 4, 2.0), (60, 2304, 256, 8, 0.0),
                 (30, 6656, 256, 8, 1.0), (30, 6912, 256, 8, 1.0),
-                (40, 6912, 256, 8, 1.0), (257, 6912, 256, 8, 1.0), (260, 1024, 768, 6, 4.0)]
+                (40, 6912, 256, 8, 1.0), (257, 6912, 256, 8, 1.0), (448, 2304, 256, 8, 1.0), (449, 2304, 256, 8, 1.0),
+                (260, 1024, 768, 6, 4.0)]
 
 
 def _stream_operands(tokens, k, n, topk, skew, weights, rows):
