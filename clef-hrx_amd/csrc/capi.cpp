@@ -470,7 +470,7 @@ int clef_moe_expert_tasks(const float* groups, int64_t tokens, float* tasks, cle
 
 size_t clef_moe_expert_workspace_bytes(int64_t tokens, int32_t topk) {
   if (tokens < 1 || topk < 1) return 0;
-  return align256(clef::expert_schedule_bytes(tokens * topk, clef::expert_tile_rows(tokens * topk, 256)));
+  return align256(clef::expert_schedule_bound(tokens * topk));
 }
 
 int clef_moe_expert_i4(const uint32_t* a, int32_t stride, const float* a_scales,
@@ -488,9 +488,9 @@ int clef_moe_expert_i4(const uint32_t* a, int32_t stride, const float* a_scales,
   if (!aligned(a, 16) || !aligned(a_scales, 4) || !aligned(w_tiled, 16) || !aligned(w_scales, 16) ||
       !aligned(groups, 4) || !aligned(out, 16) || !aligned(workspace, 16))
     return fail(kAlign);
-  if (workspace_bytes < clef_moe_expert_workspace_bytes(tokens, topk)) return fail(kWorkspace);
+  const int bm = clef::expert_tile_rows(tokens * topk, k, workspace_bytes);
+  if (workspace_bytes < align256(clef::expert_schedule_bytes(tokens * topk, bm))) return fail(kWorkspace);
   int32_t* schedule = static_cast<int32_t*>(workspace);
-  const int bm = clef::expert_tile_rows(tokens * topk, k);
   if (int rc = hip_status(clef::launch_expert_schedule(groups, tokens, bm, schedule, hs(stream)))) return rc;
   return hip_status(clef::launch_expert_i4(a, stride / 8, a_scales, w_tiled, w_scales, groups, schedule, bm,
                                            tokens, topk, k, n, input_routed ? 1 : 0, out, hs(stream)));
@@ -501,7 +501,7 @@ namespace {
 // their per-expert lists [128][routes + 1], the grouping scratch and the tile
 // schedule.
 struct UngroupedLayout {
-  size_t slots, groups, group_ws, schedule, total;
+  size_t slots, groups, group_ws, schedule;  // the schedule lies last
 };
 UngroupedLayout ungrouped_layout(int64_t tokens, int32_t topk) {
   const int64_t routes = tokens * topk;
@@ -515,15 +515,14 @@ UngroupedLayout ungrouped_layout(int64_t tokens, int32_t topk) {
   l.slots = take((size_t)routes * 2 * 4);
   l.groups = take((size_t)128 * (routes + 1) * 4);
   l.group_ws = take(clef::group_workspace_bytes(routes));
-  l.schedule = take(clef::expert_schedule_bytes(routes, clef::expert_tile_rows(routes, 256)));
-  l.total = at;
+  l.schedule = at;
   return l;
 }
 }  // namespace
 
 size_t clef_moe_expert_ungrouped_workspace_bytes(int64_t tokens, int32_t topk) {
   if (!routes_in_range(tokens, topk)) return 0;
-  return ungrouped_layout(tokens, topk).total;
+  return ungrouped_layout(tokens, topk).schedule + align256(clef::expert_schedule_bound(tokens * topk));
 }
 
 int clef_moe_expert_i4_ungrouped(const uint32_t* a, int32_t stride, const float* a_scales,
@@ -540,7 +539,9 @@ int clef_moe_expert_i4_ungrouped(const uint32_t* a, int32_t stride, const float*
       !aligned(routes, 4) || !aligned(out, 16) || !aligned(workspace, 256))
     return fail(kAlign);
   const UngroupedLayout l = ungrouped_layout(tokens, topk);
-  if (workspace_bytes < l.total) return fail(kWorkspace);
+  if (workspace_bytes < l.schedule) return fail(kWorkspace);
+  const int bm = clef::expert_tile_rows(tokens * topk, k, workspace_bytes - l.schedule);
+  if (workspace_bytes - l.schedule < align256(clef::expert_schedule_bytes(tokens * topk, bm))) return fail(kWorkspace);
   char* ws = static_cast<char*>(workspace);
   float* slots = reinterpret_cast<float*>(ws + l.slots);
   float* groups = reinterpret_cast<float*>(ws + l.groups);
@@ -550,7 +551,6 @@ int clef_moe_expert_i4_ungrouped(const uint32_t* a, int32_t stride, const float*
   // Each route slot is grouped as a token of its own (topk 1), so every slot
   // naming an expert is listed, duplicates included, under its ordinal
   // t * topk + r; E1 then reads the lists with that row pitch.
-  const int bm = clef::expert_tile_rows(routed, k);
   if (int rc = hip_status(clef::launch_route_slots(routes, tokens, topk, slots, s))) return rc;
   if (int rc = hip_status(clef::launch_group_routes(slots, routed, 1, groups, nullptr, ws + l.group_ws, s, schedule,
                                                     bm)))
@@ -574,9 +574,9 @@ int clef_moe_expert_gate_up_i4(const uint32_t* a, int32_t stride, const float* a
       !aligned(up_w, 16) || !aligned(up_s, 16) || !aligned(groups, 4) || !aligned(h, 16) ||
       !aligned(workspace, 16))
     return fail(kAlign);
-  if (workspace_bytes < clef_moe_expert_workspace_bytes(tokens, topk)) return fail(kWorkspace);
+  const int bm = clef::expert_tile_rows(tokens * topk, k, workspace_bytes);
+  if (workspace_bytes < align256(clef::expert_schedule_bytes(tokens * topk, bm))) return fail(kWorkspace);
   int32_t* schedule = static_cast<int32_t*>(workspace);
-  const int bm = clef::expert_tile_rows(tokens * topk, k);
   if (int rc = hip_status(clef::launch_expert_schedule(groups, tokens, bm, schedule, hs(stream)))) return rc;
   return hip_status(clef::launch_expert_gate_up(a, stride / 8, a_scales, gate_w, gate_s, up_w, up_s, groups,
                                                 schedule, bm, tokens, topk, k, n, h, hs(stream)));
@@ -604,13 +604,14 @@ int clef_moe_combine(const uint16_t* values, const float* routes, const float* o
 
 namespace {
 
-// Workspace carve-up of the MoE block; offsets are 256-byte aligned.
+// Workspace carve-up of the MoE block; offsets are 256-byte aligned. `bytes`:
+// what the workspace holds; the schedule, last, takes expert tiles that fit.
 struct MoeLayout {
   int bm;  // slots per expert tile
-  size_t routes, groups, order, group_ws, schedule, ax, h, ah, values, total;
+  size_t routes, groups, order, group_ws, ax, h, ah, values, schedule, total;
 };
 
-MoeLayout moe_layout(int64_t tokens, int32_t hidden, int32_t inter, int32_t topk) {
+MoeLayout moe_layout(int64_t tokens, int32_t hidden, int32_t inter, int32_t topk, size_t bytes = SIZE_MAX) {
   MoeLayout l{};
   const int64_t routed = tokens * topk;
   size_t at = 0;
@@ -625,12 +626,12 @@ MoeLayout moe_layout(int64_t tokens, int32_t hidden, int32_t inter, int32_t topk
   const size_t grouping = clef::group_workspace_bytes(tokens);
   const size_t counted = clef::group_counted_fusable(tokens, topk) ? clef::group_counted_bytes(tokens) : 0;
   l.group_ws = take(grouping > counted ? grouping : counted);  // the three-pass grouping's or the router's counts
-  l.bm = clef::expert_tile_rows(routed, hidden > inter ? hidden : inter);
-  l.schedule = take(clef::expert_schedule_bytes(routed, l.bm));
   l.ax = take((size_t)prepared_words(tokens, stride_for(hidden, 4), 4) * 4);
   l.h = take((size_t)routed * inter * 2);
   l.ah = take((size_t)prepared_words(routed, stride_for(inter, 4), 4) * 4);
   l.values = take((size_t)routed * hidden * 2);
+  l.bm = clef::expert_tile_rows(routed, hidden > inter ? hidden : inter, bytes > at ? bytes - at : 0);
+  l.schedule = take(clef::expert_schedule_bytes(routed, l.bm));
   l.total = at;
   return l;
 }
@@ -679,8 +680,7 @@ int check_moe_pointers(const uint16_t* x, const void* logits, const uint32_t* ga
 int moe_layer_run(const uint16_t* x, const void* logits, int32_t logits_dtype, int64_t tokens, int32_t hidden,
                   int32_t inter, int32_t experts, int32_t topk, const uint32_t* gate_w, const float* gate_s,
                   const uint32_t* up_w, const float* up_s, const uint32_t* down_w, const float* down_s,
-                  float* routes_out, uint16_t* out, char* ws, hipStream_t s) {
-  const MoeLayout l = moe_layout(tokens, hidden, inter, topk);
+                  float* routes_out, uint16_t* out, char* ws, const MoeLayout& l, hipStream_t s) {
   const int32_t sx = stride_for(hidden, 4), sh = stride_for(inter, 4);
   float* routes = routes_out ? routes_out : reinterpret_cast<float*>(ws + l.routes);
   float* groups = reinterpret_cast<float*>(ws + l.groups);
@@ -792,9 +792,10 @@ int clef_moe_layer(const uint16_t* x, const void* logits, int32_t logits_dtype, 
   if (int rc = check_moe_layer(tokens, hidden, inter, experts, topk)) return rc;
   if (int rc = check_moe_pointers(x, logits, gate_w, gate_s, up_w, up_s, down_w, down_s, routes_out, out)) return rc;
   if (!aligned(workspace, 256)) return fail(kAlign);
-  if (workspace_bytes < moe_layout(tokens, hidden, inter, topk).total) return fail(kWorkspace);
+  const MoeLayout l = moe_layout(tokens, hidden, inter, topk, workspace_bytes);
+  if (workspace_bytes < l.total) return fail(kWorkspace);
   return moe_layer_run(x, logits, logits_dtype, tokens, hidden, inter, experts, topk, gate_w, gate_s, up_w, up_s,
-                       down_w, down_s, routes_out, out, static_cast<char*>(workspace), hs(stream));
+                       down_w, down_s, routes_out, out, static_cast<char*>(workspace), l, hs(stream));
 }
 
 int clef_moe_layer_static(const uint16_t* x, const void* logits, int32_t logits_dtype, int64_t tokens,
@@ -804,7 +805,8 @@ int clef_moe_layer_static(const uint16_t* x, const void* logits, int32_t logits_
                           float* routes_out, uint16_t* out, clef_stream_t stream) {
   if (int rc = check_moe_layer(tokens, hidden, inter, experts, topk)) return rc;
   if (int rc = check_moe_pointers(x, logits, gate_w, gate_s, up_w, up_s, down_w, down_s, routes_out, out)) return rc;
-  const size_t need = moe_layout(tokens, hidden, inter, topk).total;
+  const MoeLayout l = moe_layout(tokens, hidden, inter, topk, kStaticScratchBytes);
+  const size_t need = l.total;
   if (need > kStaticScratchBytes) {
     std::snprintf(g_error, sizeof g_error,
                   "MoE layer needs %zu bytes of scratch; the static scratch holds %zu (use clef_moe_layer "
@@ -815,7 +817,7 @@ int clef_moe_layer_static(const uint16_t* x, const void* logits, int32_t logits_
   char* ws = nullptr;
   if (int rc = static_scratch(&ws)) return rc;
   return moe_layer_run(x, logits, logits_dtype, tokens, hidden, inter, experts, topk, gate_w, gate_s, up_w, up_s,
-                       down_w, down_s, routes_out, out, ws, hs(stream));
+                       down_w, down_s, routes_out, out, ws, l, hs(stream));
 }
 
 }  // extern "C"

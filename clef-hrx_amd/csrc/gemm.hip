@@ -2301,10 +2301,13 @@ constexpr int64_t kExpertSkinnyRoutes = 2048;
 // expert_stream_kernel.
 constexpr int kStreamMaxSteps = 26;
 
-int expert_tile_rows(int64_t routes, int depth) {
+int expert_tile_rows(int64_t routes, int depth, size_t schedule_bytes) {
   const int64_t small = depth <= kExpertSmallDepth        ? kExpertSmallRoutes
                         : depth / 256 <= kStreamMaxSteps ? kExpertSmallDeepRoutes
                                                          : kExpertSkinnyRoutes;
+  // the entries' scratch comes in whole 256-byte blocks
+  if (routes > kExpertSkinnyRoutes && schedule_bytes < (expert_schedule_bytes(routes, kExpertSmallBM) + 255) / 256 * 256)
+    return kExpertBM;
   return routes <= small ? kExpertSmallBM : kExpertBM;
 }
 
@@ -2521,6 +2524,12 @@ hipError_t launch_expert_gate_up(const uint32_t* a, int a_words, const float* as
 
 size_t expert_schedule_bytes(int64_t routes, int bm) {
   return (size_t)(kSchedEntries + 2 * expert_max_tiles(routes, bm)) * sizeof(int32_t);
+}
+
+size_t expert_schedule_bound(int64_t routes) {
+  const int64_t few = routes < kExpertSmallRoutes ? routes : kExpertSmallRoutes;
+  const size_t small = expert_schedule_bytes(few, kExpertSmallBM), large = expert_schedule_bytes(routes, kExpertBM);
+  return small > large ? small : large;
 }
 
 hipError_t launch_expert_schedule(const float* groups, int64_t tokens, int bm, int32_t* schedule, hipStream_t stream) {

@@ -122,16 +122,20 @@ hipError_t launch_expert_tasks(const float* groups, int64_t tokens, float* tasks
 // max_tiles], tiles of `bm` slots (expert_tile_rows): 32 for few routed rows
 // (tokens * topk), 128 otherwise. The expert GEMM launches pick their kernel by
 // `bm`, which must be that of the schedule they are given. `depth` is the
-// largest K of the GEMMs that share the schedule.
+// largest K of the GEMMs that share the schedule; `schedule_bytes` the scratch
+// there is for it: between kExpertSkinnyRoutes and the 32-slot tiles' limit a
+// schedule of 128-slot tiles, which is smaller, serves where theirs does not
+// fit. expert_schedule_bound suffices for every depth and any fewer routes.
 // Layout: [0] the tile count; [kSchedClaims, +16) the work counters of the
 // persistent expert kernels (eight per launch, one per XCD: the fused gate/up
 // kernel uses the first eight, the other the second eight), zeroed by every
 // writer of [0]; tile t's expert and first slot at [kSchedEntries + 2t] and
 // [kSchedEntries + 2t + 1].
 constexpr int kSchedClaims = 1, kSchedEntries = 17;
-int expert_tile_rows(int64_t routes, int depth);
+int expert_tile_rows(int64_t routes, int depth, size_t schedule_bytes = SIZE_MAX);
 int64_t expert_max_tiles(int64_t routes, int bm);
 size_t expert_schedule_bytes(int64_t routes, int bm);
+size_t expert_schedule_bound(int64_t routes);
 hipError_t launch_expert_schedule(const float* groups, int64_t tokens, int bm, int32_t* schedule, hipStream_t stream);
 // `list_stride` is the row pitch of `groups` in floats: tokens + 1 for the
 // reference's table (0 selects it), more for a table that lists every route

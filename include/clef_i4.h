@@ -339,7 +339,8 @@ int clef_moe_group_routes(const float* routes, int64_t tokens, int32_t topk, flo
  * floats. */
 int clef_moe_expert_tasks(const float* groups, int64_t tokens, float* tasks, clef_stream_t stream);
 
-/* Bytes of scratch clef_moe_expert_i4 needs (its tile schedule). */
+/* Bytes of scratch for clef_moe_expert_i4 (its tile schedule); enough for any
+ * fewer tokens too. */
 size_t clef_moe_expert_workspace_bytes(int64_t tokens, int32_t topk);
 
 /* Grouped INT4 expert GEMM over all 128 experts:

@@ -336,6 +336,21 @@ def test_router_logits_rejects(tokens, hidden, experts):
     assert rc == -1 and msg == "linear shape/dtype mismatch"
 
 
+def test_expert_workspaces_suffice_for_fewer_tokens():
+    """Scratch sized for the most tokens a caller will pass serves every
+    smaller call, whichever expert tiles that call takes."""
+    lib = clef_i4.lib()
+    tokens = [1, 8, 24, 25, 32, 33, 128, 255, 256, 257, 400, 448, 449, 511, 512, 513, 600, 700, 1024, 1500, 2048, 2049,
+              4096, 16384]
+    for topk in (1, 4, 8):
+        for size in (lib.clef_moe_expert_workspace_bytes, lib.clef_moe_expert_ungrouped_workspace_bytes,
+                     lambda t, k: lib.clef_moe_layer_workspace_bytes(t, 2048, 768, k),
+                     lambda t, k: lib.clef_moe_layer_workspace_bytes(t, 256, 256, k),
+                     lambda t, k: lib.clef_moe_layer_workspace_bytes(t, 7168, 256, k)):
+            sizes = [size(t, topk) for t in tokens]
+            assert sizes == sorted(sizes), (topk, sizes)
+
+
 def test_moe_layer_static_rejects_beyond_scratch():
     """clef_moe_layer_static allocates nothing: shapes whose intermediates
     exceed its 32 MiB static scratch are rejected before any device work."""

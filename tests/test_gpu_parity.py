@@ -781,6 +781,65 @@ def test_expert_gate_up_stream_matches_oracle(tokens, k, n, topk, skew):
         assert_same_bf16_nan_aware(bf16_host(got), want, f"gate/up stream t={tokens} k={k} n={n}")
 
 
+@pytest.mark.parametrize("tokens", [257, 400, 512])
+def test_experts_in_the_scratch_of_128_slot_tiles(tokens):
+    """Between 2049 and 4096 routed rows the expert entries prefer 32-slot
+    tiles, whose schedule takes up to 768 bytes more; with scratch for the
+    128-slot schedule only they run those, the same output, and write nothing
+    past the scratch they were given."""
+    k, n, topk = 768, 512, 8
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    rng = np.random.default_rng(tokens)
+    bf = lambda *shape: torch.randn(shape, generator=g, device="cuda", dtype=torch.bfloat16)  # noqa: E731
+    routes = random_routes(rng, tokens, skew=1.0)
+    groups, routes = to_dev_f32(oracle.group_routes(routes)[0]), to_dev_f32(routes)
+    wg, wu, wd = (clef_i4.load_quantized_weight(bf(128 * r, c) * 0.02) for r, c in ((n, k), (n, k), (k, n)))
+    a = clef_i4.prepare(bf(tokens, k))
+    c = clef_i4._n
+    # 17 counters, then two words for each of the most tiles there can be
+    small = ((17 + 2 * ((tokens * topk + 127) // 128 + 128)) * 4 + 255) // 256 * 256
+    assert small < c.value(c.clef_moe_expert_workspace_bytes, tokens, topk)
+
+    def run(entry, nbytes, *args):
+        ws = torch.full((nbytes + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+        c.launch(entry, *args, ws, nbytes)
+        assert bool((ws[nbytes:] == 0x5A).all())
+
+    def same(got, want):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+    got = torch.empty((tokens * topk, n), dtype=torch.bfloat16, device="cuda")
+    want = clef_i4.omni_expert(a, wg, groups, tokens, topk, False)
+    run(c.clef_moe_expert_i4, small, a.storage, a.stride, a.scales, wg.codes, wg.scales, groups, tokens, topk, k, n, 0,
+        got)
+    same(got, want)
+    ungrouped = c.value(c.clef_moe_expert_ungrouped_workspace_bytes, tokens, topk) \
+        - c.value(c.clef_moe_expert_workspace_bytes, tokens, topk) + small
+    run(c.clef_moe_expert_i4_ungrouped, ungrouped, a.storage, a.stride, a.scales, wg.codes, wg.scales, routes, tokens,
+        topk, k, n, 0, got.zero_())
+    same(got, want)
+    run(c.clef_moe_expert_gate_up_i4, small, a.storage, a.stride, a.scales, wg.codes, wg.scales, wu.codes, wu.scales,
+        groups, tokens, topk, k, n, got)
+    same(got, clef_i4.omni_gate_up(a, wg, wu, groups, tokens, topk))
+    for entry, args in ((c.clef_moe_expert_i4, (wg.codes, wg.scales, groups, tokens, topk, k, n, 0, got)),
+                        (c.clef_moe_expert_gate_up_i4, (wg.codes, wg.scales, wu.codes, wu.scales, groups, tokens, topk,
+                                                        k, n, got))):
+        with pytest.raises(clef_i4.ClefError, match="workspace too small"):
+            run(entry, small - 1, a.storage, a.stride, a.scales, *args)
+
+    x, logits = bf(tokens, k), bf(tokens, 128)
+    layer = clef_i4.MoeLayer(wg, wu, wd)
+    want, out = layer(x, logits), torch.empty_like(x)
+    full = c.value(c.clef_moe_layer_workspace_bytes, tokens, k, n, topk)
+    large = ((17 + 2 * ((tokens * topk + 31) // 32 + 128)) * 4 + 255) // 256 * 256
+    args = (x, logits, 0, tokens, k, n, 128, topk, wg.codes, wg.scales, wu.codes, wu.scales, wd.codes, wd.scales, None,
+            out)
+    run(c.clef_moe_layer, full - large + small, *args)
+    same(out, want)
+    with pytest.raises(clef_i4.ClefError, match="workspace too small"):
+        run(c.clef_moe_layer, full - large + small - 1, *args)
+
+
 def test_swiglu_every_bf16_gate():
     """swiglu_preserves_materialized_rounding (src/ops.rs:482-520) over all
     65536 gate bit patterns."""
