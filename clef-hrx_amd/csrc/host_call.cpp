@@ -24,10 +24,12 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
+#include <cstring>
 #include <deque>
 #include <utility>
 
 #include "build_id.inc"  // CLEF_BUILD_ID, generated by the Makefile
+#include "host_abi.inc"  // CLEF_TORCH_VERSION, likewise
 
 namespace {
 
@@ -219,7 +221,36 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "clef_host", nullptr, -1, metho
 
 }  // namespace
 
+namespace {
+
+// The functions above use torch's and Python's class layouts as their headers
+// gave them: no other version of either loads this module. (Written with
+// functions of Python's stable interface only.)
+bool built_for_this_process() {
+#define CLEF_STR2(x) #x
+#define CLEF_STR(x) CLEF_STR2(x)
+  constexpr const char* python = CLEF_STR(PY_MAJOR_VERSION) "." CLEF_STR(PY_MINOR_VERSION) ".";
+  PyObject* torch = PyImport_ImportModule("torch");
+  PyObject* version = torch != nullptr ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+  PyObject* text = version != nullptr ? PyObject_Str(version) : nullptr;
+  const char* found = text != nullptr ? PyUnicode_AsUTF8AndSize(text, nullptr) : nullptr;
+  const bool same = found != nullptr && std::strcmp(found, CLEF_TORCH_VERSION) == 0 &&
+                    std::strncmp(Py_GetVersion(), python, std::strlen(python)) == 0;
+  if (found != nullptr && !same)
+    PyErr_Format(PyExc_ImportError,
+                 "the call module was built for torch %s and Python %sx, this is torch %s and Python %s; run `make -C "
+                 "clef-hrx_amd`",
+                 CLEF_TORCH_VERSION, python, found, Py_GetVersion());
+  Py_XDECREF(text);
+  Py_XDECREF(version);
+  Py_XDECREF(torch);
+  return same;
+}
+
+}  // namespace
+
 PyMODINIT_FUNC PyInit_clef_host() {
+  if (!built_for_this_process()) return nullptr;
   PyObject* c = PyImport_ImportModule("torch._C");
   if (c == nullptr) return nullptr;
   g_device = PyObject_GetAttrString(c, "_cuda_getDevice");

@@ -490,3 +490,41 @@ def test_call_module_takes_integers_as_ctypes_does(make):
     for bad in (np.int64(FAKE), 1.0, "1"):
         with pytest.raises(TypeError, match="unsupported argument type"):
             n.launch(n.clef_swiglu, bad, None, 0, None)
+
+
+def test_call_module_loads_under_its_own_torch_only(tmp_path, monkeypatch):
+    """The call module uses torch's class layouts, so another torch than the
+    one it was built against is refused before any of its functions runs."""
+    import importlib.machinery
+    import importlib.util
+    import shutil
+
+    import torch
+
+    def load(name):  # a copy of its own: Python keeps a loaded module per file
+        path = shutil.copy(clef_i4.HOST_PATH, tmp_path / name)
+        loader = importlib.machinery.ExtensionFileLoader("clef_host", str(path))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("clef_host", loader))
+        loader.exec_module(module)
+        return module
+
+    assert load("same.so").build_id == clef_i4.lib().clef_build_id().decode()
+    monkeypatch.setattr(torch, "__version__", "2.99.0")
+    with pytest.raises(ImportError, match=r"built for torch .* this is torch 2\.99\.0"):
+        load("other.so")
+
+
+def test_library_builds_without_torch(tmp_path):
+    """The C library needs no torch: where Python finds none, make leaves the
+    binding's call module out and builds the rest."""
+    import subprocess
+
+    fake = tmp_path / "python"
+    fake.write_text("#!/bin/sh\nexec python3 -S \"$@\"\n")  # no site-packages
+    fake.chmod(0o755)
+    pkg = os.path.dirname(clef_i4.LIB_PATH) + "/.."
+    plan = [subprocess.run(["make", "-n", "-B", "-C", pkg, f"PYTHON={p}"], capture_output=True, text=True)
+            for p in ("python3", fake)]
+    assert all(p.returncode == 0 for p in plan), plan
+    assert [("host_call.cpp" in p.stdout, "libclef_i4.so" in p.stdout) for p in plan] == [(True, True), (False, True)]
+    assert "Traceback" not in plan[1].stderr
