@@ -805,15 +805,16 @@ class MoeLayer:
         self.router = router  # bf16 [128][hidden] router gate, used when no logits are given
         self.hidden = gate.cols
         self.inter = gate.rows // 128
-        self._ws = None
-        self._ws_tokens = -1
+        self._ws_size = (-1, 0)  # the last call's tokens and scratch bytes
 
     def workspace(self, tokens: int, device) -> torch.Tensor:
-        if self._ws_tokens != tokens:
+        """Scratch of one call, from torch's allocator each time: calls of
+        other streams and threads and captured graphs have their own."""
+        held, nbytes = self._ws_size
+        if held != tokens:
             nbytes = _n.value(_n.clef_moe_layer_workspace_bytes, tokens, self.hidden, self.inter, self.topk)
-            self._ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-            self._ws_tokens = tokens
-        return self._ws
+            self._ws_size = tokens, nbytes
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
     def __call__(self, x: torch.Tensor, logits: torch.Tensor | None = None, routes_out: torch.Tensor | None = None,
                  out: torch.Tensor | None = None) -> torch.Tensor:

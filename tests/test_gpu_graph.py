@@ -69,3 +69,38 @@ def test_graph_replays_match_eager(t, pm, pn):
         assert torch.equal(moe_out.view(torch.int16), want_moe.view(torch.int16)), f"replay {i}: MoE layer"
         assert torch.equal(proj_out.view(torch.int16), want_proj.view(torch.int16)), f"replay {i}: projection"
         _ = (moe_out.float().sum() + 1).item()  # eager work between replays
+
+
+def test_moe_layer_scratch_is_each_calls_own():
+    """No two calls of one layer share scratch unordered: a graph captured
+    after an eager call keeps its own when a call of another token count
+    follows (replays write no memory that eager tensors hold since), and
+    calls of two streams have theirs."""
+    d, inter, t = 512, 256, 40
+    layer = clef_i4.MoeLayer(*(clef_i4.load_quantized_weight(randn((128 * r, c), 0.02, s))
+                               for r, c, s in ((inter, d, 1), (inter, d, 2), (d, inter, 3))))
+    x, logits, x2, logits2 = randn((t, d), 1.0, 4), randn((t, 128), 1.0, 5), randn((9, d), 1.0, 6), randn((9, 128), 1.0, 7)
+    out = torch.empty_like(x)
+    nbytes = clef_i4.lib().clef_moe_layer_workspace_bytes(t, d, inter, 8)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = layer(x, logits)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layer(x, logits, out=out)
+    with torch.cuda.stream(side):
+        layer(x2, logits2)
+        held = [torch.full((nbytes,), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(4)]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        assert all(bool((h == 0x5A).all()) for h in held)
+    first = layer.workspace(t, "cuda")
+    with torch.cuda.stream(side):
+        second = layer.workspace(t, "cuda")
+    assert first.data_ptr() != second.data_ptr() and first.numel() == second.numel() == nbytes

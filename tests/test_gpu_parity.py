@@ -961,7 +961,8 @@ def test_moe_layer_degenerate_logit_rows(tokens):
     down = packed_experts(rng, hidden, inter)
     layer = clef_i4.MoeLayer(dev_weight(*gate, 128 * inter, hidden), dev_weight(*up, 128 * inter, hidden),
                              dev_weight(*down, 128 * hidden, inter))
-    layer.workspace(tokens, DEV).fill_(0xFF)
+    scratch = layer.workspace(tokens, DEV).fill_(0xFF)
+    layer.workspace = lambda *_: scratch
     routes = torch.empty((tokens, 16), dtype=torch.float32, device=DEV)
     got = bf16_host(layer(to_dev_bf16(x), to_dev_bf16(logits), routes_out=routes))
     want_routes = oracle.route(logits, 8)
