@@ -9,7 +9,8 @@ M=4096 on one MI355X.
                INT4 codes run as bf6 (e3m2 holds every code -8..7 exactly) on
                the fp6 MFMA; the output equals the INT4-operand GEMM's bit for
                bit (checked in the run), which is reported beside it
-               (int4_operand_gemm).
+               (int4_operand_gemm); so is the call on INT4 operands that
+               re-encodes both and runs the bf6 GEMM (int4_project_prepared).
   rotating_weights  the same projection in both forms with the weight cycled
                through copies that exceed the 256 MB last-level cache (INT4 14
                x 25 MB, bf6 10 x 38 MB), each with its own output, so every
@@ -57,6 +58,10 @@ sys.path.insert(0, ROOT)
 INT8_PEAK_TOPS = 5000.0  # MI355X dense int8 MFMA, 5.0 POP/s
 FP6_PEAK_TOPS = 10100.0  # MI355X dense fp6 / fp4 MFMA, 10.1 PFLOP/s
 HBM_PEAK_GBS = 8000.0
+# The GEMM on packed INT4 operands by name (256 x 256 persistent tiles): by
+# itself project_prepared re-encodes large operands and runs the bf6 GEMM, which
+# would check and time that kernel against itself.
+INT4_KERNEL = 2
 # HBM bytes moved per launch of the M4096 K4096 N12288 bf6 GEMM kernel:
 # rocprofv3 FETCH_SIZE and WRITE_SIZE passes over `bench.py --only gemm`, each
 # scaled by the reading for a plain 512 MiB copy (x2.000 fetch, x1.000 write);
@@ -106,7 +111,7 @@ def device_warmup(seconds=0.25):
     t0 = time.perf_counter()
     while time.perf_counter() - t0 < seconds:
         for _ in range(20):
-            clef_i4.project_prepared(a, w, out=out)
+            clef_i4.project_prepared(a, w, out=out, config=INT4_KERNEL)
         torch.cuda.synchronize()
 
 
@@ -139,7 +144,8 @@ def gemm_leg(args):
     quantized operands: the bf6 GEMM (codes re-encoded as e3m2, exact; weight
     re-encoded once at load, activation quantized straight into bf6) -- the
     headline -- and the GEMM on the reference's packed INT4 operands. The two
-    outputs must be identical bit for bit."""
+    outputs must be identical bit for bit, and so must that of the call that
+    takes the INT4 operands through the bf6 GEMM."""
     import torch
 
     import clef_i4
@@ -154,21 +160,28 @@ def gemm_leg(args):
 
     out = torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
     out_i4 = torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
-    i4_ms = timed(lambda: clef_i4.project_prepared(a, qw, out=out_i4), args.steps, args.warmup)
+    i4_ms = timed(lambda: clef_i4.project_prepared(a, qw, out=out_i4, config=INT4_KERNEL), args.steps, args.warmup)
     i4_prep_ms = timed(lambda: clef_i4.prepare(x, out=a.storage), args.steps, args.warmup)
     prep_ms = timed(lambda: clef_i4.prepare_f6(x, out=af.storage), args.steps, args.warmup)
     ms = timed(lambda: clef_i4.project_f6(af, fw, out=out), args.steps, args.warmup)
     torch.cuda.synchronize()
     if not torch.equal(out.view(torch.int16), out_i4.view(torch.int16)):
         raise SystemExit("bf6 GEMM output differs from the INT4 GEMM's")
+    out_call = torch.empty_like(out)
+    call_ms = timed(lambda: clef_i4.project_prepared(a, qw, out=out_call), args.steps, args.warmup)
+    if not torch.equal(out_call.view(torch.int16), out_i4.view(torch.int16)):
+        raise SystemExit("project_prepared's output differs from the INT4 GEMM's")
     ops = 2.0 * m * n * k
     # operands read once (codes + f32 scales) and the bf16 output written once
     nbytes = m * k * 3 // 4 + 4 * m + n * k * 3 // 4 + 4 * n + 2 * m * n
     i4_bytes = m * k // 2 + 4 * m + n * k // 2 + 4 * n + 2 * m * n
+    # both operands also written in the bf6 form and read back
+    call_bytes = i4_bytes + 2 * (m * k + n * k) * 3 // 4
     rot = rotating_gemm(args, a, af, qw, fw, out_i4, out)
     return {"m": m, "n": n, "k": k, "ms": ms, "tops": ops / ms / 1e9, "prepare_ms": prep_ms,
             "ops": ops, "bytes": nbytes, "rotating": rot,
-            "int4": {"ms": i4_ms, "tops": ops / i4_ms / 1e9, "prepare_ms": i4_prep_ms, "bytes": i4_bytes}}
+            "int4": {"ms": i4_ms, "tops": ops / i4_ms / 1e9, "prepare_ms": i4_prep_ms, "bytes": i4_bytes},
+            "call": {"ms": call_ms, "tops": ops / call_ms / 1e9, "bytes": call_bytes}}
 
 
 def rotating_gemm(args, a, af, qw, fw, out_i4, out_f6):
@@ -187,7 +200,7 @@ def rotating_gemm(args, a, af, qw, fw, out_i4, out_f6):
     for form, copies, make, run, want in (
             ("int4", 14, lambda: clef_i4.QuantizedWeight(qw.codes.clone(), qw.scales.clone(), qw.rows, qw.cols,
                                                          qw.stride, qw.bits),
-             lambda w, o: clef_i4.project_prepared(a, w, out=o), out_i4),
+             lambda w, o: clef_i4.project_prepared(a, w, out=o, config=INT4_KERNEL), out_i4),
             ("bf6", 10, lambda: clef_i4.F6Weight(fw.codes.clone(), fw.scales.clone(), fw.rows, fw.cols),
              lambda w, o: clef_i4.project_f6(af, w, out=o), out_f6)):
         ws = [make() for _ in range(copies)]
@@ -343,7 +356,7 @@ def attention_leg(args):
     ms = timed(step, args.steps, max(1, args.warmup // 4))
     a4 = clef_i4.prepare(x)
     for i in range(4):
-        want = clef_i4.project_prepared(a4, ws[i], residual=res if i == 3 else None)
+        want = clef_i4.project_prepared(a4, ws[i], residual=res if i == 3 else None, config=INT4_KERNEL)
         if not torch.equal(want.view(torch.int16), outs[i].view(torch.int16)):
             raise SystemExit("bf6 attention projection differs from the INT4 one")
     ops = 2.0 * m * d * (d + kv + kv + d)
@@ -395,8 +408,9 @@ def mlp_leg(args):
 
     ms = timed(block, args.steps, max(1, args.warmup // 2))
     a4 = clef_i4.prepare(x)
-    h4 = clef_i4.prepare_swiglu(clef_i4.project_prepared(a4, wg), clef_i4.project_prepared(a4, wu))
-    if not torch.equal(clef_i4.project_prepared(h4, wd).view(torch.int16), y.view(torch.int16)):
+    h4 = clef_i4.prepare_swiglu(clef_i4.project_prepared(a4, wg, config=INT4_KERNEL),
+                                clef_i4.project_prepared(a4, wu, config=INT4_KERNEL))
+    if not torch.equal(clef_i4.project_prepared(h4, wd, config=INT4_KERNEL).view(torch.int16), y.view(torch.int16)):
         raise SystemExit("bf6 MLP block differs from the INT4 one")
     ops = 2.0 * m * (2 * f) * d + 2.0 * m * d * f
     return {"ms": ms, "tops": ops / ms / 1e9}
@@ -652,6 +666,8 @@ def main():
         line["int4_operand_gemm"] = {"ms": round(i4["ms"], 4), "tops": round(i4["tops"], 1),
                                      "pct_int8_peak": round(100.0 * i4["tops"] / INT8_PEAK_TOPS, 2),
                                      "prepare_ms": round(i4["prepare_ms"], 4)}
+        line["int4_project_prepared"] = {"ms": round(g["call"]["ms"], 4), "tops": round(g["call"]["tops"], 1),
+                                         "hbm_gbs": round(g["call"]["bytes"] / g["call"]["ms"] / 1e6, 1)}
         line["rotating_weights"] = {f: {"ms": round(v["ms"], 4), "tops": round(v["tops"], 1),
                                         "pct_int8_peak": round(100.0 * v["tops"] / INT8_PEAK_TOPS, 2),
                                         "copies": v["copies"], "weight_mb_cycled": v["weight_mb_cycled"]}

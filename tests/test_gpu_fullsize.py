@@ -59,6 +59,12 @@ def check_prepared_rows(a: clef_i4.Prepared, x_rows: np.ndarray, rows: np.ndarra
     assert np.array_equal(got_s.view(np.uint32), scales.view(np.uint32)), "prepared scales"
 
 
+# project_prepared's configuration of the persistent kernel on packed INT4
+# operands (256 x 256 tiles); by itself the call re-encodes operands of these
+# sizes and runs the bf6 kernel
+INT4_KERNEL = 2
+
+
 def check_packed_blocks(w_dev: torch.Tensor, qw: clef_i4.QuantizedWeight):
     """First and last 128-row blocks of the GPU-packed weight against the
     oracle's packing of the same bf16 rows (tiles of 128 rows are contiguous
@@ -114,8 +120,12 @@ def test_attention_projection_full_shape(n):
     codes, scales, _ = oracle.prepare(u16(x[idx]), a.stride)
     want = oracle.gemm(codes, scales, *host_weight(qw), n, k, residual=u16(res[idx]))
     assert_rows(u16(out[idx]), want, rows, f"projection 16384x4096x{n} + residual")
+    # the kernel on INT4 operands, against the automatic choice and the bf6
+    # form (the same kernel, where the choice is to re-encode): every row
+    int4 = clef_i4.project_prepared(a, qw, residual=res, config=INT4_KERNEL)
+    assert torch.equal(int4.view(torch.int16), out.view(torch.int16)), f"INT4 projection 16384x4096x{n} + residual"
     f6 = clef_i4.project_f6(clef_i4.prepare_f6(x), clef_i4.f6_weight(qw), residual=res)
-    assert torch.equal(f6.view(torch.int16), out.view(torch.int16)), f"bf6 projection 16384x4096x{n} + residual"
+    assert torch.equal(f6.view(torch.int16), int4.view(torch.int16)), f"bf6 projection 16384x4096x{n} + residual"
 
 
 def test_dense_mlp_full_shape():
@@ -141,6 +151,11 @@ def test_dense_mlp_full_shape():
     h_codes, h_scales, _ = oracle.prepare_swiglu(g_want, u_want, h.stride)
     y_want = oracle.gemm(h_codes, h_scales, *host_weight(wd), d, f)
     assert_rows(u16(y[idx]), y_want, rows, "mlp down")
+    # each projection by the kernel on INT4 operands: every row of the
+    # automatic choice, which re-encodes them for the bf6 kernel
+    for what, (act, w, got) in {"gate": (a, wg, gate), "up": (a, wu, up), "down": (h, wd, y)}.items():
+        int4 = clef_i4.project_prepared(act, w, config=INT4_KERNEL)
+        assert torch.equal(int4.view(torch.int16), got.view(torch.int16)), f"INT4 mlp {what}"
     # the same block on the bf6 form of the codes (as the benchmark runs it),
     # every stage's whole output bit for bit
     af = clef_i4.prepare_f6(x)
