@@ -1,7 +1,8 @@
 """Python binding of the gfx950 INT4 path (C ABI in include/clef_i4.h).
 
-A thin ctypes layer: torch supplies device memory and the current HIP stream,
-the library does all the work. Function names follow the reference's operator
+A thin layer: torch supplies device memory and the current HIP stream, the
+call module (csrc/host_call.cpp) converts and checks arguments, the library
+does all the work. Function names follow the reference's operator
 API (src/quantized.rs, src/omni.rs, src/ops.rs) so callers read the same:
 outputs are allocated here (as the reference's Engine allocates them) and the
 C entry points only write into them.

@@ -1246,7 +1246,8 @@ hipError_t launch_decode_m(const uint32_t* a, int a_words, const float* as, cons
   if (m == 1) return launch_decode_mr<1, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
   if (m == 2) return launch_decode_mr<2, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
   if (m <= 4) return launch_decode_mr<4, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
-  if (m <= 8) return launch_decode_mr<8, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
+  if constexpr (!I8)  // INT8: four rows at most (launch_gemm_i8)
+    if (m <= 8) return launch_decode_mr<8, RESID, I8>(a, a_words, as, w, ws, m, n, k, residual, out, stream);
   return hipErrorInvalidValue;
 }
 

@@ -55,12 +55,12 @@ hipError_t launch_tile_permute(const uint16_t* src, int64_t rows, int cols, uint
 hipError_t launch_gemm_i4(const uint32_t* a, int a_words, const float* a_scales,
                           const uint32_t* w_tiled, const float* w_scales, int64_t m, int n, int k,
                           const uint16_t* residual, uint16_t* out, int config, hipStream_t stream);
-// INT8 x INT8 G1 (codes 4 per word, weights tiled as retile_codes with bits 8).
 // Q1(x) and G1 in one launch for a few rows (project_fusable).
 bool project_fusable(int64_t m, int n, int k);
 hipError_t launch_project_i4(const uint16_t* x, const uint32_t* w, const float* ws, int64_t m, int n, int k,
                              const uint16_t* residual, uint16_t* out, hipStream_t stream);
-// The INT8 ring kernel (gemm_i8.hip), 128 x 128 tiles.
+// INT8 x INT8 G1 (codes 4 per word, weights tiled as retile_codes with bits 8);
+// _ring: the ring kernel (gemm_i8.hip), 128 x 128 tiles, whatever the shape.
 hipError_t launch_gemm_i8_ring(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,
                                int64_t m, int n, int k, const uint16_t* residual, uint16_t* out, hipStream_t stream);
 hipError_t launch_gemm_i8(const uint32_t* a, int a_words, const float* as, const uint32_t* w, const float* ws,

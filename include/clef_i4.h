@@ -190,7 +190,7 @@ int clef_i4_gemm(const uint32_t* a, int32_t k_stride, const float* a_scales, con
                  const float* w_scales, int64_t m, int32_t n, int32_t k, const uint16_t* residual,
                  uint16_t* out, clef_stream_t stream);
 
-/* clef_i4_gemm with scratch: for shapes of many tiles the operands are first
+/* clef_i4_gemm with scratch: for shapes of many rows and tiles the operands are first
  * re-encoded as bf6 in the workspace (clef_i4_f6_activation,
  * clef_i4_f6_weight) and multiplied by clef_i4_gemm_f6, the same bits in less
  * time. workspace_bytes gives 0 for every other shape; with less workspace

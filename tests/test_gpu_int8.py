@@ -111,8 +111,9 @@ def test_i8_gemm_extreme_codes_and_nonfinite_rows():
 @pytest.mark.parametrize("m", [1, 3, 8])
 @pytest.mark.parametrize("n,k", [(256, 256), (512, 2304), (1024, 4096), (256, 12288)])
 def test_i8_gemm_decode_rows_match_oracle(m, n, k):
-    """At most 8 rows: the v_dot4_i32_i8 kernel, k-steps of 128 k (2 to 96 of
-    them over its 8 waves), with and without the residual."""
+    """Up to 4 rows: the v_dot4_i32_i8 kernel, k-steps of 128 k (2 to 96 of
+    them over its 8 waves); 8 rows: the split-K tiles on the same k-steps; with
+    and without the residual."""
     rng = np.random.default_rng(m * 100 + n + k)
     x = BF(rng.standard_normal((m, k)).astype(np.float32))
     w = BF((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
