@@ -428,9 +428,12 @@ __device__ __forceinline__ void ring_issue_lut(char* lds) {
 // without the MFMAs 91.0; at 128 x 128 tiles (37 x 5120 x 17408, 36.2 us) the
 // DMA and the reads alone take 35.7.
 //
-// The k-steps before a tile's last load the next tile's first. The last k-step's stage stays free: the epilogue stages its output there, and
-// the next tile's k-step NST - 1 goes into it afterwards. The epilogue's
-// stores drain under the next tile's first k-steps.
+// The k-steps before a tile's last load the next tile's first. The last k-step's
+// stage stays free: the epilogue stages its output there, and the next tile's
+// k-step NST - 1 goes into it afterwards. The epilogue's stores drain under the
+// next tile's first k-steps. A tile of NST - 1 k-steps leaves one stage of the
+// ring free from its start, which takes the next tile's k-step 0. Tiles of fewer
+// load, contract and store in turn.
 //
 // GU (fused gate/up, benches/kernels/omni_gate_up_i4.loom's dense form): a
 // tile is BM rows x BN / 2 output columns of h; its B stage holds the gate
@@ -490,7 +493,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_ring_kernel(
   while (true) {
     const int t_next = t + (int)gridDim.x;
     const bool has_next = t_next < total;
-    const bool chain = has_next && ksteps >= NST;  // this tile loads the next one's first k-steps
+    const bool chain = has_next && ksteps >= NST - 1;  // this tile loads the next one's first k-steps
     const RingTiles nxt = tile(has_next ? t_next : t);
     // What the DMA behind this tile's k-steps loads: the next tile's first
     // k-steps, or nothing (an empty resource: the stages get zeros that
@@ -514,16 +517,18 @@ __global__ __launch_bounds__(T::THREADS) void gemm_ring_kernel(
       if (fresh) {
         ring_issue<Op, T, GU>(r0, cur, voff, kb, 0);
         if (ksteps > 1) ring_issue<Op, T, GU>(r1, cur, voff, kb, 1);
-        if (ksteps > 2) ring_issue<Op, T, GU>(r2, cur, voff, kb, 2);
-        if (NST == 4 && ksteps > 3) ring_issue<Op, T, GU>(r3, cur, voff, kb, 3);
-        if (ksteps >= NST)
+        if (NST == 4 && ksteps > 2) ring_issue<Op, T, GU>(r2, cur, voff, kb, 2);
+      }  // else k-step 0 landed before the barrier that ended the last tile
+      if (ksteps >= NST)
+        ring_issue<Op, T, GU>(NST == 4 ? r3 : r2, cur, voff, kb, NST - 1);
+      else if (ksteps == NST - 1)
+        ring_issue<Op, T, GU>(NST == 4 ? r3 : r2, ahead, voff, kb, 0);
+      if (fresh) {
+        if (ksteps >= NST - 1)
           wait_stages(std::integral_constant<int, NST - 1>{}, I0{});
         else
           wait_vmcnt<0>();
         ring_lds_barrier();
-      } else {
-        // k-step 0 landed before the barrier that ended the last tile
-        ring_issue<Op, T, GU>(NST == 4 ? r3 : r2, cur, voff, kb, NST - 1);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -587,7 +592,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_ring_kernel(
     tile_body(st(rot), st((rot + 1) % NST), st((rot + 2) % NST), st((rot + 3) % NST), last, sc);
     // this tile's scales have landed: issued before k-step NST - 1, which the
     // loop waited for
-    if (ksteps < NST || !chain) wait_vmcnt<0>();
+    if (!chain) wait_vmcnt<0>();
     auto epilogue = [&](const typename Op::Acc (&sum)[T::EM][T::TN]) {
       if constexpr (GU)
         ring_epilogue_gu<T>(sum, Op::kDotPerStep * (float)kb, M, N, cur.m0, cur.n0, out, last + wave * T::EPI_WAVE, sc, lds + T::LUT_OFF);

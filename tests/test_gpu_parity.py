@@ -1341,7 +1341,8 @@ F6_PATHS = [(1, 256, 256), (33, 1024, 1280), (64, 2048, 2304), (100, 4096, 512),
             (250, 4096, 768), (140, 7168, 2304),
             (300, 4096, 256), (300, 4096, 512), (385, 4096, 768), (300, 4096, 1024), (100, 66048, 1024),
             (600, 8192, 256), (600, 8192, 512), (577, 8192, 768), (620, 22016, 768),
-            (1030, 8192, 256), (1100, 8192, 768), (2100, 8192, 1280)]
+            (1030, 8192, 256), (1100, 8192, 768), (2100, 8192, 1280),
+            (2305, 16640, 256), (2305, 16640, 512)]  # three tiles per workgroup, one k-step short of the ring and past it
 
 
 def _f6_path_operands(m, n, k, weights):
@@ -1386,7 +1387,7 @@ def test_gemm_f6_every_path(m, n, k, resid):
 @pytest.mark.parametrize("m,n,k", [(1, 256, 256), (31, 1024, 1280), (64, 4096, 768), (100, 2304, 2304),
                                    (100, 12288, 256), (90, 12288, 768), (90, 12288, 2048), (257, 4096, 512),
                                    (128, 17408, 512), (385, 8192, 256), (400, 8192, 1024), (620, 12288, 768),
-                                   (300, 12288, 256), (400, 12288, 1280), (1100, 12288, 512)])
+                                   (300, 12288, 256), (400, 12288, 1280), (1100, 12288, 512), (2305, 8448, 256)])
 def test_gemm_f6_gate_up_every_path(m, n, k):
     """The fused gate/up on each kernel: all rows bit-equal to the unfused
     INT4-operand path, sampled rows to the oracle."""
