@@ -808,14 +808,20 @@ class MoeLayer:
         self.inter = gate.rows // 128
         self._ws_size = (-1, 0)  # the last call's tokens and scratch bytes
 
-    def workspace(self, tokens: int, device) -> torch.Tensor:
-        """Scratch of one call, from torch's allocator each time: calls of
-        other streams and threads and captured graphs have their own."""
+    def workspace_bytes(self, tokens: int) -> int:
         held, nbytes = self._ws_size
         if held != tokens:
             nbytes = _n.value(_n.clef_moe_layer_workspace_bytes, tokens, self.hidden, self.inter, self.topk)
             self._ws_size = tokens, nbytes
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return nbytes
+
+    def workspace(self, tokens: int, device) -> torch.Tensor:
+        return torch.empty(self.workspace_bytes(tokens), dtype=torch.uint8, device=device)
+
+    def _scratch(self, x: torch.Tensor) -> torch.Tensor:
+        """workspace of one call, from torch's allocator each time: calls of
+        other streams and threads and captured graphs have their own."""
+        return _n.empty(x, torch.uint8, self.workspace_bytes(x.shape[0]))
 
     def __call__(self, x: torch.Tensor, logits: torch.Tensor | None = None, routes_out: torch.Tensor | None = None,
                  out: torch.Tensor | None = None) -> torch.Tensor:
@@ -826,7 +832,7 @@ class MoeLayer:
             logits = router_logits(x, self.router)  # e.project(norm, "mlp.gate"), src/omni.rs:764
         if out is None:
             out = _n.empty(x, torch.bfloat16, tokens, self.hidden)
-        ws = self.workspace(tokens, x.device)
+        ws = self._scratch(x)
         dtype = 0 if logits.dtype == torch.bfloat16 else 1
         _n.launch(_n.clef_moe_layer, x, logits, dtype, tokens, self.hidden, self.inter, 128, self.topk,
                   self.gate.codes, self.gate.scales, self.up.codes, self.up.scales, self.down.codes, self.down.scales,

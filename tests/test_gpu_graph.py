@@ -100,7 +100,7 @@ def test_moe_layer_scratch_is_each_calls_own():
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), want.view(torch.int16))
         assert all(bool((h == 0x5A).all()) for h in held)
-    first = layer.workspace(t, "cuda")
+    first = layer._scratch(x)
     with torch.cuda.stream(side):
-        second = layer.workspace(t, "cuda")
+        second = layer._scratch(x)
     assert first.data_ptr() != second.data_ptr() and first.numel() == second.numel() == nbytes

@@ -962,7 +962,7 @@ def test_moe_layer_degenerate_logit_rows(tokens):
     layer = clef_i4.MoeLayer(dev_weight(*gate, 128 * inter, hidden), dev_weight(*up, 128 * inter, hidden),
                              dev_weight(*down, 128 * hidden, inter))
     scratch = layer.workspace(tokens, DEV).fill_(0xFF)
-    layer.workspace = lambda *_: scratch
+    layer._scratch = lambda *_: scratch
     routes = torch.empty((tokens, 16), dtype=torch.float32, device=DEV)
     got = bf16_host(layer(to_dev_bf16(x), to_dev_bf16(logits), routes_out=routes))
     want_routes = oracle.route(logits, 8)
